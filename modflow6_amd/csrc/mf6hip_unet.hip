@@ -10,14 +10,10 @@
 // channel).  Every channel count the MFMA kernels see is a multiple of 16
 // (the 3 input features are padded to 16 zero channels).
 //
-// 3x3x3 convolution as an implicit GEMM: one wave computes 16 consecutive
-// voxels along W times all output channels; per tap and 16-channel chunk
-// one MFMA per 16 output channels.  A-fragment (16 voxels x 16 input
-// channels): lane l holds voxel l % 16, channels 4 (l / 16) .. +3 (one 8-byte
-// load, channels-last).  B-fragment (16 input x 16 output channels): lane l
-// holds output channel l % 16, input channels 4 (l / 16) .. +3, pre-packed
-// in that order.  Accumulator: lane l holds output channel l % 16 of voxels
-// 4 (l / 16) .. +3.
+// 3x3x3 convolution as an implicit GEMM on v_mfma_f32_16x16x32_bf16: a
+// workgroup stages the input halo of its voxel tile in LDS, a channel chunk
+// at a time, and each wave multiplies MT rows of 16 voxels by the packed
+// weights (see k_conv3).
 //
 // The backward pass reuses the same kernel for the data gradient (weights
 // flipped in the tap index and transposed in the channels), an MFMA
@@ -35,6 +31,8 @@
 namespace {
 
 typedef short s4 __attribute__((ext_vector_type(4)));
+typedef short s8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned short bf16;
 
@@ -69,83 +67,201 @@ struct Grid3 {
 
 // y[v, yoff + o] = act(bias[o] + sum_{t, c} x[v + off(t), xoff + c] W[t, c, o])
 // act: relu when relu != 0; then y *= (mask[v, moff + o] > 0) when mask != 0.
-// wp: packed fragments [27][cin / 16][NCO][64][4].  One wave per 16-voxel
-// tile; tiles = D * H * ceil(W / 16).
-template <int NCO>
+//
+// A workgroup of four waves computes WD x (4 / WD) MT x 16 voxels (d, h, w)
+// by NC tiles of 16 output channels (blockIdx.y takes the next NC tiles).
+// Per chunk of CW input channels the input halo, (WD + 2) x (TH + 2) x 18
+// voxels, is staged once in LDS, so a value read from memory serves all 27
+// taps; a wave then walks the (kd, kw) pairs of the taps and, per pair, loads
+// the MT + 2 input rows its MT output rows need and reuses them for the three
+// kh (each row feeds up to three MFMAs per output tile instead of one).
+// K of one MFMA is 32: a chunk of 32 channels of one (kd, kw) for CW = 32,
+// two (kd, kw) pairs of 16 channels for CW = 16 (cin not a multiple of 32).
+// The weights are the A operand (lane l: output channel l % 16, k = 8 (l /
+// 16) .. +7), the voxels the B operand, so a lane ends up with four
+// consecutive output channels of one voxel and stores them as 8 bytes.
+// LDS: the 16-byte pieces of a voxel are permuted by its w so that the 16
+// voxels of a row read by one quarter of the wave fall in different banks.
+// The first version (one wave per 16 voxels, activations and weights loaded
+// per tap from L2, K = 16) was bound by those loads.  On a 16 x 256 x 256
+// field the level-0 convolutions of the 16-32-64-64 network went from 228 to
+// 56 us each on average, those of level 1 from 160 to 57, and the whole
+// forward pass's convolutions from 112 to about 430 TFLOP/s.
+template <int CW>
+struct ConvGeo {
+  static constexpr int PIECES = CW / 8;                 // 16-byte pieces per voxel
+  static constexpr int STEPS = CW == 32 ? 9 : 5;        // MFMA steps over the (kd, kw) pairs
+  static constexpr int VB = CW * 2;                     // bytes per voxel
+  // byte offset in a voxel of piece q of the voxel at halo column pw
+  __device__ static int piece(int q, int pw) {
+    return CW == 32 ? ((q ^ ((pw >> 2) & 3)) << 4) : ((q ^ ((pw >> 3) & 1)) << 4);
+  }
+};
+
+// the halo of channels c0 .. c0 + CW - 1 of the tile at (d0, h0, w0) into
+// LDS, zero outside the grid; PD x PH x 18 voxels, mph = ceil(2^16 / PH)
+template <int CW>
+__device__ inline void stage_halo(char *lds, const Grid3 &g, const bf16 *__restrict__ x, int ldx,
+                                  int c0, int d0, int h0, int w0, int PD, int PH, int mph) {
+  constexpr int P = ConvGeo<CW>::PIECES;
+  const int n = PD * PH * 18 * P;
+  for (int i = threadIdx.x; i < n; i += 256) {
+    const int q = i & (P - 1), vox = i / P;
+    const int row = vox / 18, pw = vox - row * 18;
+    const int pd = (row * mph) >> 16, ph = row - pd * PH;
+    const int d = d0 + pd - 1, h = h0 + ph - 1, w = w0 + pw - 1;
+    s8 v = s8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (d >= 0 && d < g.D && h >= 0 && h < g.H && w >= 0 && w < g.W)
+      v = *reinterpret_cast<const s8 *>(x + (size_t)((d * g.H + h) * g.W + w) * ldx + c0 + 8 * q);
+    *reinterpret_cast<s8 *>(lds + vox * ConvGeo<CW>::VB + ConvGeo<CW>::piece(q, pw)) = v;
+  }
+}
+
+template <int CW, int MT, int NC>
 __global__ void __launch_bounds__(256) k_conv3(Grid3 g, const bf16 *__restrict__ x, int ldx,
-                                               int xoff, int cin, const s4 *__restrict__ wp,
-                                               const float *__restrict__ bias, int relu,
+                                               int xoff, int cin, const s8 *__restrict__ wp,
+                                               int nco, const float *__restrict__ bias, int relu,
                                                bf16 *__restrict__ y, int ldy, int yoff,
                                                const bf16 *__restrict__ mask, int ldm, int moff,
-                                               int ntiles) {
-  const int lane = threadIdx.x & 63;
-  const int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (tile >= ntiles) return;
-  const int ntw = (g.W + 15) >> 4;
-  const int w0 = (tile % ntw) << 4;
-  const int hh = (tile / ntw) % g.H;
-  const int dd = tile / (ntw * g.H);
-  const int wl = w0 + (lane & 15);
-  const int kq = lane >> 4;
-  const int ncc = cin >> 4;
-  f4 acc[NCO];
+                                               int WD, int mph) {
+  extern __shared__ char lds[];
+  using G = ConvGeo<CW>;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int WH = 4 / WD;
+  const int TH = WH * MT, PD = WD + 2, PH = TH + 2;
+  const int ntw = (g.W + 15) >> 4, nth = (g.H + TH - 1) / TH;
+  const int tile = xcd_block();
+  const int w0 = (tile % ntw) << 4, h0 = (tile / ntw) % nth * TH, d0 = tile / (ntw * nth) * WD;
+  const int wd = wv % WD, wh = wv / WD;
+  const int lw = lane & 15, kq = lane >> 4;
+  const int ct0 = blockIdx.y * NC;             // first output-channel tile
+  f4 acc[MT][NC];
 #pragma unroll
-  for (int c = 0; c < NCO; c++) acc[c] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int t = 0; t < 27; t++) {
-    const int zd = dd + t / 9 - 1, zh = hh + (t / 3) % 3 - 1, zw = wl + t % 3 - 1;
-    const bool ok = zd >= 0 && zd < g.D && zh >= 0 && zh < g.H && zw >= 0 && zw < g.W;
-    const bf16 *src = ok ? x + (size_t)((zd * g.H + zh) * g.W + zw) * ldx + xoff + 4 * kq : x;
-    const s4 *wt = wp + (size_t)t * ncc * NCO * 64 + lane;
-    for (int cc = 0; cc < ncc; cc++) {
-      s4 a = s4{0, 0, 0, 0};
-      if (ok) a = *reinterpret_cast<const s4 *>(src + 16 * cc);
+  for (int m = 0; m < MT; m++)
 #pragma unroll
-      for (int c = 0; c < NCO; c++) {
-        s4 b = wt[(cc * NCO + c) * 64];
-        acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[c], 0, 0, 0);
-      }
-    }
+    for (int c = 0; c < NC; c++) acc[m][c] = f4{0.f, 0.f, 0.f, 0.f};
+  const int rowb = 18 * G::VB, planeb = PH * rowb;
+  const int base = wd * planeb + wh * MT * rowb;
+  // fragments of output tile ct0 + c (a tile past the last reads the last's)
+  const s8 *wt[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    const int ct = ct0 + c < nco ? ct0 + c : nco - 1;
+    wt[c] = wp + (size_t)ct * (cin / CW) * G::STEPS * 3 * 64;
   }
+  for (int c0 = 0; c0 < cin; c0 += CW) {
+    if (c0) __syncthreads();
+    stage_halo<CW>(lds, g, x, ldx, xoff + c0, d0, h0, w0, PD, PH, mph);
+    __syncthreads();
+    // the weights of a step are loaded while the step before it runs
+    b8 wn[3][NC];
 #pragma unroll
-  for (int c = 0; c < NCO; c++) {
-    const int o = c * 16 + (lane & 15);
-    const float bo = bias ? bias[o] : 0.f;
+    for (int kh = 0; kh < 3; kh++)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int w = w0 + 4 * kq + e;
-      if (w >= g.W) continue;
-      const size_t v = (size_t)(dd * g.H + hh) * g.W + w;
-      float val = acc[c][e] + bo;
-      if (relu && val < 0.f) val = 0.f;
-      if (mask && !(bf2f(mask[v * ldm + moff + o]) > 0.f)) val = 0.f;
-      y[v * ldy + yoff + o] = f2bf(val);
+      for (int c = 0; c < NC; c++) wn[kh][c] = *reinterpret_cast<const b8 *>(wt[c] + kh * 64 + lane);
+#pragma unroll
+    for (int s = 0; s < G::STEPS; s++) {
+      b8 w[3][NC];
+#pragma unroll
+      for (int kh = 0; kh < 3; kh++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          w[kh][c] = wn[kh][c];
+          if (s + 1 < G::STEPS)
+            wn[kh][c] = *reinterpret_cast<const b8 *>(wt[c] + ((s + 1) * 3 + kh) * 64 + lane);
+        }
+      // this lane's (kd, kw) pair and 16-byte piece
+      int off, pw;
+      if (CW == 32) {
+        pw = lw + s % 3;
+        off = (s / 3) * planeb + pw * G::VB + G::piece(kq, pw);
+      } else {
+        const int qa = 2 * s, qb = 2 * s + 1 < 9 ? 2 * s + 1 : qa;
+        const bool hi = kq >= 2;
+        pw = lw + (hi ? qb % 3 : qa % 3);
+        off = (hi ? qb / 3 : qa / 3) * planeb + pw * G::VB + G::piece(kq & 1, pw);
+      }
+      b8 a[MT + 2];
+#pragma unroll
+      for (int r = 0; r < MT + 2; r++) {
+        a[r] = *reinterpret_cast<const b8 *>(lds + base + off + r * rowb);
+        if (CW == 16 && s == G::STEPS - 1 && kq >= 2) a[r] = b8{};   // no tenth pair
+      }
+#pragma unroll
+      for (int kh = 0; kh < 3; kh++)
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int c = 0; c < NC; c++)
+            acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kh][c], a[m + kh], acc[m][c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++) wt[c] += G::STEPS * 3 * 64;
+  }
+  const int d = d0 + wd, w = w0 + lw;
+  if (d >= g.D || w >= g.W) return;
+#pragma unroll
+  for (int m = 0; m < MT; m++) {
+    const int h = h0 + wh * MT + m;
+    if (h >= g.H) break;
+    const size_t v = (size_t)(d * g.H + h) * g.W + w;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      if (ct0 + c >= nco) break;
+      const int o = (ct0 + c) * 16 + 4 * kq;
+      s4 mk = s4{0, 0, 0, 0}, out;
+      if (mask) mk = *reinterpret_cast<const s4 *>(mask + v * ldm + moff + o);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float val = acc[m][c][e] + (bias ? bias[o + e] : 0.f);
+        if (relu && val < 0.f) val = 0.f;
+        if (mask && !(bf2f((bf16)mk[e]) > 0.f)) val = 0.f;
+        out[e] = (short)f2bf(val);
+      }
+      *reinterpret_cast<s4 *>(y + v * ldy + yoff + o) = out;
     }
   }
 }
 
-// pack W (fp32 [27][cin_real][cout]) into fragments of a cin-channel input
-// (rows cin_real..cin-1 zero); flip != 0 packs the data-gradient weights
-// Wt[t][o][c] = W[26 - t][c][o] (input / output swapped; cin_real == cin)
+// chunk width of a convolution with ci input channels
+__host__ __device__ inline int conv_cw(int ci) { return ci % 32 == 0 ? 32 : 16; }
+
+// 16-byte weight fragments of a convolution: [output tile][chunk][step][kh][lane]
+__host__ __device__ inline int conv_nfrag(int ci, int co) {
+  const int cw = conv_cw(ci);
+  return (ci / cw) * (cw == 32 ? 9 : 5) * 3 * (co >> 4) * 64;
+}
+
+// pack W (fp32 [27][cin_real][cout]) into the fragments of k_conv3 for a
+// cin-channel input (rows cin_real..cin-1 zero); flip != 0 packs the
+// data-gradient weights Wt[t][o][c] = W[26 - t][c][o] (input / output
+// swapped; cin_real == cin)
 __global__ void k_pack_w(const float *__restrict__ w, int cin_real, int cin, int cout, int flip,
-                         s4 *__restrict__ wp) {
+                         s8 *__restrict__ wp) {
   const int ci = flip ? cout : cin;   // fragment input channels
   const int co = flip ? cin : cout;   // fragment output channels
-  const int nco = co >> 4, ncc = ci >> 4;
-  const int total = 27 * ncc * nco * 64;
+  const int cw = conv_cw(ci), steps = cw == 32 ? 9 : 5;
+  const int total = conv_nfrag(ci, co);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-    const int lane = i & 63;
+    const int lane = i & 63, kq = lane >> 4;
     int r = i >> 6;
-    const int c = r % nco;
-    r /= nco;
-    const int cc = r % ncc;
-    const int t = r / ncc;
-    s4 v;
-    for (int e = 0; e < 4; e++) {
-      const int kin = cc * 16 + 4 * (lane >> 4) + e;   // fragment input channel
-      const int kout = c * 16 + (lane & 15);           // fragment output channel
-      float f;
-      if (flip) f = w[((size_t)(26 - t) * cin_real + kout) * cout + kin];
-      else f = kin < cin_real ? w[((size_t)t * cin_real + kin) * cout + kout] : 0.f;
+    const int kh = r % 3;
+    r /= 3;
+    const int s = r % steps;
+    r /= steps;
+    const int cc = r % (ci / cw), c = r / (ci / cw);
+    const int pair = cw == 32 ? s : 2 * s + (kq >> 1);           // kd 3 + kw
+    const int kin0 = cc * cw + (cw == 32 ? 8 * kq : 8 * (kq & 1));
+    const int kout = c * 16 + (lane & 15);
+    const int t = (pair / 3) * 9 + kh * 3 + pair % 3;
+    s8 v;
+    for (int e = 0; e < 8; e++) {
+      const int kin = kin0 + e;
+      float f = 0.f;
+      if (pair < 9) {
+        if (flip) f = w[((size_t)(26 - t) * cin_real + kout) * cout + kin];
+        else f = kin < cin_real ? w[((size_t)t * cin_real + kin) * cout + kout] : 0.f;
+      }
       v[e] = (short)f2bf(f);
     }
     wp[i] = v;
@@ -468,8 +584,8 @@ struct UConv {
   int cin, cout;        // cin as the kernels see it (padded to 16)
   int cin_real;         // parameter rows (the first layer: the real inputs)
   size_t w_off, b_off;  // offsets into the flat parameter vector
-  s4 *wp = nullptr;     // forward fragments
-  s4 *wt = nullptr;     // data-gradient fragments
+  s8 *wp = nullptr;     // forward fragments
+  s8 *wt = nullptr;     // data-gradient fragments
 };
 
 // levels 0..nlev-1; conv layers in the order e0a e0b e1a e1b ... (two per
@@ -527,25 +643,82 @@ inline int nblk(size_t n) {
   return (int)(b < 1 ? 1 : b);
 }
 
-int launch_conv(UNetHandle *u, const Grid3 &g, const bf16 *x, int ldx, int xoff, int cin,
-                const s4 *wp, int cout, const float *bias, int relu, bf16 *y, int ldy, int yoff,
-                const bf16 *mask, int ldm, int moff) {
-  const int ntiles = g.D * g.H * ((g.W + 15) / 16);
-  const int blocks = (ntiles + 3) / 4;
-  hipStream_t s = u->stream;
-  switch (cout / 16) {
-    case 1: k_conv3<1><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 2: k_conv3<2><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 3: k_conv3<3><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 4: k_conv3<4><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 5: k_conv3<5><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 6: k_conv3<6><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 7: k_conv3<7><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    case 8: k_conv3<8><<<blocks, 256, 0, s>>>(g, x, ldx, xoff, cin, wp, bias, relu, y, ldy, yoff, mask, ldm, moff, ntiles); break;
-    default:
-      mf6hip_set_error("unsupported channel count " + std::to_string(cout));
-      return MF6HIP_EUNSUPPORTED;
+// Tile of k_conv3 for a grid: MT output rows per wave, WD waves along d and 4 /
+// WD along h, NC output tiles per workgroup.  Four rows per wave where that
+// leaves at least two workgroups per CU (512), else two or one, and on the
+// coarsest grids one output tile per workgroup: below that, idle CUs cost
+// more than the rows' and weights' reuse gains.  WD: the split that pads the
+// grid least (the widest on a tie, which has the smallest halo).
+struct ConvTile {
+  int MT, WD, NC, tiles, gy;
+};
+
+ConvTile conv_tile(const Grid3 &g, int nco) {
+  ConvTile best{};
+  for (int step = 0; step < 4; step++) {
+    ConvTile t{};
+    t.MT = step == 0 ? 4 : step == 1 ? 2 : 1;
+    t.gy = step == 3 ? nco : (nco + 3) / 4;
+    t.NC = (nco + t.gy - 1) / t.gy;
+    long long pad = -1;
+    for (int wd = 4; wd >= 1; wd >>= 1) {
+      const int th = 4 / wd * t.MT;
+      const int nd = (g.D + wd - 1) / wd, nh = (g.H + th - 1) / th;
+      const long long v = (long long)nd * wd * nh * th;
+      if (pad < 0 || v < pad) {
+        pad = v;
+        t.WD = wd;
+        t.tiles = nd * nh * ((g.W + 15) / 16);
+      }
+    }
+    if (step == 0 || (long long)t.tiles * t.gy > (long long)best.tiles * best.gy) best = t;
+    if ((long long)best.tiles * best.gy >= 512) break;
   }
+  return best;
+}
+
+template <int CW, int MT>
+void launch_conv_nc(int nc, dim3 grid, int shm, hipStream_t s, const Grid3 &g, const bf16 *x,
+                    int ldx, int xoff, int cin, const s8 *wp, int nco, const float *bias, int relu,
+                    bf16 *y, int ldy, int yoff, const bf16 *mask, int ldm, int moff, int WD,
+                    int mph) {
+#define MF6_CONV(N)                                                                            \
+  k_conv3<CW, MT, N><<<grid, 256, shm, s>>>(g, x, ldx, xoff, cin, wp, nco, bias, relu, y, ldy, \
+                                            yoff, mask, ldm, moff, WD, mph)
+  if (nc == 1) MF6_CONV(1);
+  else if (nc == 2) MF6_CONV(2);
+  else if (nc == 3) MF6_CONV(3);
+  else MF6_CONV(4);
+#undef MF6_CONV
+}
+
+int launch_conv(UNetHandle *u, const Grid3 &g, const bf16 *x, int ldx, int xoff, int cin,
+                const s8 *wp, int cout, const float *bias, int relu, bf16 *y, int ldy, int yoff,
+                const bf16 *mask, int ldm, int moff) {
+  if (cin % 16 || cout % 16 || cout > 256) {
+    mf6hip_set_error("unsupported channel count " + std::to_string(cout));
+    return MF6HIP_EUNSUPPORTED;
+  }
+  const int nco = cout / 16, cw = conv_cw(cin);
+  const ConvTile t = conv_tile(g, nco);
+  const int PH = 4 / t.WD * t.MT + 2, PD = t.WD + 2;
+  const int shm = PD * PH * 18 * cw * 2;            // at most 62 KB
+  const int mph = (65536 + PH - 1) / PH;
+  const dim3 grid(t.tiles, t.gy);
+  hipStream_t s = u->stream;
+#define MF6_CONV(C, M)                                                                           \
+  launch_conv_nc<C, M>(t.NC, grid, shm, s, g, x, ldx, xoff, cin, wp, nco, bias, relu, y, ldy,    \
+                       yoff, mask, ldm, moff, t.WD, mph)
+  if (cw == 32) {
+    if (t.MT == 4) MF6_CONV(32, 4);
+    else if (t.MT == 2) MF6_CONV(32, 2);
+    else MF6_CONV(32, 1);
+  } else {
+    if (t.MT == 4) MF6_CONV(16, 4);
+    else if (t.MT == 2) MF6_CONV(16, 2);
+    else MF6_CONV(16, 1);
+  }
+#undef MF6_CONV
   if (hipGetLastError() != hipSuccess) { mf6hip_set_error("conv launch failed"); return MF6HIP_EHIP; }
   return MF6HIP_OK;
 }
@@ -594,9 +767,11 @@ static int u_pack(UNetHandle *u) {
   hipStream_t s = u->stream;
   for (int i = 0; i < u->nconv(); i++) {
     UConv &L = u->conv[i];
-    const int nf = 27 * (L.cin / 16) * (L.cout / 16) * 64;
-    k_pack_w<<<nblk(nf), 256, 0, s>>>(u->p + L.w_off, L.cin_real, L.cin, L.cout, 0, L.wp);
-    if (L.wt) k_pack_w<<<nblk(nf), 256, 0, s>>>(u->p + L.w_off, L.cin_real, L.cin, L.cout, 1, L.wt);
+    k_pack_w<<<nblk(conv_nfrag(L.cin, L.cout)), 256, 0, s>>>(u->p + L.w_off, L.cin_real, L.cin,
+                                                             L.cout, 0, L.wp);
+    if (L.wt)
+      k_pack_w<<<nblk(conv_nfrag(L.cout, L.cin)), 256, 0, s>>>(u->p + L.w_off, L.cin_real, L.cin,
+                                                               L.cout, 1, L.wt);
   }
   if (hipGetLastError() != hipSuccess) { mf6hip_set_error("pack launch failed"); return MF6HIP_EHIP; }
   return MF6HIP_OK;
@@ -782,9 +957,8 @@ extern "C" int mf6hip_unet_create(int nlay, int nrow, int ncol, int nin, int nle
     off += (size_t)27 * L.cin_real * L.cout;
     L.b_off = off;
     off += L.cout;
-    const size_t nf = (size_t)27 * (L.cin / 16) * (L.cout / 16) * 64;
-    if (!rc) rc = ualloc(&L.wp, nf);
-    if (!rc && i != 0) rc = ualloc(&L.wt, nf);
+    if (!rc) rc = ualloc(&L.wp, conv_nfrag(L.cin, L.cout));
+    if (!rc && i != 0) rc = ualloc(&L.wt, conv_nfrag(L.cout, L.cin));
   }
   u->wo_off = off;
   off += c[0];

@@ -126,6 +126,35 @@ def test_unet_gradients_match_oracle(shape, ch):
     assert o == g.size
 
 
+# tiles of the convolution kernels: four, two and one rows per wave (by the
+# number of tiles), waves along d or along h (one layer), one to three output
+# tiles per workgroup and two workgroups of them (64 + 48 and 16 + 64 decoder
+# channels), extents that leave partial tiles on every side
+@pytest.mark.parametrize("shape,ch", [((5, 131, 210), (16, 48)), ((3, 50, 70), (16, 64, 48)),
+                                      ((1, 33, 47), (16, 64)), ((2, 17, 16), (16, 32, 16))])
+def test_unet_conv_tiles(shape, ch):
+    D, H, W = shape
+    p = init_params(3, ch, np.random.default_rng(8))
+    net = UNet(D, H, W, 3, ch, params=p)
+    x, t = sample(shape, 9)
+    y = net.forward(x)
+    loss, g = net.grad(x, t)
+    net.destroy()
+    xo = bf16(x).astype(np.float64).T.reshape(D, H, W, 3)
+    to = bf16(t).astype(np.float64).reshape(D, H, W, 1)
+    po = to_oracle(p, 3, ch, bf16d)
+    # the bounds of the tests above: BF16 rounding flips
+    assert rel(y, U.forward(po, xo, rnd=bf16d).reshape(-1)) < 1e-2
+    lr_, gr = U.loss_and_grads(po, xo, to, rnd=bf16d)
+    assert abs(loss - lr_) <= 1e-3 * lr_
+    o = 0
+    for w, b in gr:
+        for a in (w, b):
+            assert rel(g[o:o + a.size], a.ravel()) < 3e-2
+            o += a.size
+    assert o == g.size
+
+
 def test_unet_training_reduces_loss():
     shape, ch = (2, 16, 16), (16, 16, 32, 32)
     D, H, W = shape
