@@ -17,10 +17,11 @@
 //
 // The backward pass reuses the same kernel for the data gradient (weights
 // flipped in the tap index and transposed in the channels), an MFMA
-// weight-gradient kernel with split-K partials reduced in a fixed order, and
-// elementwise kernels for ReLU masks, pooling, upsampling and the skips.
+// weight- and bias-gradient kernel with split-K partials reduced in a fixed
+// order, and elementwise kernels for ReLU masks, pooling, upsampling and the skips.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -272,91 +273,150 @@ __global__ void k_pack_w(const float *__restrict__ w, int cin_real, int cin, int
 // weight gradient: dW[t][c][o] = sum_v x[v + off(t), c] dy[v, o]
 // ---------------------------------------------------------------------------
 
-// block = (t, c-tile, o-tile, split); 4 waves; wave j of split s handles the
-// 16-voxel chunks s * 4 + j, s * 4 + j + 4 S, ...  Partial tile written to
-// part[(split * 27 + t) * cin * cout + c * cout + o] after the 4 waves are
-// summed in order.
-__global__ void __launch_bounds__(256) k_wgrad(Grid3 g, const bf16 *__restrict__ x, int ldx,
+// and the bias gradient db[o] = sum_v dy[v, o].
+//
+// A GEMM over the voxels: M = output channels, N = input channels, K = the
+// voxels, once per tap.  Workgroup (split, 16 input channels, NC tiles of 16
+// output channels) walks its share of the voxel tiles (TD x TH x 16, 256
+// voxels), stages the tile's x halo and dy in LDS (channels last, as they lie
+// in memory) and keeps all 27 taps' accumulators in registers: wave j takes
+// taps j, j + 4, ... (28 with the bias, whose x is all ones), so every staged
+// value serves all taps and output tiles.  The MFMA operands need eight
+// consecutive voxels of one channel per lane; ds_read_b64_tr_b16 transposes
+// four voxels x 16 channels on the way out of LDS (lane i of a quarter wave
+// gives the address of voxel i / 4, channels 4 (i % 4) .., and receives
+// channel i of the four voxels), so a tap's shift is only an address offset.
+// Partials go to part[split] ([27][cin][cout], then [cout]) and are summed
+// in split order by k_wgrad_reduce.  The first version (one tap and one 16 x
+// 16 tile per workgroup, voxels gathered two bytes at a time) re-read x and
+// dy 27 times: over a training step's layers (16 x 256 x 256, 16-32-64-64)
+// 630 us each on average, now 51 (the level-0 ones 87, which LDS reads
+// bound: seven transposed x reads serve only one output tile), and its own
+// bias-gradient kernels are gone.
+constexpr int WG_MAXBLK = 512;   // workgroups of one layer's gradient
+template <int NC>
+__global__ void __launch_bounds__(256, 2) k_wgrad(Grid3 g, const bf16 *__restrict__ x, int ldx,
                                                int xoff, int cin, const bf16 *__restrict__ dy,
-                                               int ldd, int doff, int cout, int nsplit,
+                                               int ldd, int doff, int cout, int TD, int mph,
                                                float *__restrict__ part) {
-  __shared__ float red[4][256];
+  extern __shared__ char lds[];
+  const int TH = 16 / TD, PD = TD + 2, PH = TH + 2;
+  char *ldy = lds + PD * PH * 18 * 32;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int b = blockIdx.x;
-  const int split = b % nsplit;
-  b /= nsplit;
+  const int kq = lane >> 4, li = lane & 15;
   const int nco = cout >> 4, ncc = cin >> 4;
-  const int ot = b % nco;
-  b /= nco;
-  const int ct = b % ncc;
-  const int t = b / ncc;
-  if (t >= 27) return;
-  const int ti = t / 9 - 1, tj = (t / 3) % 3 - 1, tk = t % 3 - 1;
-  const int ntw = (g.W + 15) >> 4;
-  const int nchunk = g.D * g.H * ntw;
-  const int kq = lane >> 4;
-  const int ci = ct * 16 + (lane & 15);   // A row
-  const int oc = ot * 16 + (lane & 15);   // B column
-  f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-  for (int ch = split * 4 + wv; ch < nchunk; ch += 4 * nsplit) {
-    const int w0 = (ch % ntw) << 4;
-    const int hh = (ch / ntw) % g.H;
-    const int dd = ch / (ntw * g.H);
-    s4 a, bb;
+  const int ct = blockIdx.y % ncc, ot0 = blockIdx.y / ncc * NC;
+  const int ntw = (g.W + 15) >> 4, nth = (g.H + TH - 1) / TH, ntd = (g.D + TD - 1) / TD;
+  const int ntiles = ntw * nth * ntd;
+  const int rowb = 18 * 32, planeb = PH * rowb;
+  // LDS offsets of this lane's two transposed reads (voxels +0..3, +4..7 of
+  // its eight) for each of the wave's taps, relative to the tile row pair
+  int off[7][2];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int w = w0 + 4 * kq + e;
-      float xv = 0.f, dv = 0.f;
-      if (w < g.W) {
-        const size_t v = (size_t)(dd * g.H + hh) * g.W + w;
-        dv = bf2f(dy[v * ldd + doff + oc]);
-        const int zd = dd + ti, zh = hh + tj, zw = w + tk;
-        if (zd >= 0 && zd < g.D && zh >= 0 && zh < g.H && zw >= 0 && zw < g.W)
-          xv = bf2f(x[(size_t)((zd * g.H + zh) * g.W + zw) * ldx + xoff + ci]);
-      }
-      a[e] = (short)f2bf(xv);
-      bb[e] = (short)f2bf(dv);
+  for (int q = 0; q < 7; q++) {
+    const int t = wv + 4 * q < 27 ? wv + 4 * q : 26;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int pw = t % 3 + 8 * (kq & 1) + 4 * u + (li >> 2);
+      off[q][u] = (t / 9) * planeb + ((t / 3) % 3 + (kq >> 1)) * rowb + pw * 32 +
+                  ConvGeo<16>::piece((li & 3) >> 1, pw) + (li & 1) * 8;
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc, 0, 0, 0);
   }
-  // lane holds column o = lane % 16, rows c = 4 (lane / 16) + e
+  const int offd = (16 * (kq >> 1) + 8 * (kq & 1) + (li >> 2)) * NC * 32 + (li & 3) * 8;
+  const short one = (short)0x3f80;
+  f4 acc[7][NC];
 #pragma unroll
-  for (int e = 0; e < 4; e++) red[wv][(4 * kq + e) * 16 + (lane & 15)] = acc[e];
-  __syncthreads();
-  const int i = threadIdx.x;   // 256 = 16 x 16 tile entries
-  const float s = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
-  const int r = i >> 4, c = i & 15;
-  part[((size_t)split * 27 + t) * cin * cout + (size_t)(ct * 16 + r) * cout + ot * 16 + c] = s;
-}
-
-// grad[i] (+)= sum over splits k of part[k * stride + i] (fixed order)
-__global__ void k_wgrad_reduce(const float *__restrict__ part, int nsplit, int n, size_t stride,
-                               float *__restrict__ grad, int accumulate) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int k = 0; k < nsplit; k++) s = s + part[(size_t)k * stride + i];
-    grad[i] = accumulate ? grad[i] + s : s;
+  for (int q = 0; q < 7; q++)
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[q][c] = f4{0.f, 0.f, 0.f, 0.f};
+  typedef __attribute__((address_space(3))) s4 *lp4;
+  auto tr8 = [](const char *p0, const char *p1) {
+    const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp4)p0);
+    const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp4)p1);
+    const s8 v = s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    return __builtin_bit_cast(b8, v);
+  };
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int w0 = (tile % ntw) << 4, h0 = (tile / ntw) % nth * TH, d0 = tile / (ntw * nth) * TD;
+    __syncthreads();
+    stage_halo<16>(lds, g, x, ldx, xoff + ct * 16, d0, h0, w0, PD, PH, mph);
+    for (int i = threadIdx.x; i < 256 * NC * 2; i += 256) {
+      const int q = i % (NC * 2), vox = i / (NC * 2);
+      const int w = w0 + (vox & 15), row = vox >> 4;
+      const int h = h0 + row % TH, d = d0 + row / TH;
+      s8 v = s8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (d < g.D && h < g.H && w < g.W && ot0 + q / 2 < nco)
+        v = *reinterpret_cast<const s8 *>(dy + (size_t)((d * g.H + h) * g.W + w) * ldd + doff +
+                                          ot0 * 16 + 8 * q);
+      *reinterpret_cast<s8 *>(ldy + vox * NC * 32 + q * 16) = v;
+    }
+    __syncthreads();
+    // K = 32 voxels a step: rows (dl, hl) and (dl, hl + 1)
+    for (int st = 0; st < 8; st++) {
+      const int dl = 2 * st / TH, hl = 2 * st % TH;
+      const char *xr = lds + dl * planeb + hl * rowb;
+      const char *dr = ldy + st * 32 * NC * 32 + offd;
+      b8 fd[NC];
+#pragma unroll
+      for (int c = 0; c < NC; c++) fd[c] = tr8(dr + c * 32, dr + c * 32 + 4 * NC * 32);
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        b8 fx = tr8(xr + off[q][0], xr + off[q][1]);
+        if (q == 6 && wv == 3)
+          fx = __builtin_bit_cast(b8, s8{one, one, one, one, one, one, one, one});
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+          acc[q][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fd[c], fx, acc[q][c], 0, 0, 0);
+      }
+    }
+  }
+  // lane: input channel li, output channels 4 kq .. + 3 of each tile
+  float *pt = part + (size_t)blockIdx.x * ((size_t)27 * cin + 1) * cout;
+#pragma unroll
+  for (int q = 0; q < 7; q++) {
+    const int t = wv + 4 * q;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      if (ot0 + c >= nco) break;
+      const int o = (ot0 + c) * 16 + 4 * kq;
+      if (t < 27)
+        *reinterpret_cast<f4 *>(pt + ((size_t)t * cin + ct * 16 + li) * cout + o) = acc[q][c];
+      else if (ct == 0 && li == 0)
+        *reinterpret_cast<f4 *>(pt + (size_t)27 * cin * cout + o) = acc[q][c];
+    }
   }
 }
 
-// bias gradient partials: block b sums voxels b, b + G, ... of channel
-// threadIdx.x % cout (cout <= 256 divides 256)
-__global__ void k_bgrad(int V, const bf16 *__restrict__ dy, int ldd, int doff, int cout,
-                        float *__restrict__ part) {
-  __shared__ float red[256];
-  const int per = 256 / cout;
-  const int o = threadIdx.x % cout, j = threadIdx.x / cout;
+// Gradient of a layer's weights and biases (adjacent in the parameter
+// vector): grad[i] (+)= sum over the splits' partials in split order, the
+// rows cin_real .. cin - 1 of a padded input left out.  Four waves take a
+// quarter of the splits each for 64 values, so the loads of a value's many
+// partials run in parallel; the quarters are added in order.
+__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, int nsplit,
+                                                      int cin, int cin_real, int cout,
+                                                      float *__restrict__ grad, int accumulate) {
+  __shared__ float red[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int nw = 27 * cin_real * cout, n = nw + cout;
+  const size_t stride = ((size_t)27 * cin + 1) * cout;
+  const int i = blockIdx.x * 64 + lane;
   float s = 0.f;
-  if (j < per)
-    for (int v = blockIdx.x * per + j; v < V; v += gridDim.x * per)
-      s = s + bf2f(dy[(size_t)v * ldd + doff + o]);
-  red[threadIdx.x] = s;
-  __syncthreads();
-  if (threadIdx.x < cout) {
-    float t = 0.f;
-    for (int k = 0; k < per; k++) t = t + red[k * cout + threadIdx.x];
-    part[blockIdx.x * cout + threadIdx.x] = t;
+  if (i < n) {
+    int e = i;
+    if (i >= nw) e = 27 * cin * cout + (i - nw);
+    else if (cin_real != cin) {
+      const int t = i / (cin_real * cout);
+      e = t * cin * cout + (i - t * cin_real * cout);
+    }
+    const int k0 = (int)((long long)nsplit * wv / 4), k1 = (int)((long long)nsplit * (wv + 1) / 4);
+#pragma unroll 8
+    for (int k = k0; k < k1; k++) s = s + part[(size_t)k * stride + e];
   }
+  red[wv][lane] = s;
+  __syncthreads();
+  if (wv != 0 || i >= n) return;
+  s = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+  grad[i] = accumulate ? grad[i] + s : s;
 }
 
 // ---------------------------------------------------------------------------
@@ -723,36 +783,60 @@ int launch_conv(UNetHandle *u, const Grid3 &g, const bf16 *x, int ldx, int xoff,
   return MF6HIP_OK;
 }
 
+// Splits of one layer's weight gradient: WG_MAXBLK workgroups over its
+// channel tiles, at most one per voxel tile.  TD: the tile shape (4 x 4, 2 x
+// 8 or 1 x 16 rows of 16 voxels) that pads the grid least.
+struct WgradTile {
+  int NC, gy, TD, nsplit;
+};
+
+WgradTile wgrad_tile(const Grid3 &g, int cin, int cout) {
+  WgradTile t{};
+  const int nco = cout / 16, ng = (nco + 3) / 4;
+  t.NC = (nco + ng - 1) / ng;
+  t.gy = cin / 16 * ng;
+  long long pad = -1;
+  int ntiles = 1;
+  for (int td = 4; td >= 1; td >>= 1) {
+    const int th = 16 / td, nd = (g.D + td - 1) / td, nh = (g.H + th - 1) / th;
+    const long long v = (long long)nd * td * nh * th;
+    if (pad < 0 || v < pad) {
+      pad = v;
+      t.TD = td;
+      ntiles = nd * nh * ((g.W + 15) / 16);
+    }
+  }
+  t.nsplit = (WG_MAXBLK + t.gy - 1) / t.gy;
+  if (t.nsplit > ntiles) t.nsplit = ntiles;
+  return t;
+}
+
+// floats of partials that a layer's weight gradient needs
+size_t wgrad_part(const Grid3 &g, int cin, int cout) {
+  return (size_t)wgrad_tile(g, cin, cout).nsplit * ((size_t)27 * cin + 1) * cout;
+}
+
 // weight + bias gradients of one conv layer into u->grad (accumulate)
 int conv_wgrad(UNetHandle *u, const Grid3 &g, const UConv &L, const bf16 *x, int ldx, int xoff,
                const bf16 *dy, int ldd, int doff, int accumulate) {
   hipStream_t s = u->stream;
-  const int tiles = 27 * (L.cin / 16) * (L.cout / 16);
-  int nsplit = 2048 / tiles;
-  if (nsplit < 1) nsplit = 1;
-  const int nchunk = g.D * g.H * ((g.W + 15) / 16);
-  if (nsplit * 4 > nchunk) nsplit = (nchunk + 3) / 4;
-  if (nsplit < 1) nsplit = 1;
-  const size_t n = (size_t)27 * L.cin * L.cout;
-  if ((size_t)nsplit * n > u->part_n) { mf6hip_set_error("partial buffer too small"); return MF6HIP_EINVAL; }
-  k_wgrad<<<tiles * nsplit, 256, 0, s>>>(g, x, ldx, xoff, L.cin, dy, ldd, doff, L.cout, nsplit,
-                                         u->part);
-  // rows of the padded first layer beyond the real inputs are not
-  // parameters: per tap keep rows 0..cin_real-1 ([27][cin][cout] partials
-  // -> [27][cin_real][cout] gradient)
-  if (L.cin_real == L.cin) {
-    k_wgrad_reduce<<<nblk(n), 256, 0, s>>>(u->part, nsplit, (int)n, n, u->grad + L.w_off,
-                                           accumulate);
-  } else {
-    const size_t nt = (size_t)L.cin_real * L.cout;
-    for (int t = 0; t < 27; t++)
-      k_wgrad_reduce<<<nblk(nt), 256, 0, s>>>(u->part + (size_t)t * L.cin * L.cout, nsplit,
-                                              (int)nt, n, u->grad + L.w_off + t * nt, accumulate);
-  }
-  const int bb = nblk((size_t)g.V());
-  const int nbb = bb > 1024 ? 1024 : bb;
-  k_bgrad<<<nbb, 256, 0, s>>>(g.V(), dy, ldd, doff, L.cout, u->part);
-  k_colsum<<<1, 256, 0, s>>>(u->part, nbb, L.cout, u->grad + L.b_off, accumulate);
+  const WgradTile t = wgrad_tile(g, L.cin, L.cout);
+  if (wgrad_part(g, L.cin, L.cout) > u->part_n) { mf6hip_set_error("partial buffer too small"); return MF6HIP_EINVAL; }
+  const int PD = t.TD + 2, PH = 16 / t.TD + 2;
+  const int shm = PD * PH * 18 * 32 + 256 * t.NC * 32;   // at most 64 KB
+  const int mph = (65536 + PH - 1) / PH;
+  const dim3 grid(t.nsplit, t.gy);
+#define MF6_WGRAD(N)                                                                          \
+  k_wgrad<N><<<grid, 256, shm, s>>>(g, x, ldx, xoff, L.cin, dy, ldd, doff, L.cout, t.TD, mph, \
+                                    u->part)
+  if (t.NC == 1) MF6_WGRAD(1);
+  else if (t.NC == 2) MF6_WGRAD(2);
+  else if (t.NC == 3) MF6_WGRAD(3);
+  else MF6_WGRAD(4);
+#undef MF6_WGRAD
+  const int n = 27 * L.cin_real * L.cout + L.cout;
+  k_wgrad_reduce<<<(n + 63) / 64, 256, 0, s>>>(u->part, t.nsplit, L.cin, L.cin_real, L.cout,
+                                               u->grad + L.w_off, accumulate);
   if (hipGetLastError() != hipSuccess) { mf6hip_set_error("wgrad launch failed"); return MF6HIP_EHIP; }
   return MF6HIP_OK;
 }
@@ -969,15 +1053,12 @@ extern "C" int mf6hip_unet_create(int nlay, int nrow, int ncol, int nin, int nle
   if (!rc) rc = ualloc(&u->grad, off);
   if (!rc) rc = ualloc(&u->m, off);
   if (!rc) rc = ualloc(&u->v, off);
-  // partials: the largest split-K buffer (2048 / tiles splits, at least 1)
+  // partials: the largest layer's weight-gradient splits
   size_t pn = 1 << 20;
   for (int i = 0; i < u->nconv(); i++) {
     const UConv &L = u->conv[i];
-    const size_t n = (size_t)27 * L.cin * L.cout;
-    const int tiles = 27 * (L.cin / 16) * (L.cout / 16);
-    int ns = 2048 / tiles;
-    if (ns < 1) ns = 1;
-    if ((size_t)ns * n > pn) pn = (size_t)ns * n;
+    const int l = i < 2 * nlev ? i / 2 : bot - 1 - (i - 2 * nlev);
+    pn = std::max(pn, wgrad_part(u->g[l], L.cin, L.cout));
   }
   u->part_n = pn;
   if (!rc) rc = ualloc(&u->part, pn);
