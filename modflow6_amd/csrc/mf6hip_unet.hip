@@ -66,8 +66,8 @@ struct Grid3 {
 // 3x3x3 convolution (forward and data gradient)
 // ---------------------------------------------------------------------------
 
-// y[v, yoff + o] = act(bias[o] + sum_{t, c} x[v + off(t), xoff + c] W[t, c, o])
-// act: relu when relu != 0; then y *= (mask[v, moff + o] > 0) when mask != 0.
+// y[v, o] = act(bias[o] + sum_{t, c} x[v + off(t), c] W[t, c, o])
+// act: relu when relu != 0; then y *= (mask[v, o] > 0) when mask != 0.
 //
 // A workgroup of four waves computes WD x (4 / WD) MT x 16 voxels (d, h, w)
 // by NC tiles of 16 output channels (blockIdx.y takes the next NC tiles).
@@ -99,11 +99,23 @@ struct ConvGeo {
   }
 };
 
+// Input of a convolution: the channels of x (stride ldx), preceded for a
+// decoder by the cu channels of a coarse tensor on the 1 x 2 x 2 coarser grid
+// (rows Hc, columns Wc), upsampled to the nearest fine voxel as they are
+// read.  (Writing the upsampled channels out first cost 47 us per decoder
+// level at 16 x 256 x 256 and as much again to read them back.)
+struct ConvSrc {
+  const bf16 *x;
+  int ldx;
+  const bf16 *up = nullptr;
+  int cu = 0, Hc = 0, Wc = 0;
+};
+
 // the halo of channels c0 .. c0 + CW - 1 of the tile at (d0, h0, w0) into
 // LDS, zero outside the grid; PD x PH x 18 voxels, mph = ceil(2^16 / PH)
 template <int CW>
-__device__ inline void stage_halo(char *lds, const Grid3 &g, const bf16 *__restrict__ x, int ldx,
-                                  int c0, int d0, int h0, int w0, int PD, int PH, int mph) {
+__device__ inline void stage_halo(char *lds, const Grid3 &g, const ConvSrc &src, int c0, int d0,
+                                  int h0, int w0, int PD, int PH, int mph) {
   constexpr int P = ConvGeo<CW>::PIECES;
   const int n = PD * PH * 18 * P;
   for (int i = threadIdx.x; i < n; i += 256) {
@@ -112,19 +124,31 @@ __device__ inline void stage_halo(char *lds, const Grid3 &g, const bf16 *__restr
     const int pd = (row * mph) >> 16, ph = row - pd * PH;
     const int d = d0 + pd - 1, h = h0 + ph - 1, w = w0 + pw - 1;
     s8 v = s8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (d >= 0 && d < g.D && h >= 0 && h < g.H && w >= 0 && w < g.W)
-      v = *reinterpret_cast<const s8 *>(x + (size_t)((d * g.H + h) * g.W + w) * ldx + c0 + 8 * q);
+    if (d >= 0 && d < g.D && h >= 0 && h < g.H && w >= 0 && w < g.W) {
+      const int c = c0 + 8 * q;
+      const bf16 *p = c < src.cu
+          ? src.up + (size_t)((d * src.Hc + (h >> 1)) * src.Wc + (w >> 1)) * src.cu + c
+          : src.x + (size_t)((d * g.H + h) * g.W + w) * src.ldx + (c - src.cu);
+      v = *reinterpret_cast<const s8 *>(p);
+    }
     *reinterpret_cast<s8 *>(lds + vox * ConvGeo<CW>::VB + ConvGeo<CW>::piece(q, pw)) = v;
   }
 }
 
+// 1x1x1 output convolution computed with the last decoder convolution (16
+// channels, from its stored BF16 values): yo[v] = sum_c y[v, c] wo[c] + bo
+struct ConvOut1 {
+  const float *wo = nullptr, *bo = nullptr;
+  float *yo = nullptr;
+};
+
 template <int CW, int MT, int NC>
-__global__ void __launch_bounds__(256) k_conv3(Grid3 g, const bf16 *__restrict__ x, int ldx,
-                                               int xoff, int cin, const s8 *__restrict__ wp,
-                                               int nco, const float *__restrict__ bias, int relu,
-                                               bf16 *__restrict__ y, int ldy, int yoff,
-                                               const bf16 *__restrict__ mask, int ldm, int moff,
-                                               int WD, int mph) {
+__global__ void __launch_bounds__(256) k_conv3(Grid3 g, ConvSrc src, int cin,
+                                               const s8 *__restrict__ wp, int nco,
+                                               const float *__restrict__ bias, int relu,
+                                               bf16 *__restrict__ y, int ldy,
+                                               const bf16 *__restrict__ mask, int ldm,
+                                               ConvOut1 o1, int WD, int mph) {
   extern __shared__ char lds[];
   using G = ConvGeo<CW>;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -152,7 +176,7 @@ __global__ void __launch_bounds__(256) k_conv3(Grid3 g, const bf16 *__restrict__
   }
   for (int c0 = 0; c0 < cin; c0 += CW) {
     if (c0) __syncthreads();
-    stage_halo<CW>(lds, g, x, ldx, xoff + c0, d0, h0, w0, PD, PH, mph);
+    stage_halo<CW>(lds, g, src, c0, d0, h0, w0, PD, PH, mph);
     __syncthreads();
     // the weights of a step are loaded while the step before it runs
     b8 wn[3][NC];
@@ -211,7 +235,7 @@ __global__ void __launch_bounds__(256) k_conv3(Grid3 g, const bf16 *__restrict__
       if (ct0 + c >= nco) break;
       const int o = (ct0 + c) * 16 + 4 * kq;
       s4 mk = s4{0, 0, 0, 0}, out;
-      if (mask) mk = *reinterpret_cast<const s4 *>(mask + v * ldm + moff + o);
+      if (mask) mk = *reinterpret_cast<const s4 *>(mask + v * ldm + o);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         float val = acc[m][c][e] + (bias ? bias[o + e] : 0.f);
@@ -219,7 +243,16 @@ __global__ void __launch_bounds__(256) k_conv3(Grid3 g, const bf16 *__restrict__
         if (mask && !(bf2f((bf16)mk[e]) > 0.f)) val = 0.f;
         out[e] = (short)f2bf(val);
       }
-      *reinterpret_cast<s4 *>(y + v * ldy + yoff + o) = out;
+      *reinterpret_cast<s4 *>(y + v * ldy + o) = out;
+      if (o1.yo) {
+        // the four lanes of a voxel hold its 16 channels
+        float t = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) t = t + bf2f((bf16)out[e]) * o1.wo[o + e];
+        t = t + __shfl_xor(t, 16);
+        t = t + __shfl_xor(t, 32);
+        if (kq == 0) o1.yo[v] = t + o1.bo[0];
+      }
     }
   }
 }
@@ -295,10 +328,9 @@ __global__ void k_pack_w(const float *__restrict__ w, int cin_real, int cin, int
 // bias-gradient kernels are gone.
 constexpr int WG_MAXBLK = 512;   // workgroups of one layer's gradient
 template <int NC>
-__global__ void __launch_bounds__(256, 2) k_wgrad(Grid3 g, const bf16 *__restrict__ x, int ldx,
-                                               int xoff, int cin, const bf16 *__restrict__ dy,
-                                               int ldd, int doff, int cout, int TD, int mph,
-                                               float *__restrict__ part) {
+__global__ void __launch_bounds__(256, 2) k_wgrad(Grid3 g, ConvSrc src, int cin,
+                                                  const bf16 *__restrict__ dy, int cout, int TD,
+                                                  int mph, float *__restrict__ part) {
   extern __shared__ char lds[];
   const int TH = 16 / TD, PD = TD + 2, PH = TH + 2;
   char *ldy = lds + PD * PH * 18 * 32;
@@ -339,14 +371,14 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(Grid3 g, const bf16 *__restric
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int w0 = (tile % ntw) << 4, h0 = (tile / ntw) % nth * TH, d0 = tile / (ntw * nth) * TD;
     __syncthreads();
-    stage_halo<16>(lds, g, x, ldx, xoff + ct * 16, d0, h0, w0, PD, PH, mph);
+    stage_halo<16>(lds, g, src, ct * 16, d0, h0, w0, PD, PH, mph);
     for (int i = threadIdx.x; i < 256 * NC * 2; i += 256) {
       const int q = i % (NC * 2), vox = i / (NC * 2);
       const int w = w0 + (vox & 15), row = vox >> 4;
       const int h = h0 + row % TH, d = d0 + row / TH;
       s8 v = s8{0, 0, 0, 0, 0, 0, 0, 0};
       if (d < g.D && h < g.H && w < g.W && ot0 + q / 2 < nco)
-        v = *reinterpret_cast<const s8 *>(dy + (size_t)((d * g.H + h) * g.W + w) * ldd + doff +
+        v = *reinterpret_cast<const s8 *>(dy + (size_t)((d * g.H + h) * g.W + w) * cout +
                                           ot0 * 16 + 8 * q);
       *reinterpret_cast<s8 *>(ldy + vox * NC * 32 + q * 16) = v;
     }
@@ -432,89 +464,78 @@ __device__ __forceinline__ int pool_count(const Grid3 &gf, int hc, int wc) {
   return nh * nw;
 }
 
-// pooled[d, h, w, c] = mean of the fine cells of coarse cell (h, w); c < C
-__global__ void k_pool(Grid3 gc, Grid3 gf, const bf16 *__restrict__ x, int ldx, int xoff, int C,
-                       bf16 *__restrict__ y, int ldy, int yoff) {
-  const int n = gc.V() * C;
+// The elementwise kernels below take eight channels (16 bytes) per thread;
+// C, strides and offsets are multiples of 16.
+__device__ __forceinline__ s8 ld8(const bf16 *p) { return *reinterpret_cast<const s8 *>(p); }
+
+// sum over the fine cells of coarse cell (d, h, w) of x[.., c .. c + 7]
+__device__ __forceinline__ void fine_sum8(const Grid3 &gf, const bf16 *__restrict__ x, int ldx,
+                                          int d, int h, int w, int c, float *s) {
+  const bool hr = 2 * h + 1 < gf.H, wr = 2 * w + 1 < gf.W;
+  const bf16 *p = x + ((size_t)(d * gf.H + 2 * h) * gf.W + 2 * w) * ldx + c;
+  const s8 z = s8{0, 0, 0, 0, 0, 0, 0, 0};
+  const s8 a = ld8(p), b = wr ? ld8(p + ldx) : z;
+  const s8 e = hr ? ld8(p + (size_t)gf.W * ldx) : z, f = hr && wr ? ld8(p + (size_t)(gf.W + 1) * ldx) : z;
+#pragma unroll
+  for (int q = 0; q < 8; q++)
+    s[q] = (bf2f((bf16)a[q]) + bf2f((bf16)b[q])) + (bf2f((bf16)e[q]) + bf2f((bf16)f[q]));
+}
+
+// pooled[v, c] = mean of the fine cells of coarse cell v; c < C
+__global__ void k_pool(Grid3 gc, Grid3 gf, const bf16 *__restrict__ x, int C,
+                       bf16 *__restrict__ y) {
+  const int C8 = C / 8, n = gc.V() * C8;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % C, v = i / C;
+    const int c = i % C8 * 8, v = i / C8;
     const int w = v % gc.W, h = (v / gc.W) % gc.H, d = v / (gc.W * gc.H);
-    const bool hr = 2 * h + 1 < gf.H, wr = 2 * w + 1 < gf.W;
-    const size_t b0 = ((size_t)(d * gf.H + 2 * h) * gf.W + 2 * w);
-    float s = bf2f(x[b0 * ldx + xoff + c]);
-    if (wr) s = s + bf2f(x[(b0 + 1) * ldx + xoff + c]);
-    if (hr) {
-      float t = bf2f(x[(b0 + gf.W) * ldx + xoff + c]);
-      if (wr) t = t + bf2f(x[(b0 + gf.W + 1) * ldx + xoff + c]);
-      s = s + t;
+    float s[8];
+    fine_sum8(gf, x, C, d, h, w, c, s);
+    const float cnt = (float)pool_count(gf, h, w);
+    s8 o;
+#pragma unroll
+    for (int q = 0; q < 8; q++) o[q] = (short)f2bf(s[q] / cnt);
+    *reinterpret_cast<s8 *>(y + (size_t)v * C + c) = o;
+  }
+}
+
+// dx (fine grid) = add + dy (coarse) / count, the pooling gradient on top of
+// the skip's (channels aoff .. of add), masked by (mask > 0)
+__global__ void k_pool_bwd(Grid3 gf, Grid3 gc, const bf16 *__restrict__ dy, int C,
+                           const bf16 *__restrict__ add, int lda, int aoff,
+                           const bf16 *__restrict__ mask, bf16 *__restrict__ dx) {
+  const int C8 = C / 8, n = gf.V() * C8;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int c = i % C8 * 8, v = i / C8;
+    const int w = v % gf.W, h = (v / gf.W) % gf.H, d = v / (gf.W * gf.H);
+    const size_t vc = (size_t)(d * gc.H + h / 2) * gc.W + w / 2;
+    const float cnt = (float)pool_count(gf, h / 2, w / 2);
+    const s8 g = ld8(dy + vc * C + c), a = ld8(add + (size_t)v * lda + aoff + c);
+    const s8 m = ld8(mask + (size_t)v * C + c);
+    s8 o;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const float t = bf2f((bf16)a[q]) + bf2f((bf16)g[q]) / cnt;
+      o[q] = (short)f2bf(bf2f((bf16)m[q]) > 0.f ? t : 0.f);
     }
-    y[(size_t)v * ldy + yoff + c] = f2bf(s / (float)((hr ? 2 : 1) * (wr ? 2 : 1)));
-  }
-}
-
-// dx (fine grid) (+)= dy (coarse) / count, the pooling gradient; then masked
-// by (mask > 0) when mask != 0
-__global__ void k_pool_bwd(Grid3 gf, Grid3 gc, const bf16 *__restrict__ dy, int ldd, int doff,
-                           int C, const bf16 *__restrict__ add, int lda, int aoff,
-                           const bf16 *__restrict__ mask, int ldm, int moff,
-                           bf16 *__restrict__ dx, int ldx, int xoff) {
-  const int n = gf.V() * C;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % C, v = i / C;
-    const int w = v % gf.W, h = (v / gf.W) % gf.H, d = v / (gf.W * gf.H);
-    const size_t vc = (size_t)(d * gc.H + h / 2) * gc.W + w / 2;
-    float g = bf2f(dy[vc * ldd + doff + c]) / (float)pool_count(gf, h / 2, w / 2);
-    if (add) g = bf2f(add[(size_t)v * lda + aoff + c]) + g;
-    if (mask && !(bf2f(mask[(size_t)v * ldm + moff + c]) > 0.f)) g = 0.f;
-    dx[(size_t)v * ldx + xoff + c] = f2bf(g);
-  }
-}
-
-// nearest 1x2x2 upsampling of a coarse tensor into a fine slice
-__global__ void k_up(Grid3 gf, Grid3 gc, const bf16 *__restrict__ x, int ldx, int xoff, int C,
-                     bf16 *__restrict__ y, int ldy, int yoff) {
-  const int n = gf.V() * C;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % C, v = i / C;
-    const int w = v % gf.W, h = (v / gf.W) % gf.H, d = v / (gf.W * gf.H);
-    const size_t vc = (size_t)(d * gc.H + h / 2) * gc.W + w / 2;
-    y[(size_t)v * ldy + yoff + c] = x[vc * ldx + xoff + c];
+    *reinterpret_cast<s8 *>(dx + (size_t)v * C + c) = o;
   }
 }
 
 // coarse gradient of the upsampling: sum over the fine cells of the coarse
-// cell, masked
-__global__ void k_up_bwd(Grid3 gc, Grid3 gf, const bf16 *__restrict__ dy, int ldd, int doff,
-                         int C, const bf16 *__restrict__ add, int lda, int aoff,
-                         const bf16 *__restrict__ mask, int ldm, int moff,
-                         bf16 *__restrict__ dx, int ldx, int xoff) {
-  const int n = gc.V() * C;
+// cell (the first C of ldd channels), masked
+__global__ void k_up_bwd(Grid3 gc, Grid3 gf, const bf16 *__restrict__ dy, int ldd, int C,
+                         const bf16 *__restrict__ mask, bf16 *__restrict__ dx) {
+  const int C8 = C / 8, n = gc.V() * C8;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % C, v = i / C;
+    const int c = i % C8 * 8, v = i / C8;
     const int w = v % gc.W, h = (v / gc.W) % gc.H, d = v / (gc.W * gc.H);
-    const bool hr = 2 * h + 1 < gf.H, wr = 2 * w + 1 < gf.W;
-    const size_t b0 = ((size_t)(d * gf.H + 2 * h) * gf.W + 2 * w);
-    float s = bf2f(dy[b0 * ldd + doff + c]);
-    if (wr) s = s + bf2f(dy[(b0 + 1) * ldd + doff + c]);
-    if (hr) {
-      float t = bf2f(dy[(b0 + gf.W) * ldd + doff + c]);
-      if (wr) t = t + bf2f(dy[(b0 + gf.W + 1) * ldd + doff + c]);
-      s = s + t;
-    }
-    if (add) s = bf2f(add[(size_t)v * lda + aoff + c]) + s;
-    if (mask && !(bf2f(mask[(size_t)v * ldm + moff + c]) > 0.f)) s = 0.f;
-    dx[(size_t)v * ldx + xoff + c] = f2bf(s);
-  }
-}
-
-// 1x1x1 output convolution y[v] = sum_c u[v, c] wo[c] + bo (fp32 out)
-__global__ void k_out(int V, const bf16 *__restrict__ u, int ldu, int C,
-                      const float *__restrict__ wo, const float *__restrict__ bo,
-                      float *__restrict__ y) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int c = 0; c < C; c++) s = s + bf2f(u[(size_t)v * ldu + c]) * wo[c];
-    y[v] = s + bo[0];
+    float s[8];
+    fine_sum8(gf, dy, ldd, d, h, w, c, s);
+    const s8 m = ld8(mask + (size_t)v * C + c);
+    s8 o;
+#pragma unroll
+    for (int q = 0; q < 8; q++) o[q] = (short)f2bf(bf2f((bf16)m[q]) > 0.f ? s[q] : 0.f);
+    *reinterpret_cast<s8 *>(dx + (size_t)v * C + c) = o;
   }
 }
 
@@ -545,54 +566,88 @@ __global__ void k_loss(int V, const float *__restrict__ y, const bf16 *__restric
   }
 }
 
-__global__ void k_loss_final(const float *__restrict__ part, int nb, float *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// one block: the sums of both columns of the nb partials (fixed order)
+__global__ void __launch_bounds__(256) k_loss_final(const float *__restrict__ part, int nb,
+                                                    float *__restrict__ out) {
+  __shared__ float red[2][4];
   float a = 0.f, b = 0.f;
-  for (int i = 0; i < nb; i++) {
+  for (int i = threadIdx.x; i < nb; i += 256) {
     a = a + part[2 * i];
     b = b + part[2 * i + 1];
   }
+  for (int o = 32; o > 0; o >>= 1) {
+    a = a + __shfl_xor(a, o);
+    b = b + __shfl_xor(b, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = a;
+    red[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  a = ((red[0][0] + red[0][1]) + red[0][2]) + red[0][3];
+  b = ((red[1][0] + red[1][1]) + red[1][2]) + red[1][3];
   out[0] = a / b;   // loss
   out[1] = b;       // sum t^2
 }
 
-// output-layer backward: g = 2 (y - t) / sum t^2 ; du[v, c] = g wo[c] masked
-// by u > 0 ; partials of d wo[c] = sum_v g u[v, c] and d bo = sum_v g
-__global__ void k_out_bwd(int V, const float *__restrict__ y, const bf16 *__restrict__ t,
-                          int ldt, int toff, const float *__restrict__ lossv,
-                          const bf16 *__restrict__ u, int ldu, int C,
-                          const float *__restrict__ wo, bf16 *__restrict__ du,
-                          float *__restrict__ part) {
-  __shared__ float red[256][17];
+// output-layer backward (16 channels): g = 2 (y - t) / sum t^2 ; du[v, c] =
+// g wo[c] masked by u > 0 ; partials of d wo[c] = sum_v g u[v, c] and d bo =
+// sum_v g, part[block * 17 + c]
+__global__ void __launch_bounds__(256) k_out_bwd(int V, const float *__restrict__ y,
+                                                 const bf16 *__restrict__ t, int ldt, int toff,
+                                                 const float *__restrict__ lossv,
+                                                 const bf16 *__restrict__ u,
+                                                 const float *__restrict__ wo,
+                                                 bf16 *__restrict__ du,
+                                                 float *__restrict__ part) {
+  __shared__ float red[4][17];
   float acc[17];
-  for (int c = 0; c <= C; c++) acc[c] = 0.f;
+#pragma unroll
+  for (int c = 0; c < 17; c++) acc[c] = 0.f;
   const float sc = 2.f / lossv[1];
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x) {
     const float g = sc * (y[v] - bf2f(t[(size_t)v * ldt + toff]));
-    for (int c = 0; c < C; c++) {
-      const float uv = bf2f(u[(size_t)v * ldu + c]);
-      acc[c] = acc[c] + g * uv;
-      du[(size_t)v * C + c] = f2bf(uv > 0.f ? g * wo[c] : 0.f);
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+      const s8 uv = ld8(u + (size_t)v * 16 + 8 * p);
+      s8 o;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const float x = bf2f((bf16)uv[q]);
+        acc[8 * p + q] = acc[8 * p + q] + g * x;
+        o[q] = (short)f2bf(x > 0.f ? g * wo[8 * p + q] : 0.f);
+      }
+      *reinterpret_cast<s8 *>(du + (size_t)v * 16 + 8 * p) = o;
     }
-    acc[C] = acc[C] + g;
+    acc[16] = acc[16] + g;
   }
-  for (int c = 0; c <= C; c++) red[threadIdx.x][c] = acc[c];
+#pragma unroll
+  for (int c = 0; c < 17; c++) {
+    for (int o = 32; o > 0; o >>= 1) acc[c] = acc[c] + __shfl_xor(acc[c], o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][c] = acc[c];
+  }
   __syncthreads();
-  if ((int)threadIdx.x <= C) {
-    float s = 0.f;
-    for (int k = 0; k < (int)blockDim.x; k++) s = s + red[k][threadIdx.x];
-    part[blockIdx.x * (C + 1) + threadIdx.x] = s;
+  if (threadIdx.x < 17) {
+    const int c = threadIdx.x;
+    part[blockIdx.x * 17 + c] = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
   }
 }
 
-// sum of per-block partial rows: out[j] (+)= sum_b part[b * n + j]
-__global__ void k_colsum(const float *__restrict__ part, int nb, int n, float *__restrict__ out,
-                         int accumulate) {
-  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int b = 0; b < nb; b++) s = s + part[(size_t)b * n + j];
-    out[j] = accumulate ? out[j] + s : s;
-  }
+// sum of per-block partial rows, one block per column: out[j] (+)= sum_b
+// part[b * n + j] (fixed order)
+__global__ void __launch_bounds__(256) k_colsum(const float *__restrict__ part, int nb, int n,
+                                                float *__restrict__ out, int accumulate) {
+  __shared__ float red[4];
+  const int j = blockIdx.x;
+  float s = 0.f;
+  for (int b = threadIdx.x; b < nb; b += 256) s = s + part[(size_t)b * n + j];
+  for (int o = 32; o > 0; o >>= 1) s = s + __shfl_xor(s, o);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  s = ((red[0] + red[1]) + red[2]) + red[3];
+  out[j] = accumulate ? out[j] + s : s;
 }
 
 // Adam (bias-corrected) on fp32 master parameters; grads scaled by gscale
@@ -609,23 +664,30 @@ __global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g
   }
 }
 
-// network input: channel 0..nin-1 from fp32 natural-order planes, rest 0
+// network input (16 channels, one voxel per thread): channels 0..nin-1 from
+// fp32 natural-order planes, rest 0
 __global__ void k_make_input(int V, int nin, const float *__restrict__ src,
-                             bf16 *__restrict__ x, int ldx) {
-  const int n = V * ldx;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % ldx, v = i / ldx;
-    x[i] = c < nin ? f2bf(src[(size_t)c * V + v]) : (bf16)0;
+                             bf16 *__restrict__ x) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+      s8 o;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int c = 8 * p + q;
+        o[q] = c < nin ? (short)f2bf(src[(size_t)c * V + v]) : (short)0;
+      }
+      *reinterpret_cast<s8 *>(x + (size_t)v * 16 + 8 * p) = o;
+    }
   }
 }
 
 // a training sample (bf16, [V][4]: 3 inputs + target) into the padded input
-__global__ void k_expand_sample(int V, const bf16 *__restrict__ s, bf16 *__restrict__ x,
-                                int ldx) {
-  const int n = V * ldx;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = i % ldx, v = i / ldx;
-    x[i] = c < 3 ? s[(size_t)v * 4 + c] : (bf16)0;
+__global__ void k_expand_sample(int V, const bf16 *__restrict__ s, bf16 *__restrict__ x) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += gridDim.x * blockDim.x) {
+    const s4 a = *reinterpret_cast<const s4 *>(s + (size_t)v * 4);
+    *reinterpret_cast<s8 *>(x + (size_t)v * 16) = s8{a[0], a[1], a[2], 0, 0, 0, 0, 0};
+    *reinterpret_cast<s8 *>(x + (size_t)v * 16 + 8) = s8{0, 0, 0, 0, 0, 0, 0, 0};
   }
 }
 
@@ -667,8 +729,7 @@ struct UNetHandle {
   bf16 *in0 = nullptr;                 // level-0 input, 16 channels
   bf16 *pin[MAXLEV] = {};              // pooled inputs (levels 1..nlev-1)
   bf16 *ha[MAXLEV] = {};               // first conv output
-  bf16 *cat[MAXLEV] = {};              // decoder inputs [up | skip] (levels < nlev-1)
-  bf16 *hbot = nullptr;                // bottom level output
+  bf16 *hb[MAXLEV] = {};               // second conv output (the skips; the bottom output)
   bf16 *u[MAXLEV] = {};                // decoder outputs (levels < nlev-1)
   float *y = nullptr;                  // fp32 output
   float *lossv = nullptr;              // [2]
@@ -682,8 +743,17 @@ struct UNetHandle {
   int nconv() const { return 3 * nlev - 1; }
   // decoder conv of level l (< nlev - 1)
   int dconv(int l) const { return 2 * nlev + (nlev - 2 - l); }
-  // channels of the upsampled part of cat[l]
+  // channels of the upsampled part of a decoder's input
   int cup(int l) const { return ch[l + 1]; }
+  // input of level l's decoder: the coarser output upsampled, then the skip
+  ConvSrc dec_src(int l) const {
+    return ConvSrc{hb[l], ch[l], l == nlev - 2 ? hb[l + 1] : this->u[l + 1], ch[l + 1],
+                   g[l + 1].H, g[l + 1].W};
+  }
+  // input of level l's first convolution
+  ConvSrc enc_src(int l) const {
+    return l == 0 ? ConvSrc{in0, 16} : ConvSrc{pin[l], ch[l - 1]};
+  }
 };
 
 namespace {
@@ -738,13 +808,12 @@ ConvTile conv_tile(const Grid3 &g, int nco) {
 }
 
 template <int CW, int MT>
-void launch_conv_nc(int nc, dim3 grid, int shm, hipStream_t s, const Grid3 &g, const bf16 *x,
-                    int ldx, int xoff, int cin, const s8 *wp, int nco, const float *bias, int relu,
-                    bf16 *y, int ldy, int yoff, const bf16 *mask, int ldm, int moff, int WD,
-                    int mph) {
-#define MF6_CONV(N)                                                                            \
-  k_conv3<CW, MT, N><<<grid, 256, shm, s>>>(g, x, ldx, xoff, cin, wp, nco, bias, relu, y, ldy, \
-                                            yoff, mask, ldm, moff, WD, mph)
+void launch_conv_nc(int nc, dim3 grid, int shm, hipStream_t s, const Grid3 &g, const ConvSrc &src,
+                    int cin, const s8 *wp, int nco, const float *bias, int relu, bf16 *y, int ldy,
+                    const bf16 *mask, int ldm, const ConvOut1 &o1, int WD, int mph) {
+#define MF6_CONV(N)                                                                             \
+  k_conv3<CW, MT, N><<<grid, 256, shm, s>>>(g, src, cin, wp, nco, bias, relu, y, ldy, mask, ldm, \
+                                            o1, WD, mph)
   if (nc == 1) MF6_CONV(1);
   else if (nc == 2) MF6_CONV(2);
   else if (nc == 3) MF6_CONV(3);
@@ -752,9 +821,9 @@ void launch_conv_nc(int nc, dim3 grid, int shm, hipStream_t s, const Grid3 &g, c
 #undef MF6_CONV
 }
 
-int launch_conv(UNetHandle *u, const Grid3 &g, const bf16 *x, int ldx, int xoff, int cin,
-                const s8 *wp, int cout, const float *bias, int relu, bf16 *y, int ldy, int yoff,
-                const bf16 *mask, int ldm, int moff) {
+int launch_conv(UNetHandle *u, const Grid3 &g, const ConvSrc &src, int cin, const s8 *wp, int cout,
+                const float *bias, int relu, bf16 *y, const bf16 *mask,
+                const ConvOut1 &o1 = ConvOut1{}) {
   if (cin % 16 || cout % 16 || cout > 256) {
     mf6hip_set_error("unsupported channel count " + std::to_string(cout));
     return MF6HIP_EUNSUPPORTED;
@@ -767,8 +836,8 @@ int launch_conv(UNetHandle *u, const Grid3 &g, const bf16 *x, int ldx, int xoff,
   const dim3 grid(t.tiles, t.gy);
   hipStream_t s = u->stream;
 #define MF6_CONV(C, M)                                                                           \
-  launch_conv_nc<C, M>(t.NC, grid, shm, s, g, x, ldx, xoff, cin, wp, nco, bias, relu, y, ldy,    \
-                       yoff, mask, ldm, moff, t.WD, mph)
+  launch_conv_nc<C, M>(t.NC, grid, shm, s, g, src, cin, wp, nco, bias, relu, y, cout, mask, cout, \
+                       o1, t.WD, mph)
   if (cw == 32) {
     if (t.MT == 4) MF6_CONV(32, 4);
     else if (t.MT == 2) MF6_CONV(32, 2);
@@ -817,8 +886,8 @@ size_t wgrad_part(const Grid3 &g, int cin, int cout) {
 }
 
 // weight + bias gradients of one conv layer into u->grad (accumulate)
-int conv_wgrad(UNetHandle *u, const Grid3 &g, const UConv &L, const bf16 *x, int ldx, int xoff,
-               const bf16 *dy, int ldd, int doff, int accumulate) {
+int conv_wgrad(UNetHandle *u, const Grid3 &g, const UConv &L, const ConvSrc &src, const bf16 *dy,
+               int accumulate) {
   hipStream_t s = u->stream;
   const WgradTile t = wgrad_tile(g, L.cin, L.cout);
   if (wgrad_part(g, L.cin, L.cout) > u->part_n) { mf6hip_set_error("partial buffer too small"); return MF6HIP_EINVAL; }
@@ -827,8 +896,7 @@ int conv_wgrad(UNetHandle *u, const Grid3 &g, const UConv &L, const bf16 *x, int
   const int mph = (65536 + PH - 1) / PH;
   const dim3 grid(t.nsplit, t.gy);
 #define MF6_WGRAD(N)                                                                          \
-  k_wgrad<N><<<grid, 256, shm, s>>>(g, x, ldx, xoff, L.cin, dy, ldd, doff, L.cout, t.TD, mph, \
-                                    u->part)
+  k_wgrad<N><<<grid, 256, shm, s>>>(g, src, L.cin, dy, L.cout, t.TD, mph, u->part)
   if (t.NC == 1) MF6_WGRAD(1);
   else if (t.NC == 2) MF6_WGRAD(2);
   else if (t.NC == 3) MF6_WGRAD(3);
@@ -868,39 +936,21 @@ static int u_forward(UNetHandle *u) {
   const int nl = u->nlev, bot = nl - 1;
   for (int l = 0; l < nl; l++) {
     const Grid3 &g = u->g[l];
-    const bf16 *xin;
-    int ldx, cin;
-    if (l == 0) { xin = u->in0; ldx = 16; cin = 16; }
-    else {
-      // pool hb_{l-1} (in cat[l-1] at offset cup(l-1)) into pin[l]
-      const int cprev = c[l - 1], cu = u->cup(l - 1);
-      k_pool<<<nblk((size_t)g.V() * cprev), 256, 0, s>>>(g, u->g[l - 1], u->cat[l - 1],
-                                                          cu + cprev, cu, cprev, u->pin[l],
-                                                          cprev, 0);
-      xin = u->pin[l]; ldx = cprev; cin = cprev;
-    }
+    if (l > 0)
+      k_pool<<<nblk((size_t)g.V() * c[l - 1] / 8), 256, 0, s>>>(g, u->g[l - 1], u->hb[l - 1],
+                                                                c[l - 1], u->pin[l]);
     const UConv &A = u->conv[2 * l], &B = u->conv[2 * l + 1];
-    UCK(launch_conv(u, g, xin, ldx, 0, cin, A.wp, A.cout, u->p + A.b_off, 1, u->ha[l], c[l], 0,
-                    nullptr, 0, 0));
-    bf16 *hb = l < bot ? u->cat[l] : u->hbot;
-    const int ldh = l < bot ? u->cup(l) + c[l] : c[bot];
-    const int offh = l < bot ? u->cup(l) : 0;
-    UCK(launch_conv(u, g, u->ha[l], c[l], 0, c[l], B.wp, B.cout, u->p + B.b_off, 1, hb, ldh, offh,
-                    nullptr, 0, 0));
+    UCK(launch_conv(u, g, u->enc_src(l), A.cin, A.wp, A.cout, u->p + A.b_off, 1, u->ha[l], nullptr));
+    UCK(launch_conv(u, g, ConvSrc{u->ha[l], c[l]}, B.cin, B.wp, B.cout, u->p + B.b_off, 1, u->hb[l],
+                    nullptr));
   }
   for (int l = bot - 1; l >= 0; l--) {
-    const Grid3 &g = u->g[l];
-    const int cu = u->cup(l), ldc = cu + c[l];
-    const bf16 *src = l == bot - 1 ? u->hbot : u->u[l + 1];
-    k_up<<<nblk((size_t)g.V() * cu), 256, 0, s>>>(g, u->g[l + 1], src, cu, 0, cu, u->cat[l],
-                                                   ldc, 0);
     const UConv &D = u->conv[u->dconv(l)];
-    UCK(launch_conv(u, g, u->cat[l], ldc, 0, ldc, D.wp, D.cout, u->p + D.b_off, 1, u->u[l], c[l],
-                    0, nullptr, 0, 0));
+    ConvOut1 o1;
+    if (l == 0) o1 = ConvOut1{u->p + u->wo_off, u->p + u->bo_off, u->y};
+    UCK(launch_conv(u, u->g[l], u->dec_src(l), D.cin, D.wp, D.cout, u->p + D.b_off, 1, u->u[l],
+                    nullptr, o1));
   }
-  const Grid3 &g0 = u->g[0];
-  k_out<<<nblk(g0.V()), 256, 0, s>>>(g0.V(), u->u[0], c[0], c[0], u->p + u->wo_off,
-                                     u->p + u->bo_off, u->y);
   if (hipGetLastError() != hipSuccess) { mf6hip_set_error("forward launch failed"); return MF6HIP_EHIP; }
   return MF6HIP_OK;
 }
@@ -911,29 +961,26 @@ static int u_backward(UNetHandle *u, const bf16 *tgt, int ldt, int toff, int acc
   hipStream_t s = u->stream;
   const int *c = u->ch;
   const int nl = u->nlev, bot = nl - 1;
-  const Grid3 &g0 = u->g[0];
-  const int V0 = g0.V();
+  const int V0 = u->g[0].V();
   const int nb = nblk(V0) > 1024 ? 1024 : nblk(V0);
   k_loss<<<nb, 256, 0, s>>>(V0, u->y, tgt, ldt, toff, u->part);
-  k_loss_final<<<1, 64, 0, s>>>(u->part, nb, u->lossv);
-  k_out_bwd<<<nb, 256, 0, s>>>(V0, u->y, tgt, ldt, toff, u->lossv, u->u[0], c[0], c[0],
-                               u->p + u->wo_off, u->gu[0], u->part);
-  k_colsum<<<1, 256, 0, s>>>(u->part, nb, c[0] + 1, u->grad + u->wo_off, accumulate);
+  k_loss_final<<<1, 256, 0, s>>>(u->part, nb, u->lossv);
+  k_out_bwd<<<nb, 256, 0, s>>>(V0, u->y, tgt, ldt, toff, u->lossv, u->u[0], u->p + u->wo_off,
+                               u->gu[0], u->part);
+  k_colsum<<<c[0] + 1, 256, 0, s>>>(u->part, nb, c[0] + 1, u->grad + u->wo_off, accumulate);
   // decoder, top to bottom
   for (int l = 0; l < bot; l++) {
     const Grid3 &g = u->g[l];
     const int cu = u->cup(l), ldc = cu + c[l];
     const UConv &D = u->conv[u->dconv(l)];
-    UCK(conv_wgrad(u, g, D, u->cat[l], ldc, 0, u->gu[l], c[l], 0, accumulate));
-    UCK(launch_conv(u, g, u->gu[l], c[l], 0, c[l], D.wt, ldc, nullptr, 0, u->gcat[l], ldc, 0,
-                    nullptr, 0, 0));
+    UCK(conv_wgrad(u, g, D, u->dec_src(l), u->gu[l], accumulate));
+    UCK(launch_conv(u, g, ConvSrc{u->gu[l], c[l]}, c[l], D.wt, ldc, nullptr, 0, u->gcat[l], nullptr));
     const Grid3 &gc = u->g[l + 1];
     // gradient of the coarser decoder output (or of the bottom output)
     // through the upsampling, masked by that output > 0
-    const bf16 *msk = l < bot - 1 ? u->u[l + 1] : u->hbot;
+    const bf16 *msk = l < bot - 1 ? u->u[l + 1] : u->hb[bot];
     bf16 *dst = l < bot - 1 ? u->gu[l + 1] : u->ghb[bot];
-    k_up_bwd<<<nblk((size_t)gc.V() * cu), 256, 0, s>>>(gc, g, u->gcat[l], ldc, 0, cu, nullptr,
-                                                        0, 0, msk, cu, 0, dst, cu, 0);
+    k_up_bwd<<<nblk((size_t)gc.V() * cu / 8), 256, 0, s>>>(gc, g, u->gcat[l], ldc, cu, msk, dst);
   }
   // encoder, bottom to top
   for (int l = bot; l >= 0; l--) {
@@ -942,21 +989,16 @@ static int u_backward(UNetHandle *u, const bf16 *tgt, int ldt, int toff, int acc
       // hb_l gradient: skip part of gcat[l] + pooled gradient from level l+1,
       // masked by hb_l > 0
       const int cu = u->cup(l), ldc = cu + c[l];
-      k_pool_bwd<<<nblk((size_t)g.V() * c[l]), 256, 0, s>>>(g, u->g[l + 1], u->gpin[l + 1], c[l],
-                                                             0, c[l], u->gcat[l], ldc, cu,
-                                                             u->cat[l], ldc, cu, u->ghb[l], c[l],
-                                                             0);
+      k_pool_bwd<<<nblk((size_t)g.V() * c[l] / 8), 256, 0, s>>>(g, u->g[l + 1], u->gpin[l + 1],
+                                                                c[l], u->gcat[l], ldc, cu,
+                                                                u->hb[l], u->ghb[l]);
     }
     const UConv &A = u->conv[2 * l], &B = u->conv[2 * l + 1];
-    UCK(conv_wgrad(u, g, B, u->ha[l], c[l], 0, u->ghb[l], c[l], 0, accumulate));
-    UCK(launch_conv(u, g, u->ghb[l], c[l], 0, c[l], B.wt, c[l], nullptr, 0, u->gha[l], c[l], 0,
-                    u->ha[l], c[l], 0));
-    const bf16 *xin = l == 0 ? u->in0 : u->pin[l];
-    const int ldx = l == 0 ? 16 : c[l - 1];
-    UCK(conv_wgrad(u, g, A, xin, ldx, 0, u->gha[l], c[l], 0, accumulate));
-    if (l > 0)
-      UCK(launch_conv(u, g, u->gha[l], c[l], 0, c[l], A.wt, c[l - 1], nullptr, 0, u->gpin[l],
-                      c[l - 1], 0, nullptr, 0, 0));
+    const ConvSrc ha{u->ha[l], c[l]}, ghb{u->ghb[l], c[l]}, gha{u->gha[l], c[l]};
+    UCK(conv_wgrad(u, g, B, ha, u->ghb[l], accumulate));
+    UCK(launch_conv(u, g, ghb, c[l], B.wt, c[l], nullptr, 0, u->gha[l], u->ha[l]));
+    UCK(conv_wgrad(u, g, A, u->enc_src(l), u->gha[l], accumulate));
+    if (l > 0) UCK(launch_conv(u, g, gha, c[l], A.wt, c[l - 1], nullptr, 0, u->gpin[l], nullptr));
   }
   if (hipGetLastError() != hipSuccess) { mf6hip_set_error("backward launch failed"); return MF6HIP_EHIP; }
   return MF6HIP_OK;
@@ -975,12 +1017,12 @@ static int u_adam(UNetHandle *u, float lr, float gscale) {
 static void u_free(UNetHandle *u) {
   if (!u) return;
   if (u->stream) hipStreamSynchronize(u->stream);
-  void *bufs[] = {u->p, u->grad, u->m, u->v, u->part, u->in0, u->hbot, u->y, u->lossv, u->data};
+  void *bufs[] = {u->p, u->grad, u->m, u->v, u->part, u->in0, u->y, u->lossv, u->data};
   for (void *b : bufs)
     if (b) hipFree(b);
   for (int l = 0; l < MAXLEV; l++) {
     void *b2[] = {u->pin[l], u->ha[l], u->ghb[l], u->gha[l], u->gpin[l],
-                  u->cat[l], u->u[l], u->gu[l], u->gcat[l]};
+                  u->hb[l], u->u[l], u->gu[l], u->gcat[l]};
     for (void *b : b2)
       if (b) hipFree(b);
   }
@@ -1073,13 +1115,12 @@ extern "C" int mf6hip_unet_create(int nlay, int nrow, int ncol, int nin, int nle
     if (!rc) rc = ualloc(&u->ghb[l], V * c[l]);
     if (!rc) rc = ualloc(&u->gha[l], V * c[l]);
     if (!rc && l > 0) rc = ualloc(&u->gpin[l], V * c[l - 1]);
+    if (!rc) rc = ualloc(&u->hb[l], V * c[l]);
     if (!rc && l < bot) {
-      rc = ualloc(&u->cat[l], V * (u->cup(l) + c[l]));
-      if (!rc) rc = ualloc(&u->u[l], V * c[l]);
+      rc = ualloc(&u->u[l], V * c[l]);
       if (!rc) rc = ualloc(&u->gu[l], V * c[l]);
       if (!rc) rc = ualloc(&u->gcat[l], V * (u->cup(l) + c[l]));
     }
-    if (!rc && l == bot) rc = ualloc(&u->hbot, V * c[bot]);
   }
   if (!rc && hipStreamCreateWithFlags(&u->stream, hipStreamNonBlocking) != hipSuccess) {
     mf6hip_set_error("hipStreamCreate failed");
@@ -1144,7 +1185,7 @@ extern "C" int mf6hip_unet_forward(void *handle, const float *x, float *y) {
   UCK(ualloc(&dx, (size_t)V0 * u->nin));
   int rc = MF6HIP_OK;
   if (hipMemcpyAsync(dx, x, sizeof(float) * V0 * u->nin, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
-  if (!rc) k_make_input<<<nblk((size_t)V0 * 16), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0, 16);
+  if (!rc) k_make_input<<<nblk(V0), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0);
   if (!rc) rc = u_forward(u);
   if (!rc && hipMemcpyAsync(y, u->y, sizeof(float) * V0, hipMemcpyDeviceToHost, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (hipStreamSynchronize(u->stream) != hipSuccess && !rc) rc = MF6HIP_EHIP;
@@ -1166,7 +1207,7 @@ extern "C" int mf6hip_unet_grad(void *handle, const float *x, const float *t, fl
   if (!rc && hipMemcpyAsync(dx, x, sizeof(float) * V0 * u->nin, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (!rc && hipMemcpyAsync(dx + (size_t)V0 * u->nin, t, sizeof(float) * V0, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (!rc) {
-    k_make_input<<<nblk((size_t)V0 * 16), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0, 16);
+    k_make_input<<<nblk(V0), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0);
     k_f32_to_bf16<<<nblk(V0), 256, 0, u->stream>>>(V0, dx + (size_t)V0 * u->nin, dt);
     rc = u_forward(u);
   }
@@ -1222,7 +1263,7 @@ extern "C" int mf6hip_unet_train(void *handle, int nsteps, int batch, const int 
       const int idx = order[st * batch + b];
       if (idx < 0 || idx >= u->nsamples) { mf6hip_set_error("sample index out of range"); rc = MF6HIP_EINVAL; break; }
       const bf16 *smp = u->data + (size_t)idx * V0 * 4;
-      k_expand_sample<<<nblk(V0 * 16), 256, 0, u->stream>>>((int)V0, smp, u->in0, 16);
+      k_expand_sample<<<nblk(V0), 256, 0, u->stream>>>((int)V0, smp, u->in0);
       rc = u_forward(u);
       if (!rc) rc = u_backward(u, smp, 4, 3, b > 0);
       if (!rc && hipMemcpyAsync(dl + (size_t)st * batch + b, u->lossv, sizeof(float), hipMemcpyDeviceToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
