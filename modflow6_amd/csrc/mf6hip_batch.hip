@@ -790,7 +790,7 @@ struct BatchHandle {
   unsigned *tl_cmask = nullptr;
   double *tl_colsum = nullptr, *tl_rc = nullptr;
   float *tl_yc = nullptr, *tl_A32 = nullptr;
-  double *tl_S3 = nullptr, *tl_Lc = nullptr, *tl_Lr = nullptr, *tl_G = nullptr;
+  double *tl_S3 = nullptr, *tl_Fi = nullptr, *tl_Gi = nullptr, *tl_Xd = nullptr;
   int *tl_dinfo = nullptr;
   GTask *dtg = nullptr;
   int ntg = 0;
@@ -1096,10 +1096,10 @@ extern "C" int mf6hip_batch_finalize(void *handle) {
     BCK(balloc(&b->tl_rc, b->cvtot));
     BCK(balloc(&b->tl_yc, b->cvtot));
     BCK(balloc(&b->tl_A32, b->aitot));
-    BCK(balloc(&b->tl_S3, 3 * (size_t)b->maxnc));
-    BCK(balloc(&b->tl_Lc, 64 * (size_t)b->maxnc));
-    BCK(balloc(&b->tl_Lr, 64 * (size_t)b->maxnc));
-    BCK(balloc(&b->tl_G, (size_t)b->maxnc * b->maxld));
+    BCK(balloc(&b->tl_S3, 7 * (size_t)b->maxnc));
+    BCK(balloc(&b->tl_Fi, 64 * (size_t)b->maxnc));
+    BCK(balloc(&b->tl_Gi, 64 * (size_t)b->maxnc));
+    BCK(balloc(&b->tl_Xd, 64 * (size_t)b->maxnc));
     BCK(balloc(&b->tl_dinfo, 1));
   }
   BCK(build_tiles(b, 1));
@@ -1144,7 +1144,7 @@ extern "C" int mf6hip_batch_set_system(void *handle, int isys, const int *ia, co
     HIPCHK(hipEventRecord(e0, b->stream));
     int info = 0;
     BCK(mf6hip_tl_setup_slice(S.L, b->A64 + S.aoff, S.tl, b->tl_cmask + S.cmo, b->tl_S3,
-                              b->tl_Lc, b->tl_Lr, b->tl_G, b->tl_A32 + S.aio, b->tl_dinfo,
+                              b->tl_Fi, b->tl_Gi, b->tl_Xd, b->tl_A32 + S.aio, b->tl_dinfo,
                               &info, b->stream));
     HIPCHK(hipEventRecord(e1, b->stream));
     HIPCHK(hipEventSynchronize(e1));
@@ -1304,8 +1304,8 @@ extern "C" int mf6hip_batch_destroy(void *handle) {
   batch_free_tilesets(b);
   void *bufs[] = {b->A64, b->b64, b->x64, b->x0, b->piv64, b->A32, b->piv32, b->d32, b->z32, b->zf32,
                   b->q32, b->p0, b->p1, b->e32, b->st, b->fs, b->active, b->rtrue, b->dtg, b->tl_cmask,
-                  b->tl_colsum, b->tl_rc, b->tl_yc, b->tl_A32, b->tl_S3, b->tl_Lc, b->tl_Lr,
-                  b->tl_G, b->tl_dinfo};
+                  b->tl_colsum, b->tl_rc, b->tl_yc, b->tl_A32, b->tl_S3, b->tl_Fi, b->tl_Gi,
+                  b->tl_Xd, b->tl_dinfo};
   for (void *p : bufs)
     if (p) hipFree(p);
   if (b->h_st) hipHostFree(b->h_st);

@@ -17,12 +17,8 @@
 //   k_tl_cmask     per column: bit k set when cell (k, column) is coupled
 //   k_tl_build     one block per aggregate: its row of S = -Ac (diagonal,
 //                  west and north couplings on the aggregate grid)
-//   k_tl_band_chol S = L L^T in one workgroup: S is banded (bandwidth naj,
-//                  the aggregate grid's width), so L is too; the trailing
-//                  window of the right-looking factorisation lives in LDS
-//   k_tl_band_inv  one wavefront per column j of S^-1: banded forward and
-//                  backward substitution of e_j, the band held across lanes
-//   k_tl_finish_rows  Ainv = -S^-1, FP64 or FP32
+//   k_tl_chain, k_tl_diag, k_tl_prop  Ainv = -S^-1, FP64 or FP32, by block
+//                  elimination over the aggregate rows
 // (aggregate grids wider than 63 take rocSOLVER's dense dpotrf + dpotri)
 // Per CG iteration (after the preconditioner kernels, before the round):
 //   the black / red backward preconditioner kernels write each column's sum
@@ -44,6 +40,7 @@
 
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "mf6hip_handle.h"
@@ -142,15 +139,6 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_tl_build(Layout L, const double *
   S3[3 * I + 2] = (cnt != 0.0 && ai > 0) ? -sn : 0.0;
 }
 
-// lower-band entry S(i, l), l <= i, from the compact rows
-__device__ inline double s_entry(const TwoLevel &T, const double *S3, int i, int l) {
-  double v = 0.0;
-  if (l == i) v = S3[3 * i];
-  if (l == i - 1) v = v + S3[3 * i + 1];
-  if (l == i - T.naj) v = v + S3[3 * i + 2];
-  return v;
-}
-
 // dense symmetric S (row-major, leading dimension ld; zeroed beforehand),
 // for rocSOLVER
 __global__ void k_tl_expand(TwoLevel T, const double *__restrict__ S3, double *__restrict__ G) {
@@ -168,88 +156,6 @@ __global__ void k_tl_expand(TwoLevel T, const double *__restrict__ S3, double *_
   }
 }
 
-// S = L L^T for S banded with bandwidth b = naj <= 63, in one workgroup.
-// Right-looking: step j takes the pivot, scales column j (rows j+1 .. j+b)
-// and subtracts its outer product from the trailing (b+1) x (b+1) window,
-// which lives in LDS with rows and columns taken modulo 64; the row j+b+1
-// enters the window from S as row j leaves it.  Lc[j (b+1) + t] = L(j+t, j)
-// (by columns), Lr[i (b+1) + t] = L(i, i-t) (by rows), Lc[j (b+1)] holding
-// the reciprocal pivot 1 / L(j, j) for the substitutions.  (A variant with
-// one barrier per column, forming column j+1 during step j's update, was
-// slower: the step is bound by the window's LDS traffic, not the barriers.)
-// info[0] = 1 + the first column whose pivot is not positive, 0 if none.
-constexpr int TL_CHOL_THREADS = 512;
-__global__ void __launch_bounds__(TL_CHOL_THREADS) k_tl_band_chol(TwoLevel T,
-                                                                  const double *__restrict__ S3,
-                                                                  double *__restrict__ Lc,
-                                                                  double *__restrict__ Lr,
-                                                                  int *info) {
-  __shared__ double W[64][65];
-  __shared__ double col[64];
-  __shared__ int bad;
-  const int n = T.nc, b = T.naj, B1 = b + 1;
-  for (int e = threadIdx.x; e < 64 * 64; e += blockDim.x) W[e >> 6][e & 63] = 0.0;
-  if (threadIdx.x == 0) bad = 0;
-  __syncthreads();
-  for (int e = threadIdx.x; e < B1 * B1; e += blockDim.x) {
-    const int i = e / B1, l = e - i * B1;
-    if (i < n && l <= i) W[i & 63][l & 63] = s_entry(T, S3, i, l);
-  }
-  // this thread's (t1, t2) pairs of the update, 1 <= t2 <= t1 <= b
-  constexpr int MAXP = (63 * 64 / 2 + TL_CHOL_THREADS - 1) / TL_CHOL_THREADS;
-  int pt1[MAXP], pt2[MAXP];
-  const int npairs = b * B1 / 2;
-#pragma unroll
-  for (int q = 0; q < MAXP; q++) {
-    const int p = (int)threadIdx.x + q * TL_CHOL_THREADS;
-    int t1 = 0, t2 = 0;
-    if (p < npairs) {
-      t1 = (int)((1.0 + sqrt(1.0 + 8.0 * (double)p)) * 0.5);
-      while (t1 * (t1 - 1) / 2 > p) t1--;
-      while ((t1 + 1) * t1 / 2 <= p) t1++;
-      t2 = p - t1 * (t1 - 1) / 2 + 1;
-    }
-    pt1[q] = t1;
-    pt2[q] = t2;
-  }
-  __syncthreads();
-  for (int j = 0; j < n; j++) {
-    if (threadIdx.x == 0) {
-      double w = W[j & 63][j & 63];
-      if (!(w > 0.0)) {
-        if (!bad) bad = j + 1;
-        w = 1.0;
-      }
-      const double d = sqrt(w);
-      col[0] = d;
-      Lc[(size_t)j * B1] = 1.0 / d;
-    }
-    __syncthreads();
-    const int t = (int)threadIdx.x + 1;
-    if (t <= b) {
-      const double v = j + t < n ? W[(j + t) & 63][j & 63] / col[0] : 0.0;
-      col[t] = v;
-      if (j + t < n) {
-        Lc[(size_t)j * B1 + t] = v;
-        Lr[(size_t)(j + t) * B1 + t] = v;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < MAXP; q++) {
-      const int t1 = pt1[q], t2 = pt2[q];
-      if (t1 > 0 && j + t1 < n) W[(j + t1) & 63][(j + t2) & 63] -= col[t1] * col[t2];
-    }
-    const int inew = j + B1;
-    if (inew < n && (int)threadIdx.x < B1) {
-      const int l = j + 1 + (int)threadIdx.x;
-      W[inew & 63][l & 63] = s_entry(T, S3, inew, l);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) info[0] = bad;
-}
-
 // lane `lane`'s value in every lane (two 32-bit readlanes; lane is uniform)
 __device__ inline double readlane64(double v, int lane) {
   const unsigned long long u = __double_as_longlong(v);
@@ -258,119 +164,260 @@ __device__ inline double readlane64(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Row j of X = S^-1 (= column j, S symmetric) by banded substitution of e_j,
-// both passes in axpy form with the band spread over the lanes: row r lives
-// in lane r mod 64, so a step reads its pivot row with one readlane and no
-// value moves between lanes.
-//   forward  L y = e_j from row j on: step m takes y_m from lane m mod 64,
-//            lanes of rows m+1 .. m+b subtract L(row, m) y_m (column m of L
-//            from Lc), and lane m mod 64 then holds row m + 64 (zero);
-//   backward L^T x = y from the last row: step i takes x_i, lanes of rows
-//            i-b .. i-1 subtract L(i, row) x_i (row i of L from Lr), and the
-//            row i-1-b enters (its lane holds a finished row, or row i when
-//            b = 63) with y_{i-1-b} from the forward pass.
-// One wavefront per j, four per block; y is kept in X's row j between the
-// passes.  The steps run in chunks of TL_CH whose band values are loaded
-// together, one chunk ahead (the loads are L2 hits whose latency is many
-// steps long).
-constexpr int TL_CH = 8;
-__global__ void __launch_bounds__(256) k_tl_band_inv(TwoLevel T, const double *__restrict__ Lc,
-                                                    const double *__restrict__ Lr,
-                                                    double *__restrict__ X) {
-  const int ln = threadIdx.x & 63;
-  const int j = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-  if (j >= T.nc) return;
-  const int n = T.nc, b = T.naj, B1 = b + 1;
-  double *xr = X + (size_t)j * T.ld;
-  auto lcol = [&](int m) {
-    const int t = (ln - m) & 63;
-    return (m < n && t >= 1 && t <= b && m + t < n) ? Lc[(size_t)m * B1 + t] : 0.0;
+// ---------------------------------------------------------------------------
+// Inverse of S for aggregate grids at most 63 wide.  With the aggregate rows
+// as blocks of b = naj unknowns S is block tridiagonal: D_i (tridiagonal) on
+// the diagonal and the diagonal matrix E_i between rows i - 1 and i.  With
+// the Schur complements from the top and from the bottom
+//   F_i = D_i - E_i F_{i-1}^-1 E_i,   G_i = D_i - E_{i+1} G_{i+1}^-1 E_{i+1}
+// the blocks of X = S^-1 are
+//   X_ii = (F_i + G_i - D_i)^-1,
+//   X_ij = -G_i^-1 E_i X_{i-1,j} (i > j),  X_ij = -F_i^-1 E_{i+1} X_{i+1,j} (i < j).
+// Only the two chains of b x b inverses are sequential, one workgroup each
+// (k_tl_chain); the diagonal blocks invert in parallel (k_tl_diag), and every
+// 16 columns of X follow from theirs by nai products with b x b matrices on
+// the FP64 matrix cores (k_tl_prop).  S is definite and diagonally dominant
+// by construction, so no pivoting is needed.  The banded Cholesky
+// factorisation and substitutions that this replaces (one workgroup, then one
+// wavefront per column of X, each nai b steps long) took 3.45 + 2.35 ms at
+// 63 x 63 aggregates and 0.77 + 0.42 ms at 28 x 37; the four kernels here take
+// 1.65 and 0.53 ms.
+// ---------------------------------------------------------------------------
+
+constexpr int TL_B = 64;   // padded block
+
+// S3 with every unknown scaled by a power of two sc (exact) that brings its
+// diagonal into [1, 4): S3s[3 I ..] as S3, X = sc X_scaled sc.  A diagonal that
+// is not positive keeps its value (and is found as a pivot).
+__global__ void k_tl_scale(TwoLevel T, const double *__restrict__ S3, double *__restrict__ S3s,
+                           double *__restrict__ sc) {
+  auto scale = [&](int I) {
+    const double d = S3[3 * I];
+    return d > 0.0 && d <= 1.7976931348623157e308 ? ldexp(1.0, -(ilogb(d) >> 1)) : 1.0;
   };
-  auto rpiv = [&](int m) { return (m >= 0 && m < n) ? Lc[(size_t)m * B1] : 1.0; };
-  double w = ln == (j & 63) ? 1.0 : 0.0;
-  double lv[TL_CH], rd[TL_CH], lvn[TL_CH], rdn[TL_CH];
-#pragma unroll
-  for (int u = 0; u < TL_CH; u++) {
-    lv[u] = lcol(j + u);
-    rd[u] = rpiv(j + u);
+  for (int I = blockIdx.x * blockDim.x + threadIdx.x; I < T.nc; I += gridDim.x * blockDim.x) {
+    const double s = scale(I);
+    sc[I] = s;
+    S3s[3 * I] = S3[3 * I] * s * s;
+    S3s[3 * I + 1] = I > 0 ? S3[3 * I + 1] * s * scale(I - 1) : 0.0;
+    S3s[3 * I + 2] = I >= T.naj ? S3[3 * I + 2] * s * scale(I - T.naj) : 0.0;
   }
-  for (int m0 = j; m0 < n; m0 += TL_CH) {
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      lvn[u] = lcol(m0 + TL_CH + u);
-      rdn[u] = rpiv(m0 + TL_CH + u);
-    }
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      const int m = m0 + u;
-      if (m < n) {
-        const double ym = readlane64(w, m & 63) * rd[u];
-        if (ln == 0) xr[m] = ym;
-        w = w - lv[u] * ym;
-        if (ln == (m & 63)) w = 0.0;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      lv[u] = lvn[u];
-      rd[u] = rdn[u];
-    }
-  }
-  // the backward pass reads, in every lane, the y that lane 0 stored
-  __threadfence_block();
-  auto lrow = [&](int i) {
-    const int t = (i - ln) & 63;
-    return (i >= 0 && t >= 1 && t <= b && i - t >= 0) ? Lr[(size_t)i * B1 + t] : 0.0;
-  };
-  auto yraw = [&](int m) { return (m >= j && m >= 0) ? xr[m] : 0.0; };
-  {
-    const int t = (n - 1 - ln) & 63;
-    w = t <= b ? yraw(n - 1 - t) : 0.0;
-  }
-  double yi[TL_CH], yin[TL_CH];
-#pragma unroll
-  for (int u = 0; u < TL_CH; u++) {
-    lv[u] = lrow(n - 1 - u);
-    rd[u] = rpiv(n - 1 - u);
-    yi[u] = yraw(n - 2 - b - u);
-  }
-  for (int i0 = n - 1; i0 >= 0; i0 -= TL_CH) {
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      lvn[u] = lrow(i0 - TL_CH - u);
-      rdn[u] = rpiv(i0 - TL_CH - u);
-      yin[u] = yraw(i0 - TL_CH - 1 - b - u);
-    }
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      const int i = i0 - u;
-      if (i >= 0) {
-        const double xi = readlane64(w, i & 63) * rd[u];
-        if (ln == 0) xr[i] = xi;
-        w = w - lv[u] * xi;
-        if (ln == ((i - 1 - b) & 63)) w = yi[u];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < TL_CH; u++) {
-      lv[u] = lvn[u];
-      rd[u] = rdn[u];
-      yi[u] = yin[u];
-    }
-  }
-  for (int c = n + ln; c < T.ld; c += 64) xr[c] = 0.0;
 }
 
-// Ainv = -X row by row (zero beyond nc), FP64 and / or FP32
-__global__ void k_tl_finish_rows(TwoLevel T, const double *__restrict__ X,
-                                 double *__restrict__ A64, float *__restrict__ A32) {
-  const size_t n = (size_t)T.nc * T.ld;
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(e % T.ld);
-    const double v = c < T.nc ? -X[e] : 0.0;
-    if (A64) A64[e] = v;
-    if (A32) A32[e] = (float)v;
+// In-place Gauss-Jordan inverse of a b x b symmetric positive definite block
+// with diagonal below 4, held by four waves, row 16 wave + q in a[q], column =
+// lane (identity beyond b).  Pivot k needs row k (published in rowbuf by its
+// owner; two rows in turn, so one barrier a pivot) and column k, which by
+// symmetry is row k again: a(i, k) = a(k, i) for rows still to come and -a(k,
+// i) for rows done.  With r(j) = a(k, j) / p, a(i, j) -= a(i, k) r(j); column k
+// becomes -a(i, k) / p by the same operation with r(k) = 1 + 1 / p (1 / p is
+// at least 1/4, so the sum loses no digits that matter).  The row of the next
+// pivot is updated and published first, so its way through LDS overlaps the
+// other rows' update.   Returns 1 + the first pivot that is not
+// positive (0: none); such a pivot is taken as 1.
+__device__ inline int tl_invert(double (&a)[16], int b, double (*rowbuf)[TL_B]) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int first = 0;
+  __syncthreads();
+  if (wv == 0) rowbuf[0][lane] = a[0];
+  __syncthreads();
+  // one pivot: kk (its row in the owning wave) is a compile-time constant
+  auto pivot = [&](auto KK, int kw) {
+    constexpr int kk = decltype(KK)::value, nq = (kk + 1) & 15;
+    const int k = 16 * kw + kk;
+    const double x = rowbuf[k & 1][lane];
+    double p = readlane64(x, k);
+    if (!(p > 0.0)) {
+      if (first == 0) first = k + 1;
+      p = 1.0;
+    }
+    // 1 / p: the hardware's estimate and two Newton steps
+    double ip = __builtin_amdgcn_rcp(p);
+    ip = fma(fma(-p, ip, 1.0), ip, ip);
+    ip = fma(fma(-p, ip, 1.0), ip, ip);
+    const double r = lane == k ? 1.0 + ip : x * ip;
+    const double rs = wv < kw ? r : -r;   // rows done take the other sign
+    const bool own = wv == kw, nown = wv == (kk < 15 ? kw : kw + 1);
+    auto upd = [&](int q) {
+      const double f = readlane64(x, 16 * wv + q);
+      a[q] = fma(f, own && q < kk ? r : rs, a[q]);
+    };
+    upd(nq);
+    if (nown) rowbuf[(k + 1) & 1][lane] = a[nq];
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+      if (q != nq && q != kk) upd(q);
+    if (own) a[kk] = lane == k ? ip : r;
+    else upd(kk);
+    __syncthreads();
+  };
+  for (int kw = 0; 16 * kw < b; kw++) {
+    const int left = b - 16 * kw;
+#define MF6_PIV(K) if (K < left) pivot(std::integral_constant<int, K>{}, kw);
+    MF6_PIV(0) MF6_PIV(1) MF6_PIV(2) MF6_PIV(3) MF6_PIV(4) MF6_PIV(5) MF6_PIV(6) MF6_PIV(7)
+    MF6_PIV(8) MF6_PIV(9) MF6_PIV(10) MF6_PIV(11) MF6_PIV(12) MF6_PIV(13) MF6_PIV(14) MF6_PIV(15)
+#undef MF6_PIV
+  }
+  return first;
+}
+
+// entry (r, c) of the padded diagonal block of aggregate row i
+__device__ inline double tl_dentry(const double *__restrict__ S3, int b, int i, int r, int c) {
+  if (r >= b || c >= b) return r == c ? 1.0 : 0.0;
+  if (r == c) return S3[3 * (i * b + r)];
+  if (r == c + 1) return S3[3 * (i * b + r) + 1];
+  if (c == r + 1) return S3[3 * (i * b + c) + 1];
+  return 0.0;
+}
+
+// coupling of aggregate (i, r) to (i - 1, r)
+__device__ inline double tl_eentry(const double *__restrict__ S3, int b, int nai, int i, int r) {
+  return (r < b && i > 0 && i < nai) ? S3[3 * (i * b + r) + 2] : 0.0;
+}
+
+// The two chains: workgroup 0 F_i^-1 for i = 0 .. nai - 1 into Fi, workgroup 1
+// G_i^-1 for i = nai - 1 .. 0 into Gi (blocks of b x b, rows b apart).  Bound
+// by the pivots' dependent latency (nai b of them).  info[0] = 1 + the first
+// unknown whose pivot is not positive (in the order of the unknowns), else 0.
+__global__ void __launch_bounds__(256) k_tl_chain(TwoLevel T, const double *__restrict__ S3,
+                                                  double *__restrict__ Fi, double *__restrict__ Gi,
+                                                  int *info) {
+  __shared__ double rowbuf[2][TL_B];
+  const int lane = threadIdx.x & 63, r0 = 16 * (int)(threadIdx.x >> 6);
+  const int b = T.naj, n = T.nai, down = blockIdx.x == 0;
+  double *out = down ? Fi : Gi;
+  double a[16], dn[16], en[16], ec;
+  int first = 0;
+  // the next block's entries are loaded while this one is inverted
+  auto load = [&](int s) {
+    const int i = down ? s : n - 1 - s, e = down ? i : i + 1;
+    ec = tl_eentry(S3, b, n, e, lane);
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      dn[q] = tl_dentry(S3, b, i, r0 + q, lane);
+      en[q] = tl_eentry(S3, b, n, e, r0 + q);
+    }
+  };
+  load(0);
+#pragma unroll
+  for (int q = 0; q < 16; q++) a[q] = 0.0;
+  for (int s = 0; s < n; s++) {
+    const int i = down ? s : n - 1 - s;
+#pragma unroll
+    for (int q = 0; q < 16; q++) a[q] = fma(-en[q] * ec, a[q], dn[q]);
+    if (s + 1 < n) load(s + 1);
+    const int bd = tl_invert(a, b, rowbuf);
+    if (bd && !first) first = i * b + bd;
+    double *o = out + (size_t)i * b * b;
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+      if (r0 + q < b && lane < b) o[(r0 + q) * b + lane] = a[q];
+  }
+  if (down && threadIdx.x == 0) info[0] = first;
+}
+
+// X_ii = (D_i - E_i F_{i-1}^-1 E_i - E_{i+1} G_{i+1}^-1 E_{i+1})^-1, one workgroup per i
+__global__ void __launch_bounds__(256) k_tl_diag(TwoLevel T, const double *__restrict__ S3,
+                                                 const double *__restrict__ Fi,
+                                                 const double *__restrict__ Gi,
+                                                 double *__restrict__ Xd) {
+  __shared__ double rowbuf[2][TL_B];
+  const int lane = threadIdx.x & 63, r0 = 16 * (int)(threadIdx.x >> 6);
+  const int b = T.naj, n = T.nai, i = blockIdx.x;
+  const double ecu = tl_eentry(S3, b, n, i, lane), ecd = tl_eentry(S3, b, n, i + 1, lane);
+  double a[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int r = r0 + q;
+    const bool in = r < b && lane < b;
+    const double f = in && i > 0 ? Fi[(size_t)(i - 1) * b * b + r * b + lane] : 0.0;
+    const double g = in && i + 1 < n ? Gi[(size_t)(i + 1) * b * b + r * b + lane] : 0.0;
+    double v = tl_dentry(S3, b, i, r, lane);
+    v = fma(-tl_eentry(S3, b, n, i, r) * ecu, f, v);
+    a[q] = fma(-tl_eentry(S3, b, n, i + 1, r) * ecd, g, v);
+  }
+  (void)tl_invert(a, b, rowbuf);
+#pragma unroll
+  for (int q = 0; q < 16; q++)
+    if (r0 + q < b && lane < b) Xd[(size_t)i * b * b + (r0 + q) * b + lane] = a[q];
+}
+
+// 16 columns of X below (blockIdx.z = 0, with the diagonal block) or above
+// the diagonal block of aggregate row j = blockIdx.x, written as Ainv = -X in
+// FP64 or FP32.  Per row block one 64 x 64 by 64 x 16 product on
+// v_mfma_f64_16x16x4_f64: wave w takes rows 16 w .., operand A (lane: row
+// l % 16, k = l / 16) from the symmetric inverse read by columns, operand B
+// (k = l / 16, column l % 16) from LDS, result rows 4 e + l / 16.  The next
+// inverse is loaded while the product runs.
+typedef double d4 __attribute__((ext_vector_type(4)));
+template <typename TA>
+__global__ void __launch_bounds__(256) k_tl_prop(TwoLevel T, const double *__restrict__ S3,
+                                                 const double *__restrict__ Fi,
+                                                 const double *__restrict__ Gi,
+                                                 const double *__restrict__ Xd,
+                                                 const double *__restrict__ sc,
+                                                 TA *__restrict__ Ainv) {
+  __shared__ double V[2][TL_B][16];
+  const int b = T.naj, n = T.nai, j = blockIdx.x, c0 = 16 * (int)blockIdx.y;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = lane & 15, kq = lane >> 4, row = 16 * wv + col;
+  const bool low = blockIdx.z == 0, colok = c0 + col < b;
+  const int step = low ? 1 : -1;
+  TA *oc = Ainv + (size_t)j * b + c0 + col;   // this lane's column
+  // columns past the last unknown are zero
+  if (low && blockIdx.y == 0)
+    for (int e = threadIdx.x; e < b * (T.ld - T.nc); e += 256) {
+      const int r = e / (T.ld - T.nc);
+      Ainv[(size_t)(j * b + r) * T.ld + T.nc + (e - r * (T.ld - T.nc))] = (TA)0;
+    }
+  const double *inv = low ? Gi : Fi;
+  double an[16], es[4], so[4];
+  const double sj = colok ? sc[j * b + c0 + col] : 0.0;
+  auto load = [&](int i) {                     // the inverse of block i
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+      const int k = 4 * t + kq;
+      an[t] = (i >= 0 && i < n && k < b && row < b) ? inv[(size_t)i * b * b + k * b + row] : 0.0;
+    }
+  };
+  // rows 16 wv + 4 e + kq of block i: the couplings that multiply them on the
+  // way to the next block, and the scales of their results
+  auto scale = [&](int i) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = 16 * wv + 4 * e + kq;
+      es[e] = tl_eentry(S3, b, n, low ? i + 1 : i, r);
+      so[e] = r < b ? sj * sc[i * b + r] : 0.0;
+    }
+  };
+  load(j + step);
+  scale(j);
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int r = 16 * wv + 4 * e + kq;
+    const double x = (r < b && colok) ? Xd[(size_t)j * b * b + r * b + c0 + col] : 0.0;
+    V[0][r][col] = es[e] * x;
+    if (low && r < b && colok) oc[(size_t)(j * b + r) * T.ld] = (TA)(-x * so[e]);
+  }
+  __syncthreads();
+  int p = 0;
+  for (int i = j + step; i >= 0 && i < n; i += step, p ^= 1) {
+    double a[16];
+#pragma unroll
+    for (int t = 0; t < 16; t++) a[t] = an[t];
+    load(i + step);
+    scale(i);
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < 16; t++)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], V[p][4 * t + kq][col], acc, 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int r = 16 * wv + 4 * e + kq;
+      V[p ^ 1][r][col] = -es[e] * acc[e];
+      if (r < b && colok) oc[(size_t)(i * b + r) * T.ld] = (TA)(acc[e] * so[e]);   // -X
+    }
+    __syncthreads();
   }
 }
 
@@ -723,16 +770,19 @@ static int tl_alloc_all(Mf6Handle *h) {
   const Layout &L = h->L;
   h->tl = mf6hip_tl_shape(L, h->s.coarse_size);
   const size_t nn = (size_t)h->tl.nc * h->tl.ld;
+  // b x b blocks for the block inverse; the dense matrix for rocSOLVER
+  const size_t nb = (size_t)h->tl.nc * h->tl.naj;
+  const bool wide = h->tl.naj > 63;
   if (hipMalloc((void **)&h->tl_cmask, sizeof(unsigned) * 2 * (size_t)L.HP) != hipSuccess ||
-      hipMalloc((void **)&h->tl_G, sizeof(double) * nn) != hipSuccess ||
+      hipMalloc((void **)&h->tl_G, sizeof(double) * (wide ? nn : nb)) != hipSuccess ||
       hipMalloc((void **)&h->tl_rc, sizeof(double) * h->tl.ld) != hipSuccess ||
       hipMalloc((void **)&h->tl_yc64, sizeof(double) * h->tl.ld) != hipSuccess ||
       hipMalloc((void **)&h->tl_yc32, sizeof(float) * h->tl.ld) != hipSuccess ||
       hipMalloc((void **)&h->tl_info, sizeof(int)) != hipSuccess ||
       hipMalloc((void **)&h->tl_colsum, sizeof(double) * (size_t)L.NRC) != hipSuccess ||
-      hipMalloc((void **)&h->tl_S3, sizeof(double) * 3 * (size_t)h->tl.nc) != hipSuccess ||
-      hipMalloc((void **)&h->tl_Lc, sizeof(double) * 64 * (size_t)h->tl.nc) != hipSuccess ||
-      hipMalloc((void **)&h->tl_Lr, sizeof(double) * 64 * (size_t)h->tl.nc) != hipSuccess) {
+      hipMalloc((void **)&h->tl_S3, sizeof(double) * 7 * (size_t)h->tl.nc) != hipSuccess ||
+      (!wide && hipMalloc((void **)&h->tl_Fi, sizeof(double) * nb) != hipSuccess) ||
+      (!wide && hipMalloc((void **)&h->tl_Gi, sizeof(double) * nb) != hipSuccess)) {
     mf6hip_set_error("hipMalloc failed (two-level preconditioner)");
     return MF6HIP_EHIP;
   }
@@ -779,7 +829,7 @@ void mf6hip_tl_free(Mf6Handle *h) {
   if (h->tl_blas) rocblas_destroy_handle((rocblas_handle)h->tl_blas);
   h->tl_blas = nullptr;
   void *bufs[] = {h->tl_cmask, h->tl_G, h->tl_rc, h->tl_yc64, h->tl_yc32, h->tl_info,
-                  h->tl_A64, h->tl_A32, h->tl_colsum, h->tl_S3, h->tl_Lc, h->tl_Lr,
+                  h->tl_A64, h->tl_A32, h->tl_colsum, h->tl_S3, h->tl_Fi, h->tl_Gi,
                   h->tl_s32, h->tl_ew, h->tl_ns, h->tl_colsq};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -788,9 +838,25 @@ void mf6hip_tl_free(Mf6Handle *h) {
   h->tl_A32 = h->tl_yc32 = nullptr;
   h->tl_info = nullptr;
   h->tl_colsum = nullptr;
-  h->tl_S3 = h->tl_Lc = h->tl_Lr = nullptr;
+  h->tl_S3 = h->tl_Fi = h->tl_Gi = nullptr;
   h->tl_s32 = h->tl_ew = h->tl_ns = nullptr;
   h->tl_colsq = nullptr;
+}
+
+// Ainv = -S^-1 of the compact rows S3 (aggregate grid at most 63 wide), FP64
+// or FP32; Fi, Gi and Xd hold nc naj doubles each, S3 7 nc (the rows, then
+// their scaled copy and the scales).
+static int tl_block_inverse(const TwoLevel &T, double *S3, double *Fi, double *Gi,
+                            double *Xd, double *A64, float *A32, int *dinfo, hipStream_t s) {
+  const dim3 grid(T.nai, (T.naj + 15) / 16, 2);
+  double *S = S3 + 3 * (size_t)T.nc, *sc = S3 + 6 * (size_t)T.nc;   // scaled rows, scales
+  k_tl_scale<<<tl_grid(T.nc), MF6_BLOCK, 0, s>>>(T, S3, S, sc);
+  k_tl_chain<<<2, 256, 0, s>>>(T, S, Fi, Gi, dinfo);
+  k_tl_diag<<<T.nai, 256, 0, s>>>(T, S, Fi, Gi, Xd);
+  if (A64) k_tl_prop<double><<<grid, 256, 0, s>>>(T, S, Fi, Gi, Xd, sc, A64);
+  if (A32) k_tl_prop<float><<<grid, 256, 0, s>>>(T, S, Fi, Gi, Xd, sc, A32);
+  HIPCHK(hipGetLastError());
+  return MF6HIP_OK;
 }
 
 // Coarse operator of the current FP64 planes: mask, S = -Ac, its inverse.
@@ -807,16 +873,10 @@ int mf6hip_tl_setup(Mf6Handle *h) {
   HIPCHK(hipGetLastError());
   int info = 0;
   if (T.naj <= 63) {
-    k_tl_band_chol<<<1, TL_CHOL_THREADS, 0, s>>>(T, h->tl_S3, h->tl_Lc, h->tl_Lr, h->tl_info);
-    HIPCHK(hipGetLastError());
+    CK(tl_block_inverse(T, h->tl_S3, h->tl_Fi, h->tl_Gi, h->tl_G, h->tl_A64, h->tl_A32,
+                        h->tl_info, s));
     HIPCHK(hipMemcpyAsync(&info, h->tl_info, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    if (info == 0) {
-      k_tl_band_inv<<<(T.nc + 3) / 4, 256, 0, s>>>(T, h->tl_Lc, h->tl_Lr, h->tl_G);
-      k_tl_finish_rows<<<tl_grid((size_t)T.nc * T.ld), MF6_BLOCK, 0, s>>>(T, h->tl_G, h->tl_A64,
-                                                                         h->tl_A32);
-      HIPCHK(hipGetLastError());
-    }
   } else {
     HIPCHK(hipMemsetAsync(h->tl_G, 0, sizeof(double) * (size_t)T.nc * T.ld, s));
     k_tl_expand<<<tl_grid(T.nc), MF6_BLOCK, 0, s>>>(T, h->tl_S3, h->tl_G);
@@ -848,13 +908,13 @@ int mf6hip_tl_setup(Mf6Handle *h) {
   return MF6HIP_OK;
 }
 
-// The banded coarse setup of one system whose FP64 planes are A (layout
-// L), into caller-owned arrays: cmask (2 HP), S3 (3 nc), Lc / Lr (64 nc),
-// scratch G (nc ld doubles) and the FP32 inverse A32 (nc ld).  For the
-// ensemble solver; aggregate grids wider than 63 are not supported there.
-// Returns the factorisation's info code through *info (0: definite).
+// The coarse setup of one system whose FP64 planes are A (layout L), into
+// caller-owned arrays: cmask (2 HP), S3 (7 nc), Fi / Gi / Xd (nc naj each)
+// and the FP32 inverse A32 (nc ld).  For the ensemble solver; aggregate grids
+// wider than 63 are not supported there.  Returns the info code of the
+// factorisation through *info (0: definite).
 int mf6hip_tl_setup_slice(const Layout &L, const double *A, const TwoLevel &T,
-                          unsigned *cmask, double *S3, double *Lc, double *Lr, double *G,
+                          unsigned *cmask, double *S3, double *Fi, double *Gi, double *Xd,
                           float *A32, int *dinfo, int *info, hipStream_t s) {
   if (T.naj > 63) {
     mf6hip_set_error("ensemble two-level: aggregate grid wider than 63");
@@ -862,14 +922,9 @@ int mf6hip_tl_setup_slice(const Layout &L, const double *A, const TwoLevel &T,
   }
   k_tl_cmask<<<tl_grid(2 * (size_t)L.HP), MF6_BLOCK, 0, s>>>(L, A, cmask);
   k_tl_build<<<T.nc, MF6_BLOCK, 0, s>>>(L, A, cmask, T, S3);
-  k_tl_band_chol<<<1, TL_CHOL_THREADS, 0, s>>>(T, S3, Lc, Lr, dinfo);
-  HIPCHK(hipGetLastError());
+  CK(tl_block_inverse(T, S3, Fi, Gi, Xd, nullptr, A32, dinfo, s));
   HIPCHK(hipMemcpyAsync(info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  if (*info != 0) return MF6HIP_OK;
-  k_tl_band_inv<<<(T.nc + 3) / 4, 256, 0, s>>>(T, Lc, Lr, G);
-  k_tl_finish_rows<<<tl_grid((size_t)T.nc * T.ld), MF6_BLOCK, 0, s>>>(T, G, nullptr, A32);
-  HIPCHK(hipGetLastError());
   return MF6HIP_OK;
 }
 

@@ -174,9 +174,9 @@ struct Mf6Handle {
   float *tl_A32 = nullptr, *tl_yc32 = nullptr;
   int *tl_info = nullptr;
   double *tl_colsum = nullptr;   // per grid column: residual summed over coupled cells
-  double *tl_S3 = nullptr;       // compact rows of S = -Ac (diagonal, west, north)
-  double *tl_Lc = nullptr;       // banded Cholesky factor of S by columns, nc x (naj + 1)
-  double *tl_Lr = nullptr;       // the same factor by rows
+  double *tl_S3 = nullptr;       // compact rows of S = -Ac (diagonal, west, north), scaled copy, scales
+  double *tl_Fi = nullptr;       // inverses of S's block Schur complements from the top, nc naj
+  double *tl_Gi = nullptr;       // the same from the bottom
   // deflated form (preconditioner = 3): per-cell row sums over the coupled
   // cells, couplings across aggregate edges, per-column sums of q (colour
   // layout, c HP + h2)
@@ -203,7 +203,7 @@ struct Mf6Handle {
 // two-level preconditioner (mf6hip_coarse.hip)
 TwoLevel mf6hip_tl_shape(const Layout &L, int target);
 int mf6hip_tl_setup_slice(const Layout &L, const double *A, const TwoLevel &T,
-                          unsigned *cmask, double *S3, double *Lc, double *Lr, double *G,
+                          unsigned *cmask, double *S3, double *Fi, double *Gi, double *Xd,
                           float *A32, int *dinfo, int *info, hipStream_t s);
 int mf6hip_tl_setup(Mf6Handle *h);
 void mf6hip_tl_free(Mf6Handle *h);
