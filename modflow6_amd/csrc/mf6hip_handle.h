@@ -34,6 +34,12 @@ struct DevPackage {
   double *depth = nullptr; // DRN depths (idepth)
 };
 
+// the outcome of a folded solve, in pinned host memory
+struct FoldHost {
+  int stop;
+  KState st;
+};
+
 struct Mf6Handle {
   Layout L{};
   mf6hip_ims_settings s{};
@@ -159,10 +165,12 @@ struct Mf6Handle {
   double last_solve_ms = 0, last_spmv_ms = 0;
   int last_spmv_n = 0;
   bool timing = false;
-  // fused FP64 CG: eight iterations captured once per handle as a HIP graph
+  // folded or fused FP64 CG: eight iterations captured once per handle as a HIP graph
   // (used when the per-launch SpMV timing is off)
   hipGraphExec_t cg_graph = nullptr;
   bool cg_graph_failed = false;
+  hipEvent_t ev_batch[2] = {nullptr, nullptr};   // end of a batch of iterations
+  FoldHost *h_fold = nullptr;
   // two-level preconditioner (preconditioner = 2): coarse shape, per-column
   // coupled-cell masks, dense coarse matrix / Cholesky workspace G, the
   // inverse (FP64 for the FP64 solve, FP32 for the mixed ones), restricted
@@ -230,6 +238,9 @@ int mf6hip_device_solve(Mf6Handle *h, int kstp, int kiter, int *icnvg,
 int mf6hip_launch_row_fixes(Mf6Handle *h);
 int mf6hip_copy_system(Mf6Handle *h, double *amat_out, double *rhs_out);
 int mf6hip_run_cg_fused(Mf6Handle *h);
+// the same for small grids (mf6hip_cgfold.hip)
+bool mf6hip_fold_takes(const Mf6Handle *h);
+int mf6hip_run_cg_fold(Mf6Handle *h);
 int mf6hip_run_cg_reliable(Mf6Handle *h, int *icnvg, int *iters);
 int mf6hip_is_symmetric(Mf6Handle *h, int *sym);
 int mf6hip_dxmax(Mf6Handle *h, double *hncg, int *lrch, const double *xa,

@@ -1607,7 +1607,8 @@ int mf6hip_device_solve(Mf6Handle *h, int kstp, int kiter, int *icnvg, int *in_i
     CK(read_state(h));
     if (!h->h_state->stop) {
       if (h->s.preconditioner == 1) CK(mf6hip_run_fcg(h));
-      else if (h->s.ilinmeth == 1 && sym && h->s.kernel_variant == 0) CK(mf6hip_run_cg_fused(h));
+      else if (h->s.ilinmeth == 1 && sym && h->s.kernel_variant == 0)
+        CK(mf6hip_fold_takes(h) ? mf6hip_run_cg_fold(h) : mf6hip_run_cg_fused(h));
       else if (h->s.ilinmeth == 1) CK(run_cg(h));
       else CK(run_bcgs(h));
     }
@@ -1866,11 +1867,13 @@ extern "C" int mf6hip_create(int neq, int nja, const int *ia, const int *ja,
     if (!rc) rc = dalloc(&h->d_amat_csr, (size_t)nja);
   }
   if (!rc) {
-    if (hipHostMalloc((void **)&h->h_state, 4 * sizeof(KState), hipHostMallocDefault) != hipSuccess) rc = MF6HIP_EHIP;
+    if (hipHostMalloc((void **)&h->h_state, 4 * sizeof(KState), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&h->h_fold, sizeof(FoldHost), hipHostMallocDefault) != hipSuccess) rc = MF6HIP_EHIP;
   }
   if (!rc) {
     hipEventCreate(&h->ev0);
     hipEventCreate(&h->ev1);
+    for (auto &e : h->ev_batch) hipEventCreateWithFlags(&e, hipEventDisableTiming);
     h->spmv_ev.resize(2 * 256);
     for (auto &e : h->spmv_ev) hipEventCreate(&e);
   }
@@ -1933,8 +1936,11 @@ extern "C" int mf6hip_destroy(void *handle) {
       if (b) hipFree(b);
   }
   if (h->h_state) hipHostFree(h->h_state);
+  if (h->h_fold) hipHostFree(h->h_fold);
   if (h->ev0) hipEventDestroy(h->ev0);
   if (h->ev1) hipEventDestroy(h->ev1);
+  for (auto &e : h->ev_batch)
+    if (e) hipEventDestroy(e);
   for (auto &e : h->spmv_ev) hipEventDestroy(e);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;

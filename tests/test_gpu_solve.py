@@ -141,6 +141,41 @@ def test_fused_cg_matches_unfused(shape):
         assert abs(res[0][3].rmax[t] - res[1][3].rmax[t]) <= 1e-9 * abs(res[1][3].rmax[t])
 
 
+# every compile-time bound of the layers (4, 8, 12, 16, 32) with a partial
+# last chunk, blocks of 64 and (the last two shapes) of 256 threads, odd and
+# even rows, a single row
+@pytest.mark.parametrize("shape", [(1, 1, 64), (1, 9, 8), (3, 64, 64), (5, 33, 17), (9, 20, 31),
+                                   (13, 24, 24), (20, 14, 15), (32, 10, 11), (10, 150, 121),
+                                   (17, 101, 90)])
+def test_folded_cg_matches_unfused(shape):
+    nlay, nrow, ncol = shape
+    case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=4)
+    sim, amat, rhs, x0 = oracle_system(case)
+    out = []
+    for variant in (0, 1):
+        sv = device_solver(case, kernel_variant=variant)
+        x, rec = x0.copy(), ConvergenceRecord(case.ims.inner_maximum)
+        icn, it = sv.solve(1, amat, rhs, x, kstp=1, record=rec)
+        sv.destroy()
+        assert icn == 1
+        out.append((x, it, rec))
+    (xa, ia, ra), (xb, ib, rb) = out
+    assert np.max(np.abs(xa - xb)) < 10 * case.ims.inner_dvclose
+    assert_same_trajectory(ra, rb, min(20, ia, ib))
+
+
+def assert_same_trajectory(ra, rb, n):
+    """The same recurrences with the dot products summed in another order:
+    round-off (1e-16 at the first iteration, below 1e-13 at the twentieth on
+    these systems), which CG amplifies later on, so that the exit iteration
+    is not compared."""
+    for t in range(n):
+        for a, b in ((ra.dvmax, rb.dvmax), (ra.rmax, rb.rmax), (ra.alpha, rb.alpha),
+                     (ra.omega, rb.omega)):
+            assert abs(a[t] - b[t]) <= 1e-9 * abs(b[t]) + 1e-14 * np.max(np.abs(b[:n]))
+        assert ra.locdv[t] == rb.locdv[t] and ra.locr[t] == rb.locr[t]
+
+
 def test_fused_cg_graph_replay_matches_eager_launches():
     """Without the per-launch timing the fused FP64 CG replays captured
     eight-iteration graphs; with it, it launches every kernel.  The same
