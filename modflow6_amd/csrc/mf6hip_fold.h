@@ -1,5 +1,5 @@
 // mf6hip_fold.h -- pieces shared by the latency-bound Krylov kernels
-// (mf6hip_cgfold.hip): wave and block reductions, the sum
+// (mf6hip_cgfold.hip, mf6hip_bcgsfold.hip): wave and block reductions, the sum
 // of partials that every block adds in the same order, column geometry.
 #pragma once
 #include "mf6hip_handle.h"

@@ -165,7 +165,7 @@ struct Mf6Handle {
   double last_solve_ms = 0, last_spmv_ms = 0;
   int last_spmv_n = 0;
   bool timing = false;
-  // folded or fused FP64 CG: eight iterations captured once per handle as a HIP graph
+  // folded or fused FP64 CG and folded BiCGSTAB: a few iterations captured once per handle as a HIP graph
   // (used when the per-launch SpMV timing is off)
   hipGraphExec_t cg_graph = nullptr;
   bool cg_graph_failed = false;
@@ -241,6 +241,10 @@ int mf6hip_run_cg_fused(Mf6Handle *h);
 // the same for small grids (mf6hip_cgfold.hip)
 bool mf6hip_fold_takes(const Mf6Handle *h);
 int mf6hip_run_cg_fold(Mf6Handle *h);
+// BiCGSTAB in folded kernels (mf6hip_bcgsfold.hip): FP64, and the mixed inner solve
+bool mf6hip_bcgs_fold_takes(const Mf6Handle *h);
+int mf6hip_run_bcgs_fold(Mf6Handle *h);
+int mf6hip_run_bcgs_fold_inner(Mf6Handle *h);
 int mf6hip_run_cg_reliable(Mf6Handle *h, int *icnvg, int *iters);
 int mf6hip_is_symmetric(Mf6Handle *h, int *sym);
 int mf6hip_dxmax(Mf6Handle *h, double *hncg, int *lrch, const double *xa,

@@ -1219,7 +1219,7 @@ static int run_bcgs(Mf6Handle *h) {
 
 // inner-solve state lives in a second KState
 __global__ void k_s_inner_init(KState *st, const double *part, const MaxLoc *mpart, int nb,
-                               double rtol, double rfloor) {
+                               double rtol, double rfloor, int itmax) {
   __shared__ MaxLoc mlds[8];
   MaxLoc m = reduce_mparts(mpart, nb, mlds);
   if (threadIdx.x == 0) {
@@ -1227,6 +1227,7 @@ __global__ void k_s_inner_init(KState *st, const double *part, const MaxLoc *mpa
     st->stop = 0;
     st->icnvg = 0;
     st->rho0 = 0.0;
+    st->itmax = itmax;
     st->inner_r0 = fabs(m.v);
     st->rclose = fmax(rtol * fabs(m.v), rfloor);
     st->dvclose = 0.0;
@@ -1292,7 +1293,7 @@ static int run_mixed_cg(Mf6Handle *h, const TP *piv32) {
     if (hm.v == 0.0) { icnvg = 1; break; }
     k_convert<double, float><<<g, MF6_BLOCK, 0, s>>>(L.NP, h->d, h->r32);
     k_s_inner_init<<<1, MF6_BLOCK, 0, s>>>(ist, h->d_part, h->d_mpart, nb, rtol,
-                                           0.5 * h->s.rclose);
+                                           0.5 * h->s.rclose, inner_max);
     float *pin = h->p32, *pout = h->p232;
     int batch = 4, done = 0;
     while (done < inner_max && total + done < h->s.iter1) {
@@ -1392,11 +1393,15 @@ static int run_mixed_bcgs(Mf6Handle *h, const TP *piv32) {
     if (fabs(hm.v) <= h->s.rclose && fabs(last_dv) <= h->s.dvclose) { icnvg = 1; break; }
     if (hm.v == 0.0) { icnvg = 1; break; }
     k_convert<double, float><<<g, MF6_BLOCK, 0, s>>>(L.NP, h->d, r);
-    HIPCHK(hipMemcpyAsync(dhat, r, sizeof(float) * L.NP, hipMemcpyDeviceToDevice, s));
+    const int left = h->s.iter1 - total;
     k_s_inner_init<<<1, MF6_BLOCK, 0, s>>>(ist, h->d_part, h->d_mpart, nb, rtol,
-                                           0.5 * h->s.rclose);
+                                           0.5 * h->s.rclose,
+                                           inner_max < left ? inner_max : left);
     int batch = 4, done = 0;
-    while (done < inner_max && total + done < h->s.iter1) {
+    const bool fold = mf6hip_bcgs_fold_takes(h);
+    if (fold) CK(mf6hip_run_bcgs_fold_inner(h));
+    else HIPCHK(hipMemcpyAsync(dhat, r, sizeof(float) * L.NP, hipMemcpyDeviceToDevice, s));
+    while (!fold && done < inner_max && total + done < h->s.iter1) {
       for (int it = 0; it < batch; it++) {
         k_dot<float><<<nb, MF6_BLOCK, 0, s>>>(L.NP, dhat, r, h->d_part, ist);
         k_s_bcgs_rho<<<1, MF6_BLOCK, 0, s>>>(ist, h->d_part, nb);
@@ -1610,7 +1615,7 @@ int mf6hip_device_solve(Mf6Handle *h, int kstp, int kiter, int *icnvg, int *in_i
       else if (h->s.ilinmeth == 1 && sym && h->s.kernel_variant == 0)
         CK(mf6hip_fold_takes(h) ? mf6hip_run_cg_fold(h) : mf6hip_run_cg_fused(h));
       else if (h->s.ilinmeth == 1) CK(run_cg(h));
-      else CK(run_bcgs(h));
+      else CK(mf6hip_bcgs_fold_takes(h) ? mf6hip_run_bcgs_fold(h) : run_bcgs(h));
     }
   }
   if (h->s.iscl != 0) CK(ims_scale(h, 1));

@@ -200,6 +200,38 @@ def test_fused_cg_graph_replay_matches_eager_launches():
     gs.destroy()
 
 
+# the folded BiCGSTAB against the one-pass kernels: layer bounds (4, 8, 16,
+# 32) with partial chunks, 64 and 256 threads, a column or a chunk of it per
+# thread, a single row; the squeeze of the partials (more than 2048 blocks:
+# the last)
+@pytest.mark.parametrize("shape", [(1, 1, 64), (2, 30, 32), (3, 33, 17), (5, 24, 21), (9, 20, 31),
+                                   (17, 14, 15), (32, 10, 11), (3, 130, 141), (4, 300, 240),
+                                   (6, 263, 261), (1, 730, 730)])
+def test_folded_bicgstab_matches_one_pass(shape):
+    nlay, nrow, ncol = shape
+    case = configs.transient_newton(seed=5, nlay=nlay, nrow=nrow, ncol=ncol, nwel=3, nper=1,
+                                    nstp=2, perlen=10.0)
+    sim, amat, rhs, x0 = oracle_system(case)
+    out = []
+    for variant in (0, 1):
+        sv = device_solver(case, kernel_variant=variant)
+        x, rec = x0.copy(), ConvergenceRecord(case.ims.inner_maximum)
+        icn, it = sv.solve(1, amat, rhs, x, kstp=1, record=rec)
+        sv.destroy()
+        assert icn == 1
+        out.append((x, it, rec))
+    (xa, ia, ra), (xb, ib, rb) = out
+    assert np.max(np.abs(xa - xb)) < 10 * case.ims.inner_dvclose
+    assert_same_trajectory(ra, rb, min(6, ia, ib))
+    for precision in (_lib.MF6HIP_MIXED, _lib.MF6HIP_MIXED_FP16):
+        sv = device_solver(case, precision=precision)
+        x = x0.copy()
+        icn, it = sv.solve(1, amat, rhs, x, kstp=1)
+        sv.destroy()
+        assert icn == 1
+        assert np.max(np.abs(x - xb)) < 10 * case.ims.inner_dvclose
+
+
 @pytest.mark.parametrize("precision", [_lib.MF6HIP_MIXED, _lib.MF6HIP_MIXED_FP16])
 def test_mixed_bicgstab_newton_system(precision):
     """Mixed-precision BiCGSTAB (FP32 ILU0 + SpMV BiCGSTAB inside FP64
