@@ -35,10 +35,7 @@
 #include <cstring>
 #include <string>
 
-#include "mf6hip_handle.h"
-
-#define DPREC_F 2.220446049250313080847263336181640625e-16
-#define DSAME_F (100.0 * DPREC_F)
+#include "mf6hip_fold.h"
 
 #define CK(x)                         \
   do {                                \
@@ -48,26 +45,8 @@
 
 namespace {
 
-template <typename T>
-__device__ inline T wsum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
-__device__ inline MaxLoc wmax(MaxLoc a) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    MaxLoc b;
-    b.v = __shfl_xor(a.v, o);
-    b.loc = __shfl_xor(a.loc, o);
-    a = maxloc_pick(a, b);
-  }
-  return a;
-}
-
 __device__ inline double bsum(double v, double *lds) {
-  v = wsum(v);
+  v = csum(v);
   int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   __syncthreads();
   if (l == 0) lds[w] = v;
@@ -79,7 +58,7 @@ __device__ inline double bsum(double v, double *lds) {
 }
 
 __device__ inline MaxLoc bmax(MaxLoc a, MaxLoc *lds) {
-  a = wmax(a);
+  a = cmax(a);
   int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   __syncthreads();
   if (l == 0) lds[w] = a;
@@ -90,21 +69,10 @@ __device__ inline MaxLoc bmax(MaxLoc a, MaxLoc *lds) {
   return r;
 }
 
-__device__ inline double rsum(const double *part, int nb, double *lds) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < nb; i += blockDim.x) s = s + part[i];
-  return bsum(s, lds);
-}
-
 __device__ inline MaxLoc rmaxl(const MaxLoc *part, int nb, MaxLoc *lds) {
   MaxLoc a{0.0, -1};
   for (int i = threadIdx.x; i < nb; i += blockDim.x) a = maxloc_pick(a, part[i]);
   return bmax(a, lds);
-}
-
-__device__ inline int is_close_(double a, double b) {
-  if (a == b) return 1;
-  return fabs(a - b) <= fmax(DSAME_F * fmax(fabs(a), fabs(b)), 0.0);
 }
 
 template <typename TP>
@@ -1283,38 +1251,40 @@ __global__ void k_f_flush(int np, TX *__restrict__ x, const TV *__restrict__ p,
 // scalar kernels
 // ---------------------------------------------------------------------------
 
-__device__ inline void testcnvg_(int icnvgopt, int *icnvg, int iiter, double dvmax, double rmax,
-                                 double rmax0, double epfact, double dvclose, double rclose) {
-  if (icnvgopt == 0) {
-    if (fabs(dvmax) <= dvclose && fabs(rmax) <= rclose) *icnvg = 1;
-  } else if (icnvgopt == 1) {
-    if (fabs(dvmax) <= dvclose && fabs(rmax) <= rclose) *icnvg = iiter == 1 ? 1 : -1;
-  } else if (icnvgopt == 2) {
-    if (fabs(dvmax) <= dvclose || rmax <= rclose) *icnvg = 1;
-    else if (rmax <= rmax0 * epfact) *icnvg = -1;
-  } else if (icnvgopt == 3) {
-    if (fabs(dvmax) <= dvclose) *icnvg = 1;
-    else if (rmax <= rmax0 * rclose) *icnvg = -1;
-  } else if (icnvgopt == 4) {
-    if (fabs(dvmax) <= dvclose && rmax <= rclose) *icnvg = 1;
-    else if (rmax <= rmax0 * epfact) *icnvg = -1;
-  }
-}
-
 // End of a round: test the iteration whose residual the preconditioner
 // kernels just produced, then rho / beta of the next iteration.
 // Colour partials sit at part[slot * nblk + b] for b < ncol (the colour
 // kernels' grid).
-// The one-block scalar kernels run MF6_RBLOCK threads, so each thread adds
-// only a few of the (thousands of) block partials: their loads come from
-// other XCDs' writes and the loop over them is latency-bound.
+// The one-block scalar kernels are bound by the latency of the partials (other
+// XCDs' writes) and of the reduction after them, not by work: MF6_RBLOCK
+// threads with two partials of every array in flight each, DPP sums within a
+// wave, and one more DPP step over the 16 waves' sums, a row of 16 lanes per
+// quantity.  (Shuffles through LDS and one thread adding the waves' sums took
+// 8.7 us and 4.0 us at 7x251x333, with fewer partials; now 4.1 and 3.2, and 5.9 and
+// 4.4 at 10x1000x1000.)
 #define MF6_RBLOCK 1024
+static_assert(MF6_RBLOCK / 64 == 16, "a row of 16 lanes holds the waves' sums");
+
+// sum and maximum over each row of 16 lanes
+__device__ inline double row_sum(double v) {
+  v = v + dpp64<DPP_X1>(v);
+  v = v + dpp64<DPP_X2>(v);
+  v = v + dpp64<DPP_HMIRROR>(v);
+  return v + dpp64<DPP_MIRROR>(v);
+}
+__device__ inline MaxLoc row_max(MaxLoc v) {
+  v = cmax_dpp<DPP_X1>(v);
+  v = cmax_dpp<DPP_X2>(v);
+  v = cmax_dpp<DPP_HMIRROR>(v);
+  return cmax_dpp<DPP_MIRROR>(v);
+}
 
 __global__ void __launch_bounds__(MF6_RBLOCK) k_f_round(KState *st, FState *fs,
                                                         const double *part,
                                                         const MaxLoc *mpart, int nblk,
                                                         int ncol, double *hist, int *hloc,
-                                                        int ncoarse = 0, int nonsym = 0) {
+                                                        FoldHost *hf, int ncoarse = 0,
+                                                        int nonsym = 0) {
   __shared__ double lds[4][MF6_RBLOCK / 64];
   __shared__ MaxLoc mlds[2][MF6_RBLOCK / 64];
   // the state is read before the partials (and the stop flag is only acted
@@ -1322,49 +1292,70 @@ __global__ void __launch_bounds__(MF6_RBLOCK) k_f_round(KState *st, FState *fs,
   const int stop = st->stop;
   KState S;
   double pmax = 0.0;
-  int ploc = -1;
+  int ploc = -1, restart = 0;
   if (threadIdx.x == 0) {
     S = *st;
     pmax = fs->pmax;
     ploc = fs->ploc;
+    restart = fs->restart;
   }
-  // the six reductions in one pass over the partials (independent loads in
-  // flight together); per slot the summation order is that of rsum/rmaxl
-  double a[4] = {0.0, 0.0, 0.0, 0.0};
-  MaxLoc mm[2] = {{0.0, -1}, {0.0, -1}};
-  for (int i = threadIdx.x; i < ncol; i += blockDim.x) {
-    a[0] = a[0] + part[P_SS_R * nblk + i];
-    a[1] = a[1] + part[P_SS_B * nblk + i];
-    a[2] = a[2] + part[P_RHO_B * nblk + i];
-    a[3] = a[3] + part[P_RHO_R * nblk + i];
-    mm[0] = maxloc_pick(mm[0], mpart[M_D_R * nblk + i]);
-    mm[1] = maxloc_pick(mm[1], mpart[M_D_B * nblk + i]);
-  }
+  // the six reductions in one pass over the partials, two slots of each per
+  // trip (a slot off the end is read again at the last one and dropped)
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  MaxLoc m0{0.0, -1}, m1{0.0, -1};
   // two-level preconditioner: rho gains rc.yc (partials of the coarse GEMV)
-  for (int i = threadIdx.x; i < ncoarse; i += blockDim.x) a[3] = a[3] + part[P_RHO_C * nblk + i];
-  const int w = threadIdx.x >> 6, ln = threadIdx.x & 63;
+  double rc = 0.0;
+  const int nmax = ncol > ncoarse ? ncol : ncoarse;
+  for (int i0 = threadIdx.x; i0 < nmax; i0 += 2 * MF6_RBLOCK) {
+    double v[2][4], c[2] = {0.0, 0.0};
+    MaxLoc w[2][2];
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    a[q] = wsum(a[q]);
-    if (ln == 0) lds[q][w] = a[q];
+    for (int u = 0; u < 2; u++) {
+      const int i = i0 + u * MF6_RBLOCK, j = i < ncol ? i : ncol - 1;
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[u][q] = part[q * nblk + j];
+      w[u][0] = mpart[M_D_R * nblk + j];
+      w[u][1] = mpart[M_D_B * nblk + j];
+      if (ncoarse > 0) c[u] = part[P_RHO_C * nblk + (i < ncoarse ? i : ncoarse - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int i = i0 + u * MF6_RBLOCK;
+      if (i < ncoarse) rc = rc + c[u];
+      if (i >= ncol) continue;
+      a0 = a0 + v[u][0];
+      a1 = a1 + v[u][1];
+      a2 = a2 + v[u][2];
+      a3 = a3 + v[u][3];
+      m0 = maxloc_pick(m0, w[u][0]);
+      m1 = maxloc_pick(m1, w[u][1]);
+    }
   }
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    mm[q] = wmax(mm[q]);
-    if (ln == 0) mlds[q][w] = mm[q];
+  a0 = csum(a0);
+  a1 = csum(a1);
+  a2 = csum(a2);
+  a3 = csum(a3 + rc);
+  m0 = cmax(m0);
+  m1 = cmax(m1);
+  const int w = threadIdx.x >> 6, ln = threadIdx.x & 63;
+  if (ln == 0) {
+    lds[P_SS_R][w] = a0;
+    lds[P_SS_B][w] = a1;
+    lds[P_RHO_B][w] = a2;
+    lds[P_RHO_R][w] = a3;
+    mlds[M_D_R][w] = m0;
+    mlds[M_D_B][w] = m1;
   }
   __syncthreads();
-  if (threadIdx.x != 0 || stop) return;
-  double tot[4] = {0.0, 0.0, 0.0, 0.0};
-  MaxLoc mt[2] = {{0.0, -1}, {0.0, -1}};
-  for (int v = 0; v < (int)(blockDim.x >> 6); v++) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) tot[q] = tot[q] + lds[q][v];
-    mt[0] = maxloc_pick(mt[0], mlds[0][v]);
-    mt[1] = maxloc_pick(mt[1], mlds[1][v]);
-  }
-  const double ssr = tot[0], ssb = tot[1], rb = tot[2], rr = tot[3];
-  MaxLoc md = maxloc_pick(mt[0], mt[1]);
+  if (threadIdx.x >= 64 || stop) return;
+  // wave 0: row q of the lanes adds quantity q over the waves
+  const double tot = row_sum(lds[ln >> 4][ln & 15]);
+  const MaxLoc mt = row_max(mlds[(ln >> 4) & 1][ln & 15]);
+  const double ssr = __shfl(tot, 16 * P_SS_R), ssb = __shfl(tot, 16 * P_SS_B);
+  const double rb = __shfl(tot, 16 * P_RHO_B), rr = __shfl(tot, 16 * P_RHO_R);
+  const MaxLoc md = maxloc_pick(MaxLoc{__shfl(mt.v, 0), __shfl(mt.loc, 0)},
+                                MaxLoc{__shfl(mt.v, 16), __shfl(mt.loc, 16)});
+  if (threadIdx.x != 0) return;
   double rho_new = rb + rr;
   int it = S.iter;   // iteration whose residual was just formed (0: initial)
   fs->apend_d = 0.0;
@@ -1388,18 +1379,23 @@ __global__ void __launch_bounds__(MF6_RBLOCK) k_f_round(KState *st, FState *fs,
     int o = S.icnvgopt;
     double rcnvg = (o == 2 || o == 3 || o == 4) ? l2norm : md.v;
     int icnvg = S.icnvg;
-    testcnvg_(o, &icnvg, it, deltax, rcnvg, S.l2norm0, S.epfact, S.dvclose, S.rclose);
+    c_testcnvg(o, &icnvg, it, deltax, rcnvg, S.l2norm0, S.epfact, S.dvclose, S.rclose);
     if (rcnvg == 0.0) icnvg = 1;
     st->icnvg = icnvg;
-    if (icnvg != 0) { st->stop = 1; return; }
-    if (is_close_(S.rho, S.rho0)) { st->stop = 2; return; }
-    if (S.rho == 0.0) { st->stop = 2; return; }
-    st->rho0 = S.rho;
-    if (it >= S.itmax) { st->stop = 3; return; }
+    int why = 0;
+    if (icnvg != 0) why = 1;
+    else if (c_close(S.rho, S.rho0) || S.rho == 0.0) why = 2;
+    else st->rho0 = S.rho;
+    if (why == 0 && it >= S.itmax) why = 3;
+    if (why != 0) {
+      st->stop = why;
+      c_publish(hf, st, why);
+      return;
+    }
   }
   st->rho = rho_new;
   if (it > 0) st->beta = rho_new / S.rho;   // rho0 was just set to the old rho
-  if (fs->restart) {
+  if (restart) {
     st->beta = 0.0;
     fs->restart = 0;
   }
@@ -1427,24 +1423,33 @@ __global__ void __launch_bounds__(MF6_RBLOCK) k_f_alpha(KState *st, FState *fs,
   }
   double a = 0.0;
   MaxLoc mm{0.0, -1};
-  for (int i = threadIdx.x; i < nblk; i += blockDim.x) {
-    a = a + part[P_PQ * nblk + i];
-    mm = maxloc_pick(mm, mpart[M_P * nblk + i]);
+  for (int i0 = threadIdx.x; i0 < nblk; i0 += 4 * MF6_RBLOCK) {
+    double v[4];
+    MaxLoc w[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int i = i0 + u * MF6_RBLOCK, j = i < nblk ? i : nblk - 1;
+      v[u] = part[P_PQ * nblk + j];
+      w[u] = mpart[M_P * nblk + j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (i0 + u * MF6_RBLOCK >= nblk) continue;
+      a = a + v[u];
+      mm = maxloc_pick(mm, w[u]);
+    }
   }
   const int w = threadIdx.x >> 6, ln = threadIdx.x & 63;
-  a = wsum(a);
-  mm = wmax(mm);
+  a = csum(a);
+  mm = cmax(mm);
   if (ln == 0) { lds[w] = a; mlds[w] = mm; }
   __syncthreads();
-  if (threadIdx.x != 0 || stop) return;
-  double pq = 0.0;
-  MaxLoc mp{0.0, -1};
-  for (int v = 0; v < (int)(blockDim.x >> 6); v++) {
-    pq = pq + lds[v];
-    mp = maxloc_pick(mp, mlds[v]);
-  }
+  if (threadIdx.x >= 64 || stop) return;
+  const double pq = row_sum(lds[ln & 15]);
+  const MaxLoc mp = row_max(mlds[ln & 15]);
+  if (threadIdx.x != 0) return;
   double den = pq;
-  den = den + copysign(DPREC_F, den);
+  den = den + copysign(DPREC_C, den);
   st->pq = pq;
   st->alpha = rho / den;
   st->iter = iter + 1;
@@ -1612,13 +1617,6 @@ static void launch_pc(Mf6Handle *h, const TM *A, const TP *piv, TV *d, const TV 
                                                     cm, cs);
 }
 
-static int read_states(Mf6Handle *h) {
-  HIPCHK(hipMemcpyAsync(h->h_state, h->d_state, 3 * sizeof(KState), hipMemcpyDeviceToHost,
-                        h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  return MF6HIP_OK;
-}
-
 // Enqueue n fused FP64 CG iterations starting at an even round (the two
 // direction buffers alternate; n even keeps the parity).
 static void enqueue_fused64(Mf6Handle *h, int n, int nbc, int nb) {
@@ -1641,7 +1639,7 @@ static void enqueue_fused64(Mf6Handle *h, int n, int nbc, int nb) {
       mf6hip_tl_enqueue<double>(h, (const double *)nullptr, h->tl_yc64, h->d_part + P_RHO_C * nb,
                                 nb, st);
     k_f_round<<<1, MF6_RBLOCK, 0, s>>>(st, fs, h->d_part, h->d_mpart, nb, nbc, h->d_hist,
-                                      h->d_hloc, tl ? mf6hip_tl_nslot(h, nb) : 0, defl ? 1 : 0);
+                                      h->d_hloc, h->h_fold, tl ? mf6hip_tl_nslot(h, nb) : 0, defl ? 1 : 0);
     double *pin = pbuf[round & 1], *pout = pbuf[(round + 1) & 1];
     launch_f_pupdate<double, double>(L, nb, s, h->z, pin, pout, h->x, h->d_mpart, st, fs,
                                      tl ? h->tl_yc64 : nullptr, h->tl_cmask, h->tl);
@@ -1662,7 +1660,7 @@ static void enqueue_fused64(Mf6Handle *h, int n, int nbc, int nb) {
 // Capture FUSED_GRAPH_ITERS iterations as a graph (once per handle; the
 // buffers and grid sizes are fixed for the handle's life).  The graph holds
 // kernel launches only.
-constexpr int FUSED_GRAPH_ITERS = 8;
+constexpr int FUSED_GRAPH_ITERS = 4;
 
 static bool fused64_graph(Mf6Handle *h, int nbc, int nb) {
   if (h->cg_graph) return true;
@@ -1701,19 +1699,15 @@ int mf6hip_run_cg_fused(Mf6Handle *h) {
   const int nb = nbs > nbc ? nbs : nbc;
   double *pbuf[2] = {h->p, h->p2};
   const bool graph = !h->timing && fused64_graph(h, nbc, nb);
-  int batch = graph ? FUSED_GRAPH_ITERS : 4;
+  h->h_fold->stop = 0;   // nothing of an earlier solve is still running
   // round 0: preconditioner of the initial residual; batches are even
-  while (true) {
-    if (graph) {
-      for (int r = 0; r < batch / FUSED_GRAPH_ITERS; r++) HIPCHK(hipGraphLaunch(h->cg_graph, s));
-    } else {
-      enqueue_fused64(h, batch, nbc, nb);
-    }
+  CK(fold_batches(h, FUSED_GRAPH_ITERS, [&]() -> int {
+    if (graph) HIPCHK(hipGraphLaunch(h->cg_graph, s));
+    else enqueue_fused64(h, FUSED_GRAPH_ITERS, nbc, nb);
     HIPCHK(hipGetLastError());
-    CK(read_states(h));
-    if (h->h_state->stop) break;
-    if (batch < 64) batch *= 2;
-  }
+    return MF6HIP_OK;
+  }));
+  h->h_state[0] = h->h_fold->st;
   // apply the pending head update of the last iteration: the direction of
   // iteration m lives in pbuf[m & 1]
   int m = h->h_state->iter;
@@ -1744,6 +1738,10 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
   // coarse correction), so replacements come more often.
   const int R = h->s.inner_fp32_max > 0 ? h->s.inner_fp32_max
                                         : (h->s.preconditioner >= 2 ? 32 : 64);
+  // the replacement follows the first of 8, 24, 56, 88, ... rounds that is
+  // at least R
+  int period = 8;
+  for (int b = 16; period < R; period += b, b = 32) {}
   HIPCHK(hipMemsetAsync(fs, 0, sizeof(FState), s));
   HIPCHK(hipMemsetAsync(h->q32, 0, sizeof(float) * L.NP, s));
   HIPCHK(hipMemsetAsync(h->e32, 0, sizeof(float) * L.NP, s));
@@ -1756,43 +1754,57 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
   const bool tl = h->s.preconditioner >= 2, defl = h->s.preconditioner == 3;
   if (defl) mf6hip_tl_colsum<float>(h, h->r32);
   *icnvg = 0;
-  while (!done) {
-    int batch = 8;
-    while (true) {
-      for (int it = 0; it < batch; it++, round++) {
-        if (defl)
-          mf6hip_tl_enqueue<float>(h, (const float *)nullptr, h->tl_yc32,
-                                   h->d_part + P_RHO_C * nb, nb, st, &fs->apend_d);
-        launch_pc<TMP, float, TP>(h, Apc, piv32, h->r32, h->q32, h->zf32, h->z32, st, fs, nbc,
-                                  nb, sc);
-        if (tl && !defl)
-          mf6hip_tl_enqueue<float>(h, (const float *)nullptr, h->tl_yc32,
-                                   h->d_part + P_RHO_C * nb, nb, st);
-        k_f_round<<<1, MF6_RBLOCK, 0, s>>>(st, fs, h->d_part, h->d_mpart, nb, nbc, h->d_hist,
-                                          h->d_hloc, tl ? mf6hip_tl_nslot(h, nb) : 0, defl ? 1 : 0);
-        float *pin = pbuf[round & 1], *pout = pbuf[(round + 1) & 1];
-        launch_f_pupdate<float, float>(L, nb, s, h->z32, pin, pout, h->e32, h->d_mpart, st, fs,
-                                       tl ? h->tl_yc32 : nullptr, h->tl_cmask, h->tl);
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        if (h->timing && (h->spmv_calls++ % h->spmv_sample) == 0 &&
-            2 * (h->last_spmv_n + 1) <= (int)h->spmv_ev.size()) {
-          const int slot = h->last_spmv_n++;
-          e0 = h->spmv_ev[2 * slot];
-          e1 = h->spmv_ev[2 * slot + 1];
-        }
-        launch_f_spmv<float, float>(L, nb, s, h->A32, pout, h->q32, h->d_part, st,
-                                    defl ? h->tl_cmask : nullptr, defl ? h->tl_colsq : nullptr,
-                                    e0, e1);
-        k_f_alpha<<<1, MF6_RBLOCK, 0, s>>>(st, fs, h->d_part, h->d_mpart, nb);
+  // a batch of rounds, and the event at its end
+  auto enqueue = [&](int batch, int ev) -> int {
+    for (int it = 0; it < batch; it++, round++) {
+      if (defl)
+        mf6hip_tl_enqueue<float>(h, (const float *)nullptr, h->tl_yc32,
+                                 h->d_part + P_RHO_C * nb, nb, st, &fs->apend_d);
+      launch_pc<TMP, float, TP>(h, Apc, piv32, h->r32, h->q32, h->zf32, h->z32, st, fs, nbc,
+                                nb, sc);
+      if (tl && !defl)
+        mf6hip_tl_enqueue<float>(h, (const float *)nullptr, h->tl_yc32,
+                                 h->d_part + P_RHO_C * nb, nb, st);
+      k_f_round<<<1, MF6_RBLOCK, 0, s>>>(st, fs, h->d_part, h->d_mpart, nb, nbc, h->d_hist,
+                                        h->d_hloc, h->h_fold,
+                                        tl ? mf6hip_tl_nslot(h, nb) : 0, defl ? 1 : 0);
+      float *pin = pbuf[round & 1], *pout = pbuf[(round + 1) & 1];
+      launch_f_pupdate<float, float>(L, nb, s, h->z32, pin, pout, h->e32, h->d_mpart, st, fs,
+                                     tl ? h->tl_yc32 : nullptr, h->tl_cmask, h->tl);
+      hipEvent_t e0 = nullptr, e1 = nullptr;
+      if (h->timing && (h->spmv_calls++ % h->spmv_sample) == 0 &&
+          2 * (h->last_spmv_n + 1) <= (int)h->spmv_ev.size()) {
+        const int slot = h->last_spmv_n++;
+        e0 = h->spmv_ev[2 * slot];
+        e1 = h->spmv_ev[2 * slot + 1];
       }
-      HIPCHK(hipGetLastError());
-      CK(read_states(h));
-      if (h->h_state->stop) break;
-      if (h->h_state->iter - last_replace >= R) break;
-      if (batch < 32) batch *= 2;
+      launch_f_spmv<float, float>(L, nb, s, h->A32, pout, h->q32, h->d_part, st,
+                                  defl ? h->tl_cmask : nullptr, defl ? h->tl_colsq : nullptr,
+                                  e0, e1);
+      k_f_alpha<<<1, MF6_RBLOCK, 0, s>>>(st, fs, h->d_part, h->d_mpart, nb);
     }
-    KState hs = h->h_state[0];
-    int m = hs.iter;
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipEventRecord(h->ev_batch[ev], s));
+    return MF6HIP_OK;
+  };
+  h->h_fold->stop = 0;   // nothing of an earlier solve is still running
+  while (!done) {
+    // batches of four rounds up to the replacement, one queued ahead of the
+    // one waited for (a round after the stop costs its launches)
+    const int due = last_replace + period;
+    int ev = 0, stop = 0;
+    CK(enqueue(4, 0));
+    while (true) {
+      const bool more = round < due;
+      if (more) CK(enqueue(4, ev ^ 1));
+      HIPCHK(hipEventSynchronize(h->ev_batch[ev]));
+      stop = __atomic_load_n(&h->h_fold->stop, __ATOMIC_ACQUIRE);
+      if (stop != 0 || !more) break;
+      ev ^= 1;
+    }
+    if (stop != 0) h->h_state[0] = h->h_fold->st;
+    const KState hs = h->h_state[0];   // read where stop != 0 only
+    const int m = stop != 0 ? hs.iter : round;
     // replace the residual: x += xhat + pending alpha p ; d32 = b - A x
     // the head update of iteration m (direction p_m) is still pending, and
     // so is alpha q for d when no test ran yet: fold both into the FP64
@@ -1804,11 +1816,11 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
     k_r_residual<<<nb, MF6_BLOCK, 0, s>>>(L, h->A, h->x, h->b, h->r32, h->d_mpart);
     k_r_after<<<1, MF6_BLOCK, 0, s>>>(st, fs, h->d_mpart, nb, rout, tl ? 1 : 0);
     if (defl) mf6hip_tl_colsum<float>(h, h->r32);
-    double hr[2];
-    HIPCHK(hipMemcpyAsync(hr, rout, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
     last_replace = m;
-    if (hs.stop != 0) {
+    if (stop != 0) {
+      double hr[2];
+      HIPCHK(hipMemcpyAsync(hr, rout, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
       bool true_ok = fabs(hr[0]) <= h->s.rclose;
       if (hs.stop == 1 && true_ok) { *icnvg = 1; done = true; break; }
       if (hs.stop == 3 || m >= total_budget) { done = true; break; }
@@ -1820,6 +1832,7 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
       h->h_state[0].icnvg = 0;
       h->h_state[0].iter = m;
       HIPCHK(hipMemcpyAsync(st, h->h_state, sizeof(KState), hipMemcpyHostToDevice, s));
+      h->h_fold->stop = 0;
     }
   }
   *iters = h->h_state[0].iter;

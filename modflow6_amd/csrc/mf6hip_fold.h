@@ -186,9 +186,8 @@ __device__ inline void c_testcnvg(int o, int *icnvg, int it, double dvmax, doubl
 // What a solve leaves in pinned host memory when its test stops it: the host
 // needs no copy to see it, only the end of the batch that holds the test.
 __device__ inline void c_publish(FoldHost *hf, const KState *st, int stop) {
-  KState f = *st;
-  f.stop = stop;
-  hf->st = f;
+  hf->st = *st;
+  hf->st.stop = stop;
   __threadfence_system();
   __hip_atomic_store(&hf->stop, stop, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
