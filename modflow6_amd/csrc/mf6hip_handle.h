@@ -37,6 +37,7 @@ struct DevPackage {
 // the outcome of a folded solve, in pinned host memory
 struct FoldHost {
   int stop;
+  int off;     // flexible CG: the network is off for the rest of the solve
   KState st;
 };
 
@@ -252,8 +253,6 @@ int mf6hip_dxmax(Mf6Handle *h, double *hncg, int *lrch, const double *xa,
 
 // solver pieces shared with the flexible CG (mf6hip_fcg.hip)
 // z = ILU0(r); the kernels return at once when st is given and st->stop is set
-int mf6hip_ilu_apply64(Mf6Handle *h, const double *r, double *z, const KState *st);
-int mf6hip_spmv64(Mf6Handle *h, const double *x, double *y);
 int mf6hip_run_fcg(Mf6Handle *h);
 int mf6hip_stage_system(const Layout &L, const int *ia1, int nja, const double *amat,
                         const double *rhs, const double *x0, double relax, double *A64,

@@ -1055,18 +1055,6 @@ int mf6hip_stage_system(const Layout &L, const int *ia1, int nja, const double *
   return rc;
 }
 
-int mf6hip_ilu_apply64(Mf6Handle *h, const double *r, double *z, const KState *st) {
-  launch_ilu_apply<double, double, double>(h, h->A, h->invpiv, r, h->zf, z, st);
-  HIPCHK(hipGetLastError());
-  return MF6HIP_OK;
-}
-
-int mf6hip_spmv64(Mf6Handle *h, const double *x, double *y) {
-  launch_spmv<double, double>(h, h->A, x, y);
-  HIPCHK(hipGetLastError());
-  return MF6HIP_OK;
-}
-
 static void timed_spmv_begin(Mf6Handle *h, int &slot) {
   slot = -1;
   if (!h->timing) return;

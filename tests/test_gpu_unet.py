@@ -214,6 +214,35 @@ def test_fcg_without_network_matches_pcg():
     assert np.max(np.abs(xl - xr)) < 10 * case.ims.inner_dvclose
 
 
+# the layer bounds of the sweeps (4, 8, 16, 32) with partial chunks, 64 and 256
+# threads a block, a column or a chunk of it per thread, a single row; more
+# directions than one pass of dot products takes (fcg_m > 8)
+@pytest.mark.parametrize("shape,fcg_m,net", [
+    ((1, 1, 64), 8, False), ((3, 33, 17), 12, False), ((5, 24, 21), 8, True),
+    ((9, 20, 31), 9, True), ((17, 14, 15), 3, False), ((32, 10, 11), 8, False),
+    ((3, 130, 141), 8, True), ((1, 380, 367), 8, False)])
+def test_fcg_shapes_match_pcg(shape, fcg_m, net):
+    nlay, nrow, ncol = shape
+    case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=5 if nrow > 1 else 1)
+    sim, amat, rhs, x0 = oracle_system(case)
+    ref = device_solver(case)
+    xr = x0.copy()
+    ic, it_ref = ref.solve(1, amat, rhs, xr)
+    ref.destroy()
+    sv = device_solver(case, preconditioner=1)
+    u = UNet(nlay, nrow, ncol, 3, (16, 16, 32, 32), seed=2) if net else None
+    sv.attach_unet(u, features(case), fcg_m=fcg_m)
+    xl = x0.copy()
+    icl, it_l = sv.solve(1, amat, rhs, xl)
+    sv.destroy()
+    if u:
+        u.destroy()
+    assert ic == 1 and icl == 1
+    if not net:
+        assert abs(it_l - it_ref) <= max(3, it_ref // 20)
+    assert np.max(np.abs(xl - xr)) < 10 * case.ims.inner_dvclose
+
+
 def test_trained_network_gain_over_flexible_cg_without_it():
     """What the trained network gains: a 6-level network trained on the
     device on ILU0-PCG (residual, error) pairs of eight seeded 4 x 64 x 64
