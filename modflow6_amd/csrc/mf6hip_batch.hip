@@ -27,10 +27,11 @@
 // residual replacement restarts the directions.
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
-#include "mf6hip_handle.h"
+#include "mf6hip_fold.h"
 
 namespace {
 
@@ -69,51 +70,13 @@ struct Tile {
 enum { P_SS_R = 0, P_SS_B = 1, P_RHO_B = 2, P_RHO_R = 3, P_PQ = 4, P_RHO_C = 5 };
 enum { M_D_R = 0, M_D_B = 1, M_P = 2, M_TRUE = 3 };
 
-template <typename T>
-__device__ inline T wsum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
-__device__ inline MaxLoc wmax(MaxLoc a) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    MaxLoc b;
-    b.v = __shfl_xor(a.v, o);
-    b.loc = __shfl_xor(a.loc, o);
-    a = maxloc_pick(a, b);
-  }
-  return a;
-}
-
-// block sum / max, result valid in thread 0
-__device__ inline double bsum(double v, double *lds) {
-  v = wsum(v);
-  const int w = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) lds[w] = v;
-  __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) s = s + lds[i];
-  return s;
-}
-
-__device__ inline MaxLoc bmax(MaxLoc a, MaxLoc *lds) {
-  a = wmax(a);
-  const int w = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) lds[w] = a;
-  __syncthreads();
-  MaxLoc r{0.0, -1};
-  if (threadIdx.x == 0)
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) r = maxloc_pick(r, lds[i]);
-  return r;
-}
-
 // ---------------------------------------------------------------------------
-// stencil kernels (FP32)
+// stencil kernels (FP32).  A tile is a few hundred columns, each walked by one
+// thread: bound by the latency of a layer's loads (one to three waves a SIMD), so
+// the loads of C_CH layers are issued before the first is used.  Eight systems of
+// 64 to 320 columns a side and five layers: 15.6 ms with loops that loaded layer
+// by layer, scalar kernels that reduced through LDS shuffles and heads reordered
+// on the host, 10.3 ms now.
 // ---------------------------------------------------------------------------
 
 __global__ void __launch_bounds__(MF6_BLOCK) kb_red_fwd(const BSys *sys, const Tile *tiles,
@@ -122,47 +85,66 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_red_fwd(const BSys *sys, const T
                                                         const float *q, float *zf, double *part,
                                                         MaxLoc *mpart, int T, const KState *st,
                                                         const BFState *fs) {
-  __shared__ double lds[8];
-  __shared__ MaxLoc mlds[8];
+  __shared__ double lds[4];
+  __shared__ MaxLoc mlds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int s = tiles[tile].sys;
-    if (st[s].stop) continue;
+    const int s = tiles[tile].sys, base = tiles[tile].base;
     const Layout L = sys[s].L;
     const float *A = A32 + sys[s].aoff;
-    const float *pv = piv + sys[s].voff;
-    float *dd = d + sys[s].voff;
-    const float *qq = q + sys[s].voff;
-    float *zz = zf + sys[s].voff;
-    const int NP = L.NP;
+    const float *__restrict__ pv = piv + sys[s].voff;
+    float *__restrict__ dd = d + sys[s].voff;
+    const float *__restrict__ qq = q + sys[s].voff;
+    float *__restrict__ zz = zf + sys[s].voff;
+    const float *__restrict__ A6 = A + 6 * (size_t)L.NP;
     const float alpha = (float)fs[s].apend_d;
+    if (st[s].stop) continue;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     double ss = 0.0;
     MaxLoc md{0.0, -1};
     for (int c = 0; c < cpt; c++) {
-      const int h2 = tiles[tile].base + c * blockDim.x + threadIdx.x;
+      const int h2 = base + c * MF6_BLOCK + threadIdx.x;
       if (h2 >= L.HP0) continue;
       const int l = col_l(L, 0, h2);
       float zup = 0.f, lup = 0.f;
-      for (int k = 0; k < L.nlay; k++) {
-        const int pos = k * L.HP + h2;
-        float dv = dd[pos];
-        dv = dv - alpha * qq[pos];
-        dd[pos] = dv;
-        md = maxloc_pick(md, MaxLoc{(double)dv, k * L.NRC + l});
-        ss = ss + (double)dv * (double)dv;
-        float tv = dv;
-        if (k > 0) tv = tv - lup * zup;
-        zz[pos] = tv;
-        zup = tv;
-        lup = A[6 * NP + pos] * pv[pos];
+      for (int k0 = 0; k0 < L.nlay; k0 += C_CH) {
+        float dv[C_CH], qv[C_CH], a6[C_CH], pq[C_CH];
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int pos = (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * L.HP + h2;
+          dv[u] = dd[pos];
+          qv[u] = qq[pos];
+          a6[u] = A6[pos];
+          pq[u] = pv[pos];
+        }
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u;
+          if (k >= L.nlay) continue;
+          const int pos = k * L.HP + h2;
+          const float v = dv[u] - alpha * qv[u];
+          dd[pos] = v;
+          md = maxloc_pick(md, MaxLoc{(double)v, k * L.NRC + l});
+          ss = ss + (double)v * (double)v;
+          float tv = v;
+          if (k > 0) tv = tv - lup * zup;
+          zz[pos] = tv;
+          zup = tv;
+          lup = a6[u] * pq[u];
+        }
       }
     }
-    ss = bsum(ss, lds);
-    if (threadIdx.x == 0) part[P_SS_R * T + tile] = ss;
-    md = bmax(md, mlds);
-    if (threadIdx.x == 0) mpart[M_D_R * T + tile] = md;
+    ss = call_sum<MF6_BLOCK>(ss, lds);
+    md = call_max<MF6_BLOCK>(md, mlds);
+    if (threadIdx.x == 0) {
+      part[P_SS_R * T + tile] = ss;
+      mpart[M_D_R * T + tile] = md;
+    }
   }
 }
 
+// NL bounds every system's layers at compile time: a column's values stay in
+// registers between the forward and the backward sweep
+template <int NL>
 __global__ void __launch_bounds__(MF6_BLOCK) kb_black(const BSys *sys, const Tile *tiles,
                                                       int ntiles, int cpt, const float *A32,
                                                       const float *piv, float *d, const float *q,
@@ -170,88 +152,104 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_black(const BSys *sys, const Til
                                                       MaxLoc *mpart, int T, const KState *st,
                                                       const BFState *fs,
                                                       const unsigned *cmask, double *colsum) {
-  __shared__ double lds[8];
-  __shared__ MaxLoc mlds[8];
+  __shared__ double lds[2][4];
+  __shared__ MaxLoc mlds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int s = tiles[tile].sys;
-    if (st[s].stop) continue;
+    const int s = tiles[tile].sys, base = tiles[tile].base;
     const Layout L = sys[s].L;
-    const float *A = A32 + sys[s].aoff;
-    const float *pv = piv + sys[s].voff;
+    const float *__restrict__ A = A32 + sys[s].aoff;
+    const float *__restrict__ pv = piv + sys[s].voff;
     const unsigned *cms = colsum ? cmask + sys[s].cmo : nullptr;
     double *css = colsum ? colsum + sys[s].cso : nullptr;
-    float *dd = d + sys[s].voff;
-    const float *qq = q + sys[s].voff;
-    const float *zr = zf + sys[s].voff;
-    float *zz = z + sys[s].voff;
-    const int NP = L.NP;
+    float *__restrict__ dd = d + sys[s].voff;
+    const float *__restrict__ qq = q + sys[s].voff;
+    const float *__restrict__ zr = zf + sys[s].voff;
+    float *__restrict__ zz = z + sys[s].voff;
+    const int NP = L.NP, HP = L.HP;
     const float alpha = (float)fs[s].apend_d;
+    if (st[s].stop) continue;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     double ss = 0.0, rho = 0.0;
     MaxLoc md{0.0, -1};
     for (int c = 0; c < cpt; c++) {
-      const int h2 = tiles[tile].base + c * blockDim.x + threadIdx.x;
+      const int h2 = base + c * MF6_BLOCK + threadIdx.x;
       if (h2 >= L.HP1) continue;
-      const int l = col_l(L, 1, h2);
-      const int i = l / L.ncol, j = l - i * L.ncol;
       // off-grid neighbours read position 0 (in range); a select drops
       // their term, so no lane waits inside a branch
-      const bool hb = i > 0, hl = j > 0, hr = j < L.ncol - 1, hf = i < L.nrow - 1;
-      const int ib = hb ? hn(l, -L.ncol) : 0;
-      const int il = hl ? hn(l, -1) : 0;
-      const int ir = hr ? hn(l, 1) : 0;
-      const int ifr = hf ? hn(l, L.ncol) : 0;
+      const CGeo G(L, 1, h2);
+      const unsigned cm = css ? cms[HP + h2] : 0u;
       float zup = 0.f, lup = 0.f;
-      const unsigned cm = css ? cms[L.HP + h2] : 0u;
       double cs = 0.0;
-      for (int k = 0; k < L.nlay; k++) {
-        const int pos = L.H + k * L.HP + h2;
-        const int rb = k * L.HP;
-        float dv = dd[pos];
-        dv = dv - alpha * qq[pos];
-        dd[pos] = dv;
-        if ((cm >> k) & 1u) cs = cs + (double)dv;
-        md = maxloc_pick(md, MaxLoc{(double)dv, k * L.NRC + l});
-        ss = ss + (double)dv * (double)dv;
-        float tv = dv;
-        {
-          const auto t_ = (A[5 * NP + rb + ib] * pv[rb + ib]) * zr[rb + ib];
-          tv = hb ? tv - t_ : tv;
+      float zc[NL], pc[NL], ac[NL], dc[NL];
+#pragma unroll
+      for (int k0 = 0; k0 < NL; k0 += C_CH) {
+        if (k0 >= L.nlay) break;
+        float ab[C_CH], al[C_CH], ar[C_CH], af[C_CH], pb[C_CH], pl[C_CH], pr[C_CH], pf[C_CH];
+        float zb[C_CH], zl[C_CH], zq[C_CH], zw[C_CH], qv[C_CH];
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
+          const int pos = L.H + k * HP + h2, rb = k * HP;
+          dc[k0 + u] = dd[pos];
+          qv[u] = qq[pos];
+          ab[u] = A[5 * NP + rb + G.ib];
+          pb[u] = pv[rb + G.ib];
+          zb[u] = zr[rb + G.ib];
+          al[u] = A[4 * NP + rb + G.il];
+          pl[u] = pv[rb + G.il];
+          zl[u] = zr[rb + G.il];
+          ar[u] = A[4 * NP + pos];
+          pr[u] = pv[rb + G.ir];
+          zq[u] = zr[rb + G.ir];
+          af[u] = A[5 * NP + pos];
+          pf[u] = pv[rb + G.ifr];
+          zw[u] = zr[rb + G.ifr];
+          ac[k0 + u] = A[6 * NP + pos];
+          pc[k0 + u] = pv[pos];
         }
-        {
-          const auto t_ = (A[4 * NP + rb + il] * pv[rb + il]) * zr[rb + il];
-          tv = hl ? tv - t_ : tv;
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u;
+          if (k >= L.nlay) continue;
+          const float v = dc[k] - alpha * qv[u];
+          dc[k] = v;
+          dd[L.H + k * HP + h2] = v;
+          if ((cm >> k) & 1u) cs = cs + (double)v;
+          md = maxloc_pick(md, MaxLoc{(double)v, k * L.NRC + G.l});
+          ss = ss + (double)v * (double)v;
+          float tv = v;
+          tv = G.hb ? tv - (ab[u] * pb[u]) * zb[u] : tv;
+          tv = G.hl ? tv - (al[u] * pl[u]) * zl[u] : tv;
+          tv = G.hr ? tv - (ar[u] * pr[u]) * zq[u] : tv;
+          tv = G.hf ? tv - (af[u] * pf[u]) * zw[u] : tv;
+          if (k > 0) tv = tv - lup * zup;
+          zc[k] = tv;
+          zup = tv;
+          lup = ac[k] * pc[k];
         }
-        {
-          const auto t_ = (A[4 * NP + pos] * pv[rb + ir]) * zr[rb + ir];
-          tv = hr ? tv - t_ : tv;
-        }
-        {
-          const auto t_ = (A[5 * NP + pos] * pv[rb + ifr]) * zr[rb + ifr];
-          tv = hf ? tv - t_ : tv;
-        }
-        if (k > 0) tv = tv - lup * zup;
-        zz[pos] = tv;
-        zup = tv;
-        lup = A[6 * NP + pos] * pv[pos];
       }
-      if (css) css[l] = cs;
+      if (css) css[G.l] = cs;
       float zdn = 0.f;
-      for (int k = L.nlay - 1; k >= 0; k--) {
-        const int pos = L.H + k * L.HP + h2;
-        float tv = zz[pos];
-        if (k < L.nlay - 1) tv = tv - A[6 * NP + pos] * zdn;
-        tv = tv * pv[pos];
-        zz[pos] = tv;
-        zdn = tv;
-        rho = rho + (double)dd[pos] * (double)tv;
+#pragma unroll
+      for (int k = NL - 1; k >= 0; k--) {
+        if (k < L.nlay) {
+          float tv = zc[k];
+          if (k < L.nlay - 1) tv = tv - ac[k] * zdn;
+          tv = tv * pc[k];
+          zz[L.H + k * HP + h2] = tv;
+          zdn = tv;
+          rho = rho + (double)dc[k] * (double)tv;
+        }
       }
     }
-    ss = bsum(ss, lds);
-    if (threadIdx.x == 0) part[P_SS_B * T + tile] = ss;
-    rho = bsum(rho, lds);
-    if (threadIdx.x == 0) part[P_RHO_B * T + tile] = rho;
-    md = bmax(md, mlds);
-    if (threadIdx.x == 0) mpart[M_D_B * T + tile] = md;
+    ss = call_sum<MF6_BLOCK>(ss, lds[0]);
+    rho = call_sum<MF6_BLOCK>(rho, lds[1]);
+    md = call_max<MF6_BLOCK>(md, mlds);
+    if (threadIdx.x == 0) {
+      part[P_SS_B * T + tile] = ss;
+      part[P_RHO_B * T + tile] = rho;
+      mpart[M_D_B * T + tile] = md;
+    }
   }
 }
 
@@ -261,66 +259,68 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_red_bwd(const BSys *sys, const T
                                                         const float *zf, float *z, double *part,
                                                         int T, const KState *st,
                                                         const unsigned *cmask, double *colsum) {
-  __shared__ double lds[8];
+  __shared__ double lds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int s = tiles[tile].sys;
-    if (st[s].stop) continue;
+    const int s = tiles[tile].sys, base = tiles[tile].base;
     const Layout L = sys[s].L;
-    const float *A = A32 + sys[s].aoff;
-    const float *pv = piv + sys[s].voff;
+    const float *__restrict__ A = A32 + sys[s].aoff;
+    const float *__restrict__ pv = piv + sys[s].voff;
     const unsigned *cms = colsum ? cmask + sys[s].cmo : nullptr;
     double *css = colsum ? colsum + sys[s].cso : nullptr;
-    const float *dd = d + sys[s].voff;
-    const float *zr = zf + sys[s].voff;
+    const float *__restrict__ dd = d + sys[s].voff;
+    const float *__restrict__ zr = zf + sys[s].voff;
     float *zz = z + sys[s].voff;
-    const int NP = L.NP;
+    const int NP = L.NP, HP = L.HP;
+    if (st[s].stop) continue;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     double rho = 0.0;
     for (int c = 0; c < cpt; c++) {
-      const int h2 = tiles[tile].base + c * blockDim.x + threadIdx.x;
+      const int h2 = base + c * MF6_BLOCK + threadIdx.x;
       if (h2 >= L.HP0) continue;
-      const int l = col_l(L, 0, h2);
-      const int i = l / L.ncol, j = l - i * L.ncol;
-      // off-grid neighbours read position 0 (in range); a select drops
-      // their term, so no lane waits inside a branch
-      const bool hb = i > 0, hl = j > 0, hr = j < L.ncol - 1, hf = i < L.nrow - 1;
-      const int ib = hb ? hn(l, -L.ncol) : 0;
-      const int il = hl ? hn(l, -1) : 0;
-      const int ir = hr ? hn(l, 1) : 0;
-      const int ifr = hf ? hn(l, L.ncol) : 0;
-      float zdn = 0.f;
+      const CGeo G(L, 0, h2);
       const unsigned cm = css ? cms[h2] : 0u;
+      float zdn = 0.f;
       double cs = 0.0;
-      for (int k = L.nlay - 1; k >= 0; k--) {
-        const int pos = k * L.HP + h2;
-        const int bb = L.H + k * L.HP;
-        float tv = zr[pos];
-        if (k < L.nlay - 1) tv = tv - A[6 * NP + pos] * zdn;
-        {
-          const auto t_ = A[5 * NP + bb + ib] * zz[bb + ib];
-          tv = hb ? tv - t_ : tv;
+      for (int k0 = L.nlay - 1; k0 >= 0; k0 -= C_CH) {
+        float zv[C_CH], a6[C_CH], ab[C_CH], al[C_CH], ar[C_CH], af[C_CH], zb[C_CH], zl[C_CH],
+            zq[C_CH], zw[C_CH], pp[C_CH], dv[C_CH];
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 - u > 0 ? k0 - u : 0;
+          const int pos = k * HP + h2, bb = L.H + k * HP;
+          zv[u] = zr[pos];
+          a6[u] = A[6 * NP + pos];
+          ab[u] = A[5 * NP + bb + G.ib];
+          zb[u] = zz[bb + G.ib];
+          al[u] = A[4 * NP + bb + G.il];
+          zl[u] = zz[bb + G.il];
+          ar[u] = A[4 * NP + pos];
+          zq[u] = zz[bb + G.ir];
+          af[u] = A[5 * NP + pos];
+          zw[u] = zz[bb + G.ifr];
+          pp[u] = pv[pos];
+          dv[u] = dd[pos];
         }
-        {
-          const auto t_ = A[4 * NP + bb + il] * zz[bb + il];
-          tv = hl ? tv - t_ : tv;
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 - u;
+          if (k < 0) continue;
+          float tv = zv[u];
+          if (k < L.nlay - 1) tv = tv - a6[u] * zdn;
+          tv = G.hb ? tv - ab[u] * zb[u] : tv;
+          tv = G.hl ? tv - al[u] * zl[u] : tv;
+          tv = G.hr ? tv - ar[u] * zq[u] : tv;
+          tv = G.hf ? tv - af[u] * zw[u] : tv;
+          tv = tv * pp[u];
+          zz[k * HP + h2] = tv;
+          zdn = tv;
+          rho = rho + (double)dv[u] * (double)tv;
+          if ((cm >> k) & 1u) cs = cs + (double)dv[u];
         }
-        {
-          const auto t_ = A[4 * NP + pos] * zz[bb + ir];
-          tv = hr ? tv - t_ : tv;
-        }
-        {
-          const auto t_ = A[5 * NP + pos] * zz[bb + ifr];
-          tv = hf ? tv - t_ : tv;
-        }
-        tv = tv * pv[pos];
-        zz[pos] = tv;
-        zdn = tv;
-        const float dv = dd[pos];
-        rho = rho + (double)dv * (double)tv;
-        if ((cm >> k) & 1u) cs = cs + (double)dv;
       }
-      if (css) css[l] = cs;
+      if (css) css[G.l] = cs;
     }
-    rho = bsum(rho, lds);
+    rho = call_sum<MF6_BLOCK>(rho, lds);
     if (threadIdx.x == 0) part[P_RHO_R * T + tile] = rho;
   }
 }
@@ -332,46 +332,56 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_pupdate(const BSys *sys, const T
                                                         MaxLoc *mpart, int T, const KState *st,
                                                         const BFState *fs, const unsigned *cmask,
                                                         const float *yc) {
-  __shared__ MaxLoc mlds[8];
+  __shared__ MaxLoc mlds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int s = tiles[tile].sys;
-    if (st[s].stop) continue;
+    const int s = tiles[tile].sys, base = tiles[tile].base;
     const Layout L = sys[s].L;
     const long long vo = sys[s].voff;
-    const float *pin = (fs[s].pcur ? p1 : p0) + vo;
-    float *pout = (fs[s].pcur ? p0 : p1) + vo;
-    const float *zz = z + vo;
-    float *ee = e + vo;
+    const float *__restrict__ pin = (fs[s].pcur ? p1 : p0) + vo;
+    float *__restrict__ pout = (fs[s].pcur ? p0 : p1) + vo;
+    const float *__restrict__ zz = z + vo;
+    float *__restrict__ ee = e + vo;
     const bool first = st[s].iter == 0;
     const float beta = (float)st[s].beta;
     const float ax = (float)fs[s].apend_x;
+    if (st[s].stop) continue;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     MaxLoc mp{0.0, -1};
     for (int c = 0; c < cpt; c++) {
-      const int t = tiles[tile].base + c * blockDim.x + threadIdx.x;
+      const int t = base + c * MF6_BLOCK + threadIdx.x;
       const int cc = t & 1, h2 = t >> 1;
       if (h2 >= ncols_of(L, cc)) continue;
       const int l = col_l(L, cc, h2);
       const int own = cc * L.H + h2;
       // two-level: z completed by the prolongation of the coarse correction
       const unsigned cm = yc ? cmask[sys[s].cmo + cc * L.HP + h2] : 0u;
-      const float yv = cm ? yc[sys[s].cvo + tl_agg(sys[s].tl, L, l)] : 0.f;
-      for (int k = 0; k < L.nlay; k++) {
-        const int pos = own + k * L.HP;
-        float zv = zz[pos];
-        if ((cm >> k) & 1u) zv = zv + yv;
-        float pv;
-        if (first) {
-          pv = zv;
-        } else {
-          const float po = pin[pos];
-          pv = zv + beta * po;
-          ee[pos] = ee[pos] + ax * po;
+      const float yv = yc ? yc[sys[s].cvo + tl_agg(sys[s].tl, L, l)] : 0.f;
+      for (int k0 = 0; k0 < L.nlay; k0 += C_CH) {
+        float zv[C_CH], po[C_CH], ev[C_CH];
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int pos = own + (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * L.HP;
+          zv[u] = zz[pos];
+          po[u] = pin[pos];
+          ev[u] = ee[pos];
         }
-        pout[pos] = pv;
-        mp = maxloc_pick(mp, MaxLoc{(double)pv, k * L.NRC + l});
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u;
+          if (k >= L.nlay) continue;
+          const int pos = own + k * L.HP;
+          float v = zv[u];
+          if ((cm >> k) & 1u) v = v + yv;
+          if (!first) {
+            v = v + beta * po[u];
+            ee[pos] = ev[u] + ax * po[u];
+          }
+          pout[pos] = v;
+          mp = maxloc_pick(mp, MaxLoc{(double)v, k * L.NRC + l});
+        }
       }
     }
-    mp = bmax(mp, mlds);
+    mp = call_max<MF6_BLOCK>(mp, mlds);
     if (threadIdx.x == 0) mpart[M_P * T + tile] = mp;
   }
 }
@@ -382,66 +392,67 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_spmv(const BSys *sys, const Tile
                                                      const float *p0, const float *p1, float *q,
                                                      double *part, int T, const KState *st,
                                                      const BFState *fs) {
-  __shared__ double lds[8];
+  __shared__ double lds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int s = tiles[tile].sys;
-    if (st[s].stop) continue;
+    const int s = tiles[tile].sys, base = tiles[tile].base;
     const Layout L = sys[s].L;
     const long long vo = sys[s].voff;
-    const float *A = A32 + sys[s].aoff;
-    const float *p = (fs[s].pcur ? p0 : p1) + vo;   // the direction just formed
-    float *qq = q + vo;
-    const int NP = L.NP;
+    const float *__restrict__ A = A32 + sys[s].aoff;
+    const float *__restrict__ p = (fs[s].pcur ? p0 : p1) + vo;   // the direction just formed
+    float *__restrict__ qq = q + vo;
+    const int NP = L.NP, HP = L.HP;
+    if (st[s].stop) continue;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     double sum = 0.0;
     for (int c = 0; c < cpt; c++) {
-      const int t = tiles[tile].base + c * blockDim.x + threadIdx.x;
+      const int t = base + c * MF6_BLOCK + threadIdx.x;
       const int cc = t & 1, h2 = t >> 1;
       if (h2 >= ncols_of(L, cc)) continue;
-      const int l = col_l(L, cc, h2);
-      const int i = l / L.ncol, j = l - i * L.ncol;
-      // off-grid neighbours read position 0 (in range); a select drops
-      // their term, so no lane waits inside a branch
-      const bool hb = i > 0, hl = j > 0, hr = j < L.ncol - 1, hf = i < L.nrow - 1;
-      const int ib = hb ? hn(l, -L.ncol) : 0;
-      const int il = hl ? hn(l, -1) : 0;
-      const int ir = hr ? hn(l, 1) : 0;
-      const int ifr = hf ? hn(l, L.ncol) : 0;
+      const CGeo G(L, cc, h2);
       const int own = cc * L.H + h2;
       const int oth = (1 - cc) * L.H;
-      float pprev = 0.f, pcur = p[own], aup = 0.f;
-      for (int k = 0; k < L.nlay; k++) {
-        const int pos = own + k * L.HP;
-        const int ob = oth + k * L.HP;
-        const float pnext = (k + 1 < L.nlay) ? p[pos + L.HP] : 0.f;
-        const float adn = A[6 * NP + pos];
-        float tq = 0.f;
-        tq = tq + A[pos] * pcur;
-        if (k > 0) tq = tq + aup * pprev;
-        {
-          const auto t_ = A[5 * NP + ob + ib] * p[ob + ib];
-          tq = hb ? tq + t_ : tq;
+      float pprev = 0.f, aup = 0.f;
+      for (int k0 = 0; k0 < L.nlay; k0 += C_CH) {
+        float po[C_CH + 1], a0[C_CH], a6[C_CH], ab[C_CH], al[C_CH], ar[C_CH], af[C_CH], pb[C_CH],
+            pl[C_CH], pr[C_CH], pf[C_CH];
+#pragma unroll
+        for (int u = 0; u < C_CH + 1; u++)
+          po[u] = p[own + (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * HP];
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
+          const int pos = own + k * HP, ob = oth + k * HP;
+          a0[u] = A[pos];
+          a6[u] = A[6 * NP + pos];
+          ab[u] = A[5 * NP + ob + G.ib];
+          pb[u] = p[ob + G.ib];
+          al[u] = A[4 * NP + ob + G.il];
+          pl[u] = p[ob + G.il];
+          ar[u] = A[4 * NP + pos];
+          pr[u] = p[ob + G.ir];
+          af[u] = A[5 * NP + pos];
+          pf[u] = p[ob + G.ifr];
         }
-        {
-          const auto t_ = A[4 * NP + ob + il] * p[ob + il];
-          tq = hl ? tq + t_ : tq;
+#pragma unroll
+        for (int u = 0; u < C_CH; u++) {
+          const int k = k0 + u;
+          if (k >= L.nlay) continue;
+          float tq = 0.f;
+          tq = tq + a0[u] * po[u];
+          if (k > 0) tq = tq + aup * pprev;
+          tq = G.hb ? tq + ab[u] * pb[u] : tq;
+          tq = G.hl ? tq + al[u] * pl[u] : tq;
+          tq = G.hr ? tq + ar[u] * pr[u] : tq;
+          tq = G.hf ? tq + af[u] * pf[u] : tq;
+          if (k < L.nlay - 1) tq = tq + a6[u] * po[u + 1];
+          qq[own + k * HP] = tq;
+          sum = sum + (double)po[u] * (double)tq;
+          aup = a6[u];
+          pprev = po[u];
         }
-        {
-          const auto t_ = A[4 * NP + pos] * p[ob + ir];
-          tq = hr ? tq + t_ : tq;
-        }
-        {
-          const auto t_ = A[5 * NP + pos] * p[ob + ifr];
-          tq = hf ? tq + t_ : tq;
-        }
-        if (k < L.nlay - 1) tq = tq + adn * pnext;
-        qq[pos] = tq;
-        sum = sum + (double)pcur * (double)tq;
-        aup = adn;
-        pprev = pcur;
-        pcur = pnext;
       }
     }
-    sum = bsum(sum, lds);
+    sum = call_sum<MF6_BLOCK>(sum, lds);
     if (threadIdx.x == 0) part[P_PQ * T + tile] = sum;
   }
 }
@@ -455,101 +466,98 @@ __device__ inline void testcnvg0(int *icnvg, double dvmax, double rmax, double d
   if (fabs(dvmax) <= dvclose && fabs(rmax) <= rclose) *icnvg = 1;
 }
 
-__device__ inline int is_close_b(double a, double b) {
-  if (a == b) return 1;
-  return fabs(a - b) <= fmax(100.0 * 2.220446049250313080847263336181640625e-16 *
-                                 fmax(fabs(a), fabs(b)), 0.0);
-}
-
 __global__ void __launch_bounds__(MF6_BLOCK) kb_round(const BSys *sys, KState *st, BFState *fs,
                                                       const double *part, const MaxLoc *mpart,
                                                       int T) {
-  __shared__ double lds[8];
-  __shared__ MaxLoc mlds[8];
+  __shared__ double lds[4][4];
+  __shared__ MaxLoc mlds[2][4];
   const int s = blockIdx.x;
-  if (st[s].stop) return;
-  const BSys S = sys[s];
+  const int tr0 = sys[s].tr0, ntr = sys[s].ntr, tb0 = sys[s].tb0, ntb = sys[s].ntb;
+  const int tg0 = sys[s].tg0, ntg = sys[s].ntg;
+  // the state's loads overlap the partials'
+  const KState k = st[s];
+  const double pmax = fs[s].pmax;
+  const int ploc = fs[s].ploc, restart = fs[s].restart;
+  if (k.stop) return;
   double a[4] = {0.0, 0.0, 0.0, 0.0};
   MaxLoc mm[2] = {{0.0, -1}, {0.0, -1}};
-  for (int i = threadIdx.x; i < S.ntr; i += blockDim.x) {
-    a[0] = a[0] + part[P_SS_R * T + S.tr0 + i];
-    a[3] = a[3] + part[P_RHO_R * T + S.tr0 + i];
-    mm[0] = maxloc_pick(mm[0], mpart[M_D_R * T + S.tr0 + i]);
+  for (int i = threadIdx.x; i < ntr; i += MF6_BLOCK) {
+    a[0] = a[0] + part[P_SS_R * T + tr0 + i];
+    a[3] = a[3] + part[P_RHO_R * T + tr0 + i];
+    mm[0] = maxloc_pick(mm[0], mpart[M_D_R * T + tr0 + i]);
   }
-  for (int i = threadIdx.x; i < S.ntb; i += blockDim.x) {
-    a[1] = a[1] + part[P_SS_B * T + S.tb0 + i];
-    a[2] = a[2] + part[P_RHO_B * T + S.tb0 + i];
-    mm[1] = maxloc_pick(mm[1], mpart[M_D_B * T + S.tb0 + i]);
+  for (int i = threadIdx.x; i < ntb; i += MF6_BLOCK) {
+    a[1] = a[1] + part[P_SS_B * T + tb0 + i];
+    a[2] = a[2] + part[P_RHO_B * T + tb0 + i];
+    mm[1] = maxloc_pick(mm[1], mpart[M_D_B * T + tb0 + i]);
   }
   // two-level: rho gains rc.yc (partials of the system's coarse GEMV blocks)
-  for (int i = threadIdx.x; i < S.ntg; i += blockDim.x) a[3] = a[3] + part[P_RHO_C * T + S.tg0 + i];
-  const double ssr = bsum(a[0], lds);
-  const double ssb = bsum(a[1], lds);
-  const double rb = bsum(a[2], lds);
-  const double rr = bsum(a[3], lds);
-  const MaxLoc mdr = bmax(mm[0], mlds);
-  const MaxLoc mdb = bmax(mm[1], mlds);
+  for (int i = threadIdx.x; i < ntg; i += MF6_BLOCK) a[3] = a[3] + part[P_RHO_C * T + tg0 + i];
+  const double ssr = call_sum<MF6_BLOCK>(a[0], lds[0]);
+  const double ssb = call_sum<MF6_BLOCK>(a[1], lds[1]);
+  const double rb = call_sum<MF6_BLOCK>(a[2], lds[2]);
+  const double rr = call_sum<MF6_BLOCK>(a[3], lds[3]);
+  const MaxLoc md = maxloc_pick(call_max<MF6_BLOCK>(mm[0], mlds[0]),
+                                call_max<MF6_BLOCK>(mm[1], mlds[1]));
   if (threadIdx.x != 0) return;
-  KState &k = st[s];
-  BFState &f = fs[s];
-  const MaxLoc md = maxloc_pick(mdr, mdb);
+  KState *o = st + s;
   const double rho_new = rb + rr;
-  const int it = k.iter;
-  f.apend_d = 0.0;
-  if (it > 0) {
-    const double deltax = k.alpha * f.pmax;
-    k.deltax = deltax;
-    k.xloc = f.ploc;
-    k.rmax = md.v;
-    k.rloc = md.loc;
-    k.l2norm = sqrt(ssr + ssb);
+  fs[s].apend_d = 0.0;
+  if (k.iter > 0) {
+    const double deltax = k.alpha * pmax;
+    o->deltax = deltax;
+    o->xloc = ploc;
+    o->rmax = md.v;
+    o->rloc = md.loc;
+    o->l2norm = sqrt(ssr + ssb);
     int icnvg = k.icnvg;
     testcnvg0(&icnvg, deltax, md.v, k.dvclose, k.rclose);
     if (md.v == 0.0) icnvg = 1;
-    k.icnvg = icnvg;
-    if (icnvg != 0) { k.stop = 1; return; }
-    if (is_close_b(k.rho, k.rho0)) { k.stop = 2; return; }
-    if (k.rho == 0.0) { k.stop = 2; return; }
-    k.rho0 = k.rho;
-    if (it >= k.itmax) { k.stop = 3; return; }
+    o->icnvg = icnvg;
+    if (icnvg != 0) { o->stop = 1; return; }
+    if (c_close(k.rho, k.rho0)) { o->stop = 2; return; }
+    if (k.rho == 0.0) { o->stop = 2; return; }
+    o->rho0 = k.rho;
+    if (k.iter >= k.itmax) { o->stop = 3; return; }
+    o->beta = rho_new / k.rho;
   }
-  k.rho = rho_new;
-  if (it > 0) k.beta = rho_new / k.rho0;
-  if (f.restart) {
-    k.beta = 0.0;
-    f.restart = 0;
+  o->rho = rho_new;
+  if (restart) {
+    o->beta = 0.0;
+    fs[s].restart = 0;
   }
 }
 
 __global__ void __launch_bounds__(MF6_BLOCK) kb_alpha(const BSys *sys, KState *st, BFState *fs,
                                                       const double *part, const MaxLoc *mpart,
                                                       int T) {
-  __shared__ double lds[8];
-  __shared__ MaxLoc mlds[8];
+  __shared__ double lds[4];
+  __shared__ MaxLoc mlds[4];
   const int s = blockIdx.x;
-  if (st[s].stop) return;
-  const BSys S = sys[s];
+  const int ti0 = sys[s].ti0, nti = sys[s].nti;
+  const int stop = st[s].stop, iter = st[s].iter, pcur = fs[s].pcur;
+  const double rho = st[s].rho;
+  if (stop) return;
   double a = 0.0;
   MaxLoc mm{0.0, -1};
-  for (int i = threadIdx.x; i < S.nti; i += blockDim.x) {
-    a = a + part[P_PQ * T + S.ti0 + i];
-    mm = maxloc_pick(mm, mpart[M_P * T + S.ti0 + i]);
+  for (int i = threadIdx.x; i < nti; i += MF6_BLOCK) {
+    a = a + part[P_PQ * T + ti0 + i];
+    mm = maxloc_pick(mm, mpart[M_P * T + ti0 + i]);
   }
-  const double pq = bsum(a, lds);
-  const MaxLoc mp = bmax(mm, mlds);
+  const double pq = call_sum<MF6_BLOCK>(a, lds);
+  const MaxLoc mp = call_max<MF6_BLOCK>(mm, mlds);
   if (threadIdx.x != 0) return;
+  const double alpha = rho / (pq + copysign(DPREC_C, pq));
   KState &k = st[s];
   BFState &f = fs[s];
-  double den = pq;
-  den = den + copysign(2.220446049250313080847263336181640625e-16, den);
   k.pq = pq;
-  k.alpha = k.rho / den;
-  k.iter = k.iter + 1;
-  f.apend_x = k.alpha;
-  f.apend_d = k.alpha;
+  k.alpha = alpha;
+  k.iter = iter + 1;
+  f.apend_x = alpha;
+  f.apend_d = alpha;
   f.pmax = mp.v;
   f.ploc = mp.loc;
-  f.pcur = 1 - f.pcur;   // the direction just formed is the current one
+  f.pcur = 1 - pcur;   // the direction just formed is the current one
 }
 
 // ---------------------------------------------------------------------------
@@ -588,7 +596,7 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_residual(const BSys *sys, const 
                                                          const double *x, const double *b,
                                                          float *d32, MaxLoc *mpart, int T,
                                                          const int *active) {
-  __shared__ MaxLoc mlds[8];
+  __shared__ MaxLoc mlds[4];
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const int s = tiles[tile].sys;
     if (!active[s]) continue;
@@ -597,6 +605,7 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_residual(const BSys *sys, const 
     const double *A = A64 + sys[s].aoff;
     const double *xx = x + vo;
     const int NP = L.NP;
+    if (tile != (int)blockIdx.x) __syncthreads();   // lds is no longer read
     MaxLoc m{0.0, -1};
     for (int c = 0; c < cpt; c++) {
       const int t = tiles[tile].base + c * blockDim.x + threadIdx.x;
@@ -641,7 +650,7 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_residual(const BSys *sys, const 
         m = maxloc_pick(m, MaxLoc{r, k * L.NRC + l});
       }
     }
-    m = bmax(m, mlds);
+    m = call_max<MF6_BLOCK>(m, mlds);
     if (threadIdx.x == 0) mpart[M_TRUE * T + tile] = m;
   }
 }
@@ -650,14 +659,14 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_residual(const BSys *sys, const 
 __global__ void __launch_bounds__(MF6_BLOCK) kb_after(const BSys *sys, BFState *fs,
                                                       const MaxLoc *mpart, int T, double *out,
                                                       const int *active, int restart) {
-  __shared__ MaxLoc mlds[8];
+  __shared__ MaxLoc mlds[4];
   const int s = blockIdx.x;
   if (!active[s]) return;
   const BSys S = sys[s];
   MaxLoc m{0.0, -1};
   for (int i = threadIdx.x; i < S.nti; i += blockDim.x)
     m = maxloc_pick(m, mpart[M_TRUE * T + S.ti0 + i]);
-  m = bmax(m, mlds);
+  m = call_max<MF6_BLOCK>(m, mlds);
   if (threadIdx.x != 0) return;
   fs[s].apend_d = 0.0;
   fs[s].apend_x = 0.0;
@@ -691,7 +700,7 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_tl_gather(const BSys *sys, const
       const int i = ai * Tl.ha + t / Tl.ha, j = aj * Tl.ha + t % Tl.ha;
       if (i < S.L.nrow && j < S.L.ncol) v = v + cs[i * S.L.ncol + j];
     }
-    v = wsum(v);
+    v = csum(v);
     if (ln == 0) rc[S.cvo + I] = v;
   }
 }
@@ -704,7 +713,7 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_tl_gemv(const BSys *sys, const G
                                                         const float *Ainv, float *yc,
                                                         double *part, int T, const KState *st) {
   extern __shared__ double xs[];
-  __shared__ double lds[8];
+  __shared__ double lds[4];
   const int w = threadIdx.x >> 6, ln = threadIdx.x & 63;
   for (int task = blockIdx.x; task < ntasks; task += gridDim.x) {
     const int s = tasks[task].sys;
@@ -725,14 +734,24 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_tl_gemv(const BSys *sys, const G
         s0 = s0 + (double)a.x * xs[c] + (double)a.y * xs[c + 1] + (double)a.z * xs[c + 2] +
              (double)a.w * xs[c + 3];
       }
-      s0 = wsum(s0);
+      s0 = csum(s0);
       if (ln == 0) {
         yc[S.cvo + I] = (float)s0;
         acc = xs[I] * (double)(float)s0;
       }
     }
-    acc = bsum(acc, lds);
+    acc = call_sum<MF6_BLOCK>(acc, lds);
     if (threadIdx.x == 0) part[P_RHO_C * T + task] = acc;
+  }
+}
+
+// heads of one system in natural order; one thread per column
+__global__ void kb_natural(Layout L, const double *__restrict__ x, double *__restrict__ out) {
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < 2 * L.HP0; t += gridDim.x * blockDim.x) {
+    const int c = t & 1, h2 = t >> 1;
+    if (h2 >= ncols_of(L, c)) continue;
+    const int l = col_l(L, c, h2), own = c * L.H + h2;
+    for (int k = 0; k < L.nlay; k++) out[k * L.NRC + l] = x[own + k * L.HP];
   }
 }
 
@@ -753,6 +772,7 @@ struct BatchHandle {
   std::vector<BSys> sys;
   std::vector<mf6hip_ims_settings> set;
   long long ptot = 0, vtot = 0;        // plane / vector lengths
+  int maxlay = 0, maxn = 0;            // most layers and cells of a system
   double *A64 = nullptr, *b64 = nullptr, *x64 = nullptr, *x0 = nullptr, *piv64 = nullptr;
   float *A32 = nullptr, *piv32 = nullptr, *d32 = nullptr, *z32 = nullptr, *zf32 = nullptr,
         *q32 = nullptr, *p0 = nullptr, *p1 = nullptr, *e32 = nullptr;
@@ -775,6 +795,8 @@ struct BatchHandle {
     std::vector<int> grids;
     std::vector<hipGraphExec_t> execs;
   } tsets[2];
+  double *xnat = nullptr;              // one system's heads in natural order
+  std::mutex xmut;
   int *h_act = nullptr;                // pinned: active flags staged to the device
   KState *st = nullptr;
   BFState *fs = nullptr;
@@ -896,9 +918,15 @@ void launch_iteration(BatchHandle *b) {
   kb_red_fwd<<<g, MF6_BLOCK, 0, s>>>(b->dsys, b->dtr, b->ntr, c, b->A32, b->piv32, b->d32, b->q32,
                                      b->zf32, b->part, b->mpart, T, b->st, b->fs);
   double *cs = b->tl ? b->tl_colsum : nullptr;
-  kb_black<<<g, MF6_BLOCK, 0, s>>>(b->dsys, b->dtb, b->ntb, c, b->A32, b->piv32, b->d32, b->q32,
-                                   b->zf32, b->z32, b->part, b->mpart, T, b->st, b->fs,
-                                   b->tl_cmask, cs);
+#define MF6_BB(N)                                                                           \
+  kb_black<N><<<g, MF6_BLOCK, 0, s>>>(b->dsys, b->dtb, b->ntb, c, b->A32, b->piv32, b->d32, \
+                                      b->q32, b->zf32, b->z32, b->part, b->mpart, T, b->st, \
+                                      b->fs, b->tl_cmask, cs)
+  if (b->maxlay <= 4) MF6_BB(4);
+  else if (b->maxlay <= 8) MF6_BB(8);
+  else if (b->maxlay <= 16) MF6_BB(16);
+  else MF6_BB(32);
+#undef MF6_BB
   kb_red_bwd<<<g, MF6_BLOCK, 0, s>>>(b->dsys, b->dtr, b->ntr, c, b->A32, b->piv32, b->d32,
                                      b->zf32, b->z32, b->part, T, b->st, b->tl_cmask, cs);
   if (b->tl) {
@@ -1040,6 +1068,8 @@ extern "C" int mf6hip_batch_add(void *handle, const mf6hip_ims_settings *setting
     if (S.tl.nc > b->maxnc) b->maxnc = S.tl.nc;
     if (S.tl.ld > b->maxld) b->maxld = S.tl.ld;
   }
+  if (S.L.nlay > b->maxlay) b->maxlay = S.L.nlay;
+  if (S.L.N > b->maxn) b->maxn = S.L.N;
   b->ptot += (long long)MF6_NSLOT * S.L.NP;
   b->vtot += S.L.NP;
   b->sys.push_back(S);
@@ -1063,6 +1093,7 @@ extern "C" int mf6hip_batch_finalize(void *handle) {
   BCK(balloc(&b->b64, v));
   BCK(balloc(&b->x64, v));
   BCK(balloc(&b->x0, v));
+  BCK(balloc(&b->xnat, b->maxn));
   BCK(balloc(&b->piv64, v));
   BCK(balloc(&b->piv32, v));
   BCK(balloc(&b->d32, v));
@@ -1291,9 +1322,13 @@ extern "C" int mf6hip_batch_get_x(void *handle, int isys, double *x) {
   if (!b || !b->finalized || !x) { mf6hip_set_error("bad argument"); return MF6HIP_EINVAL; }
   if (isys < 0 || isys >= b->nsys) { mf6hip_set_error("system index out of range"); return MF6HIP_EINVAL; }
   const Layout &L = b->sys[isys].L;
-  std::vector<double> tmp(L.NP);
-  HIPCHK(hipMemcpy(tmp.data(), b->x64 + b->sys[isys].voff, sizeof(double) * L.NP, hipMemcpyDeviceToHost));
-  for (int n = 0; n < L.N; n++) x[n] = tmp[pos_of_natural(L, n)];
+  // into natural order on the device (one buffer: a lock for callers' threads)
+  std::lock_guard<std::mutex> lock(b->xmut);
+  kb_natural<<<(2 * L.HP0 + 255) / 256, 256, 0, b->stream>>>(L, b->x64 + b->sys[isys].voff,
+                                                             b->xnat);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(x, b->xnat, sizeof(double) * L.N, hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipStreamSynchronize(b->stream));
   return MF6HIP_OK;
 }
 
@@ -1302,7 +1337,7 @@ extern "C" int mf6hip_batch_destroy(void *handle) {
   if (!b) return MF6HIP_OK;
   if (b->stream) hipStreamSynchronize(b->stream);
   batch_free_tilesets(b);
-  void *bufs[] = {b->A64, b->b64, b->x64, b->x0, b->piv64, b->A32, b->piv32, b->d32, b->z32, b->zf32,
+  void *bufs[] = {b->A64, b->b64, b->x64, b->x0, b->xnat, b->piv64, b->A32, b->piv32, b->d32, b->z32, b->zf32,
                   b->q32, b->p0, b->p1, b->e32, b->st, b->fs, b->active, b->rtrue, b->dtg, b->tl_cmask,
                   b->tl_colsum, b->tl_rc, b->tl_yc, b->tl_A32, b->tl_S3, b->tl_Fi, b->tl_Gi,
                   b->tl_Xd, b->tl_dinfo};
