@@ -156,14 +156,6 @@ __global__ void k_tl_expand(TwoLevel T, const double *__restrict__ S3, double *_
   }
 }
 
-// lane `lane`'s value in every lane (two 32-bit readlanes; lane is uniform)
-__device__ inline double readlane64(double v, int lane) {
-  const unsigned long long u = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, lane);
-  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), lane);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 // ---------------------------------------------------------------------------
 // Inverse of S for aggregate grids at most 63 wide.  With the aggregate rows
 // as blocks of b = naj unknowns S is block tridiagonal: D_i (tridiagonal) on
@@ -181,7 +173,7 @@ __device__ inline double readlane64(double v, int lane) {
 // factorisation and substitutions that this replaces (one workgroup, then one
 // wavefront per column of X, each nai b steps long) took 3.45 + 2.35 ms at
 // 63 x 63 aggregates and 0.77 + 0.42 ms at 28 x 37; the four kernels here take
-// 1.65 and 0.53 ms.
+// 1.05 and 0.34 ms.
 // ---------------------------------------------------------------------------
 
 constexpr int TL_B = 64;   // padded block
@@ -204,114 +196,177 @@ __global__ void k_tl_scale(TwoLevel T, const double *__restrict__ S3, double *__
   }
 }
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+
 // In-place Gauss-Jordan inverse of a b x b symmetric positive definite block
-// with diagonal below 4, held by four waves, row 16 wave + q in a[q], column =
-// lane (identity beyond b).  Pivot k needs row k (published in rowbuf by its
-// owner; two rows in turn, so one barrier a pivot) and column k, which by
-// symmetry is row k again: a(i, k) = a(k, i) for rows still to come and -a(k,
-// i) for rows done.  With r(j) = a(k, j) / p, a(i, j) -= a(i, k) r(j); column k
-// becomes -a(i, k) / p by the same operation with r(k) = 1 + 1 / p (1 / p is
-// at least 1/4, so the sum loses no digits that matter).  The row of the next
-// pivot is updated and published first, so its way through LDS overlaps the
-// other rows' update.   Returns 1 + the first pivot that is not
-// positive (0: none); such a pivot is taken as 1.
-__device__ inline int tl_invert(double (&a)[16], int b, double (*rowbuf)[TL_B]) {
+// (identity beyond b) in four waves, four pivots a step on the FP64 matrix
+// cores.  Wave w holds rows 16 w .., tile t columns 16 t .., in the layout of
+// the matrix results: row 4 e + lane / 16 and column lane % 16 in a[t][e].
+// With K the first pivot of a step, P its 4 x 4 block and rows K .. K + 3
+// published in rowbuf by their owner (two in turn, one barrier a step):
+//   X = rows K .. K + 3 with the identity in the pivot columns   (4 x 64)
+//   a(i, :) -= a(i, K ..) P^-1 X, the pivot columns of a taken as zero
+//   a(K .., :) = P^-1 X.
+// A lane's row value is its operand B as it stands, and by symmetry (a(i, k) =
+// a(k, i) for rows still to come, -a(k, i) for rows done) the first element
+// of P^-1 times it is its operand A of the update.  P^-1 comes from the LDL^T
+// factors of P, which every lane computes, and the solve for the lane's own
+// column of the identity.  The owner forms its rows P^-1 X after the next
+// pivots are published, beside the next step's factors.  Returns 1 + the first
+// pivot that is not positive (0: none); such a pivot is taken as 1.
+//
+// One pivot at a time (a row through LDS, 16 multiply-adds a lane and a
+// barrier) took 0.39 us a pivot, a step here 0.85 us.
+__device__ inline int tl_invert(d4 (&a)[4], int b, double (*rowbuf)[4][TL_B]) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, k4 = lane >> 4;
   int first = 0;
   __syncthreads();
-  if (wv == 0) rowbuf[0][lane] = a[0];
-  __syncthreads();
-  // one pivot: kk (its row in the owning wave) is a compile-time constant
-  auto pivot = [&](auto KK, int kw) {
-    constexpr int kk = decltype(KK)::value, nq = (kk + 1) & 15;
-    const int k = 16 * kw + kk;
-    const double x = rowbuf[k & 1][lane];
-    double p = readlane64(x, k);
-    if (!(p > 0.0)) {
-      if (first == 0) first = k + 1;
-      p = 1.0;
-    }
-    // 1 / p: the hardware's estimate and two Newton steps
-    double ip = __builtin_amdgcn_rcp(p);
-    ip = fma(fma(-p, ip, 1.0), ip, ip);
-    ip = fma(fma(-p, ip, 1.0), ip, ip);
-    const double r = lane == k ? 1.0 + ip : x * ip;
-    const double rs = wv < kw ? r : -r;   // rows done take the other sign
-    const bool own = wv == kw, nown = wv == (kk < 15 ? kw : kw + 1);
-    auto upd = [&](int q) {
-      const double f = readlane64(x, 16 * wv + q);
-      a[q] = fma(f, own && q < kk ? r : rs, a[q]);
-    };
-    upd(nq);
-    if (nown) rowbuf[(k + 1) & 1][lane] = a[nq];
+  if (wv == 0)
 #pragma unroll
-    for (int q = 0; q < 16; q++)
-      if (q != nq && q != kk) upd(q);
-    if (own) a[kk] = lane == k ? ip : r;
-    else upd(kk);
+    for (int t = 0; t < 4; t++) rowbuf[0][t][lane] = a[t][0];
+  __syncthreads();
+  auto step = [&](auto KK) {
+    constexpr int K = decltype(KK)::value, tk = K / 16, ek = (K / 4) & 3;
+    const double(*buf)[TL_B] = rowbuf[(K / 4) & 1];
+    double x[4], P[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = i; j < 4; j++) P[i][j] = buf[tk][16 * i + 4 * ek + j];
+#pragma unroll
+    for (int t = 0; t < 4; t++) x[t] = buf[t][lane];
+    const double xw = buf[wv][lane];
+    // P = L D L^T: L in the lower part of P, the reciprocals of D in id
+    double id[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      double p = P[k][k];
+      const bool bad = !(p > 0.0);
+      first = bad && first == 0 ? K + k + 1 : first;
+      p = bad ? 1.0 : p;
+      // 1 / p: the hardware's estimate and two Newton steps
+      double ip = __builtin_amdgcn_rcp(p);
+      ip = fma(fma(-p, ip, 1.0), ip, ip);
+      ip = fma(fma(-p, ip, 1.0), ip, ip);
+      id[k] = ip;
+#pragma unroll
+      for (int i = k + 1; i < 4; i++) P[i][k] = P[k][i] * ip;
+#pragma unroll
+      for (int i = k + 1; i < 4; i++)
+#pragma unroll
+        for (int j = i; j < 4; j++) P[i][j] = fma(-P[i][k], P[k][j], P[i][j]);
+    }
+    // column k4 of P^-1
+    double y[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      y[i] = k4 == i ? 1.0 : 0.0;
+#pragma unroll
+      for (int j = 0; j < i; j++) y[i] = fma(-P[i][j], y[j], y[i]);
+    }
+#pragma unroll
+    for (int i = 3; i >= 0; i--) {
+      y[i] = y[i] * id[i];
+#pragma unroll
+      for (int j = i + 1; j < 4; j++) y[i] = fma(-P[j][i], y[j], y[i]);
+    }
+    const double pa = c16 == 0 ? y[0] : c16 == 1 ? y[1] : c16 == 2 ? y[2] : c16 == 3 ? y[3] : 0.0;
+    const bool pc = (c16 >> 2) == ek;   // a pivot column of tile tk
+    const d4 zero = {0.0, 0.0, 0.0, 0.0};
+    const double w = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, xw, zero, 0, 0, 0)[0];
+    const double f = 16 * wv + c16 < K ? w : -w;
+    x[tk] = pc ? (k4 == (c16 & 3) ? 1.0 : 0.0) : x[tk];
+#pragma unroll
+    for (int e = 0; e < 4; e++) a[tk][e] = pc ? 0.0 : a[tk][e];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+      a[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(f, x[t], a[t], 0, 0, 0);
+    constexpr int K1 = K + 4;
+    if (K1 < TL_B && wv == K1 / 16)
+#pragma unroll
+      for (int t = 0; t < 4; t++) rowbuf[(K1 / 4) & 1][t][lane] = a[t][(K1 / 4) & 3];
     __syncthreads();
+    if (wv == tk)
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        a[t][ek] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, x[t], zero, 0, 0, 0)[0];
   };
-  for (int kw = 0; 16 * kw < b; kw++) {
-    const int left = b - 16 * kw;
-#define MF6_PIV(K) if (K < left) pivot(std::integral_constant<int, K>{}, kw);
-    MF6_PIV(0) MF6_PIV(1) MF6_PIV(2) MF6_PIV(3) MF6_PIV(4) MF6_PIV(5) MF6_PIV(6) MF6_PIV(7)
-    MF6_PIV(8) MF6_PIV(9) MF6_PIV(10) MF6_PIV(11) MF6_PIV(12) MF6_PIV(13) MF6_PIV(14) MF6_PIV(15)
+#define MF6_PIV(K) if (K < b) step(std::integral_constant<int, K>{});
+  MF6_PIV(0) MF6_PIV(4) MF6_PIV(8) MF6_PIV(12) MF6_PIV(16) MF6_PIV(20) MF6_PIV(24) MF6_PIV(28)
+  MF6_PIV(32) MF6_PIV(36) MF6_PIV(40) MF6_PIV(44) MF6_PIV(48) MF6_PIV(52) MF6_PIV(56) MF6_PIV(60)
 #undef MF6_PIV
-  }
   return first;
 }
 
-// entry (r, c) of the padded diagonal block of aggregate row i
-__device__ inline double tl_dentry(const double *__restrict__ S3, int b, int i, int r, int c) {
-  if (r >= b || c >= b) return r == c ? 1.0 : 0.0;
-  if (r == c) return S3[3 * (i * b + r)];
-  if (r == c + 1) return S3[3 * (i * b + r) + 1];
-  if (c == r + 1) return S3[3 * (i * b + c) + 1];
-  return 0.0;
+// column c of the padded diagonal block of aggregate row i: its diagonal and
+// the couplings to c - 1 and c + 1 (no branch: a wave that loads ahead must not
+// wait at one)
+struct TlCol {
+  double d, lo, hi;
+};
+__device__ inline TlCol tl_dcol(const double *__restrict__ S3, int b, int i, int c) {
+  const int I = i * b + (c < b ? c : 0), J = i * b + (c + 1 < b ? c + 1 : 0);
+  const double d = S3[3 * I], lo = S3[3 * I + 1], hi = S3[3 * J + 1];
+  return TlCol{c < b ? d : 1.0, c > 0 && c < b ? lo : 0.0, c + 1 < b ? hi : 0.0};
+}
+__device__ inline double tl_dentry(const TlCol &v, int r, int c) {
+  return r == c ? v.d : r == c - 1 ? v.lo : r == c + 1 ? v.hi : 0.0;
 }
 
 // coupling of aggregate (i, r) to (i - 1, r)
 __device__ inline double tl_eentry(const double *__restrict__ S3, int b, int nai, int i, int r) {
-  return (r < b && i > 0 && i < nai) ? S3[3 * (i * b + r) + 2] : 0.0;
+  const bool in = r < b && i > 0 && i < nai;
+  const double v = S3[in ? 3 * (i * b + r) + 2 : 2];
+  return in ? v : 0.0;
 }
 
 // The two chains: workgroup 0 F_i^-1 for i = 0 .. nai - 1 into Fi, workgroup 1
 // G_i^-1 for i = nai - 1 .. 0 into Gi (blocks of b x b, rows b apart).  Bound
-// by the pivots' dependent latency (nai b of them).  info[0] = 1 + the first
+// by the dependent latency of the steps (nai b / 4 of them): 0.85 ms at 63 x 63,
+// 0.27 at 28 x 37.  info[0] = 1 + the first
 // unknown whose pivot is not positive (in the order of the unknowns), else 0.
 __global__ void __launch_bounds__(256) k_tl_chain(TwoLevel T, const double *__restrict__ S3,
                                                   double *__restrict__ Fi, double *__restrict__ Gi,
                                                   int *info) {
-  __shared__ double rowbuf[2][TL_B];
-  const int lane = threadIdx.x & 63, r0 = 16 * (int)(threadIdx.x >> 6);
+  __shared__ double rowbuf[2][4][TL_B];
+  const int lane = threadIdx.x & 63, c0 = lane & 15;
+  const int r0 = 16 * (int)(threadIdx.x >> 6) + (lane >> 4);
   const int b = T.naj, n = T.nai, down = blockIdx.x == 0;
   double *out = down ? Fi : Gi;
-  double a[16], dn[16], en[16], ec;
+  d4 a[4];
+  TlCol dn[4];
+  double en[4], ec[4];
   int first = 0;
   // the next block's entries are loaded while this one is inverted
   auto load = [&](int s) {
     const int i = down ? s : n - 1 - s, e = down ? i : i + 1;
-    ec = tl_eentry(S3, b, n, e, lane);
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      dn[q] = tl_dentry(S3, b, i, r0 + q, lane);
-      en[q] = tl_eentry(S3, b, n, e, r0 + q);
+    for (int t = 0; t < 4; t++) {
+      ec[t] = tl_eentry(S3, b, n, e, 16 * t + c0);
+      en[t] = tl_eentry(S3, b, n, e, r0 + 4 * t);
+      dn[t] = tl_dcol(S3, b, i, 16 * t + c0);
     }
   };
   load(0);
 #pragma unroll
-  for (int q = 0; q < 16; q++) a[q] = 0.0;
+  for (int t = 0; t < 4; t++) a[t] = d4{0.0, 0.0, 0.0, 0.0};
   for (int s = 0; s < n; s++) {
     const int i = down ? s : n - 1 - s;
 #pragma unroll
-    for (int q = 0; q < 16; q++) a[q] = fma(-en[q] * ec, a[q], dn[q]);
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        a[t][q] = fma(-en[q] * ec[t], a[t][q], tl_dentry(dn[t], r0 + 4 * q, 16 * t + c0));
     if (s + 1 < n) load(s + 1);
     const int bd = tl_invert(a, b, rowbuf);
     if (bd && !first) first = i * b + bd;
     double *o = out + (size_t)i * b * b;
 #pragma unroll
-    for (int q = 0; q < 16; q++)
-      if (r0 + q < b && lane < b) o[(r0 + q) * b + lane] = a[q];
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (r0 + 4 * q < b && 16 * t + c0 < b) o[(r0 + 4 * q) * b + 16 * t + c0] = a[t][q];
   }
   if (down && threadIdx.x == 0) info[0] = first;
 }
@@ -321,25 +376,34 @@ __global__ void __launch_bounds__(256) k_tl_diag(TwoLevel T, const double *__res
                                                  const double *__restrict__ Fi,
                                                  const double *__restrict__ Gi,
                                                  double *__restrict__ Xd) {
-  __shared__ double rowbuf[2][TL_B];
-  const int lane = threadIdx.x & 63, r0 = 16 * (int)(threadIdx.x >> 6);
+  __shared__ double rowbuf[2][4][TL_B];
+  const int lane = threadIdx.x & 63, c0 = lane & 15;
+  const int r0 = 16 * (int)(threadIdx.x >> 6) + (lane >> 4);
   const int b = T.naj, n = T.nai, i = blockIdx.x;
-  const double ecu = tl_eentry(S3, b, n, i, lane), ecd = tl_eentry(S3, b, n, i + 1, lane);
-  double a[16];
+  d4 a[4];
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int r = r0 + q;
-    const bool in = r < b && lane < b;
-    const double f = in && i > 0 ? Fi[(size_t)(i - 1) * b * b + r * b + lane] : 0.0;
-    const double g = in && i + 1 < n ? Gi[(size_t)(i + 1) * b * b + r * b + lane] : 0.0;
-    double v = tl_dentry(S3, b, i, r, lane);
-    v = fma(-tl_eentry(S3, b, n, i, r) * ecu, f, v);
-    a[q] = fma(-tl_eentry(S3, b, n, i + 1, r) * ecd, g, v);
+  for (int t = 0; t < 4; t++) {
+    const int c = 16 * t + c0;
+    const TlCol dc = tl_dcol(S3, b, i, c);
+    const double ecu = tl_eentry(S3, b, n, i, c), ecd = tl_eentry(S3, b, n, i + 1, c);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int r = r0 + 4 * q;
+      const bool in = r < b && c < b;
+      const double f = in && i > 0 ? Fi[(size_t)(i - 1) * b * b + r * b + c] : 0.0;
+      const double g = in && i + 1 < n ? Gi[(size_t)(i + 1) * b * b + r * b + c] : 0.0;
+      double v = tl_dentry(dc, r, c);
+      v = fma(-tl_eentry(S3, b, n, i, r) * ecu, f, v);
+      a[t][q] = fma(-tl_eentry(S3, b, n, i + 1, r) * ecd, g, v);
+    }
   }
   (void)tl_invert(a, b, rowbuf);
 #pragma unroll
-  for (int q = 0; q < 16; q++)
-    if (r0 + q < b && lane < b) Xd[(size_t)i * b * b + (r0 + q) * b + lane] = a[q];
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (r0 + 4 * q < b && 16 * t + c0 < b)
+        Xd[(size_t)i * b * b + (r0 + 4 * q) * b + 16 * t + c0] = a[t][q];
 }
 
 // 16 columns of X below (blockIdx.z = 0, with the diagonal block) or above
@@ -349,7 +413,6 @@ __global__ void __launch_bounds__(256) k_tl_diag(TwoLevel T, const double *__res
 // l % 16, k = l / 16) from the symmetric inverse read by columns, operand B
 // (k = l / 16, column l % 16) from LDS, result rows 4 e + l / 16.  The next
 // inverse is loaded while the product runs.
-typedef double d4 __attribute__((ext_vector_type(4)));
 template <typename TA>
 __global__ void __launch_bounds__(256) k_tl_prop(TwoLevel T, const double *__restrict__ S3,
                                                  const double *__restrict__ Fi,
