@@ -41,6 +41,26 @@ def test_ensemble_matches_oracle(tune):
         assert np.max(np.abs(h - ho)) < 10 * c.ims.inner_dvclose
 
 
+# the layer bounds of the black sweep (4, 8, 16, 32), whole and partial chunks
+# of four layers, one and two columns per thread
+@pytest.mark.parametrize("nlay_range,pre,tune", [((1, 1), 0, False), ((3, 4), 2, True),
+                                                 ((6, 8), 0, True), ((9, 13), 2, False),
+                                                 ((18, 22), 0, False), ((32, 32), 2, True)])
+def test_ensemble_layer_bounds(nlay_range, pre, tune):
+    cases = [realisation(s, nlay_range=nlay_range, n_range=(13, 41), nwel_range=(0, 4))
+             for s in range(70, 73)]
+    ens = Ensemble(cases, preconditioner=pre)
+    if tune:
+        ens.autotune()
+    icnvg, iters, ms = ens.solve()
+    heads = [ens.heads(i) for i in range(len(cases))]
+    ens.destroy()
+    for c, h, ic in zip(cases, heads, icnvg):
+        ho, icn, ito = oracle_heads(c)
+        assert ic == 1 and icn == 1
+        assert np.max(np.abs(h - ho)) < 10 * c.ims.inner_dvclose
+
+
 def test_ensemble_solve_twice_same_result():
     cases = [realisation(s, nlay_range=(2, 3), n_range=(16, 40), nwel_range=(0, 4))
              for s in range(60, 64)]
