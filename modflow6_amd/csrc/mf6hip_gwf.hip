@@ -461,12 +461,33 @@ struct GncDev {
   double *cond;             // the conductance gnc_fmsav saves
 };
 
-// sln_buildsystem for one model: one thread per row
-__global__ void __launch_bounds__(MF6_BLOCK) k_formulate(GwfDev g, BndDev bd, GncDev G, HfbDev F,
+// Under NEWTON: npf_cf's sat (gwf-npf.f90:444-470) and, for npf_fn, its
+// derivative, once per cell instead of once per row that reads it (seven times;
+// each is a few FP64 divisions)
+__global__ void __launch_bounds__(MF6_BLOCK) k_sat(GwfDev g, const double *__restrict__ x,
+                                                   double *__restrict__ derv) {
+  const Layout &L = g.L;
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < L.NP; p += gridDim.x * blockDim.x) {
+    const int r = p >= L.H ? p - L.H : p;
+    if (r % L.HP >= ncols_of(L, p >= L.H)) continue;
+    const double h = x[p];
+    g.sat[p] = cell_sat(g, p, h);
+    if (g.fn) derv[p] = g.icelltype[p] != 0 ? sqsat_deriv(g.top[p], g.bot[p], h, g.satomega) : 0.0;
+  }
+}
+
+// sln_buildsystem for one model: one thread per row.  The values of the six
+// neighbours that most rows need are loaded together, before the first is used
+// (an absent neighbour reads the cell itself); derv holds k_sat's derivatives.
+// 5x500x500 under NEWTON 170 us (the loads inside each neighbour's branch) -> 108
+// and 15 for k_sat; 10x1000x1000 confined 502 -> 368.  Bound by latency still:
+// three waves a SIMD, and the boundary list's dependent loads.
+__global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd, GncDev G, HfbDev F,
                                                          int iss,
                                                          double delt,
                                                          const double *__restrict__ x,
                                                          const double *__restrict__ xold,
+                                                         const double *__restrict__ derv,
                                                          double *__restrict__ A,
                                                          double *__restrict__ rhs) {
   const Layout &L = g.L;
@@ -475,7 +496,8 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_formulate(GwfDev g, BndDev bd, Gn
     int c, k, i, j, l;
     if (!pos_to_cell(L, p, c, k, i, j, l)) continue;
     const double hcell = x[p];
-    g.sat[p] = cell_sat(g, p, hcell);   // npf_cf (gwf-npf.f90:444-470)
+    // npf_cf (gwf-npf.f90:444-470); under NEWTON k_sat has run
+    if (g.inewton == 0) g.sat[p] = cell_sat(g, p, hcell);
     // neighbour table in ascending natural order: up, back, left, right,
     // front, down.  nb = position, dir = connection plane, lower = pair
     // (nb, n) has nb first
@@ -487,16 +509,38 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_formulate(GwfDev g, BndDev bd, Gn
     pres[3] = j < L.ncol - 1;
     pres[4] = i < L.nrow - 1;
     pres[5] = k < L.nlay - 1;
-    npos[0] = pres[0] ? p - L.HP : -1;
-    npos[5] = pres[5] ? p + L.HP : -1;
+    npos[0] = pres[0] ? p - L.HP : p;
+    npos[5] = pres[5] ? p + L.HP : p;
     {
       const int ob = (1 - c) * L.H + k * L.HP;
-      npos[1] = pres[1] ? ob + hn(l, -L.ncol) : -1;
-      npos[2] = pres[2] ? ob + hn(l, -1) : -1;
-      npos[3] = pres[3] ? ob + hn(l, 1) : -1;
-      npos[4] = pres[4] ? ob + hn(l, L.ncol) : -1;
+      npos[1] = pres[1] ? ob + hn(l, -L.ncol) : p;
+      npos[2] = pres[2] ? ob + hn(l, -1) : p;
+      npos[3] = pres[3] ? ob + hn(l, 1) : p;
+      npos[4] = pres[4] ? ob + hn(l, L.ncol) : p;
     }
     const int dirs[6] = {2, 1, 0, 0, 1, 2};
+    const int ibp = g.ibound[p], ictp = g.icelltype[p];
+    double xm[6], cs[6], sm[6], dm[6], satp = 0.0, dervp = 0.0;
+    int ibm[6], ictm[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+      const int m = npos[s];
+      xm[s] = x[m];
+      cs[s] = g.condsat[dirs[s] * N + (s < 3 ? m : p)];
+      ibm[s] = g.ibound[m];
+      ictm[s] = g.icelltype[m];
+      sm[s] = dm[s] = 0.0;
+    }
+    if (g.inewton != 0) {
+      satp = g.sat[p];
+#pragma unroll
+      for (int s = 0; s < 6; s++) sm[s] = g.sat[npos[s]];
+      if (g.fn) {
+        dervp = derv[p];
+#pragma unroll
+        for (int s = 0; s < 6; s++) dm[s] = derv[npos[s]];
+      }
+    }
     double off[6];
     double diag = 0.0;
     // --- npf_fc
@@ -507,11 +551,19 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_formulate(GwfDev g, BndDev bd, Gn
       int m = npos[s];
       int dir = dirs[s];
       double cond;
-      if (s < 3) {   // m < n: pair (m, n), condsat stored at m
+      // the cases of hcond and vcond that need no more than the values above
+      if (ibp == 0 || ibm[s] == 0) {
+        cond = 0.0;
+      } else if ((ictp == 0 && ictm[s] == 0) || (dir == 2 && g.ivarcv == 0)) {
+        cond = cs[s];
+      } else if (dir != 2 && g.inewton == 1) {
+        const bool upm = s < 3 ? xm[s] > hcell : !(hcell > xm[s]);   // m upstream
+        cond = (upm ? sm[s] : satp) * cs[s];
+      } else if (s < 3) {   // m < n: pair (m, n), condsat stored at m
         int im = i - (s == 1), jm = j - (s == 2);
-        cond = pair_cond(g, dir, m, p, im, jm, x[m], hcell, g.condsat[dir * N + m]);
+        cond = pair_cond(g, dir, m, p, im, jm, xm[s], hcell, cs[s]);
       } else {
-        cond = pair_cond(g, dir, p, m, i, j, hcell, x[m], g.condsat[dir * N + p]);
+        cond = pair_cond(g, dir, p, m, i, j, hcell, xm[s], cs[s]);
       }
       off[s] = off[s] + cond;
       diag = diag + (-cond);
@@ -622,33 +674,26 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_formulate(GwfDev g, BndDev bd, Gn
         if (!pres[s]) continue;
         int dir = dirs[s];
         if (dir == 2 && g.ivarcv == 0) continue;
-        int m = npos[s];
-        int pa, pb_;
-        double csat;
-        if (s < 3) { pa = m; pb_ = p; csat = g.condsat[dir * N + m]; }
-        else { pa = p; pb_ = m; csat = g.condsat[dir * N + p]; }
-        double ha = x[pa], hb = x[pb_];
-        int iups = pb_;
-        if (hb < ha) iups = pa;
-        int idn = (iups == pa) ? pb_ : pa;
-        if (g.icelltype[iups] == 0) continue;
-        double topup = g.top[iups], botup = g.bot[iups];
-        double consterm = -csat * (x[iups] - x[idn]);
-        double derv = sqsat_deriv(topup, botup, x[iups], g.satomega);
-        if (iups == pa) {
-          double term = consterm * derv;
-          if (pa == p) {          // this row is n (upstream)
+        // pair (a, b), a the lower node: this row is b for s < 3
+        const double ha = s < 3 ? xm[s] : hcell, hb = s < 3 ? hcell : xm[s];
+        const bool upa = hb < ha, upm = upa == (s < 3);   // a, m upstream
+        if ((upm ? ictm[s] : ictp) == 0) continue;
+        const double consterm = -cs[s] * (upa ? ha - hb : hb - ha);
+        const double derv_ = upm ? dm[s] : dervp;
+        if (upa) {
+          double term = consterm * derv_;
+          if (s >= 3) {           // this row is n (upstream)
             b = b + term * ha;
             diag = diag + term;
           } else {                // this row is m
             b = b - term * ha;
-            if (g.ibound[p] > 0) off[s] = off[s] + (-term);
+            if (ibp > 0) off[s] = off[s] + (-term);
           }
         } else {
-          double term = -consterm * derv;
-          if (pa == p) {          // row n, m upstream
+          double term = -consterm * derv_;
+          if (s >= 3) {           // row n, m upstream
             b = b + term * hb;
-            if (g.ibound[p] > 0) off[s] = off[s] + term;
+            if (ibp > 0) off[s] = off[s] + term;
           } else {                // row m (upstream)
             b = b - term * hb;
             diag = diag + (-term);
@@ -2049,8 +2094,10 @@ extern "C" int mf6hip_gwf_formulate(void *handle, int kiter, int inewton, double
   }
   GwfDev g = make_dev(h);
   g.fn = h->m.inewton && inewton;
+  // z: free between solves
+  if (g.inewton != 0) k_sat<<<ggrid(L.N), MF6_BLOCK, 0, s>>>(g, h->x, h->z);
   k_formulate<<<ggrid(L.N), MF6_BLOCK, 0, s>>>(g, bd, gnc_dev(h), hfb_dev(h), h->iss, h->delt, h->x,
-                                               h->xold, h->A, h->b);
+                                               h->xold, h->z, h->A, h->b);
   HIPCHK(hipGetLastError());
   if (amat_out || rhs_out) CK(mf6hip_copy_system(h, amat_out, rhs_out));
   return MF6HIP_OK;
