@@ -743,6 +743,10 @@ struct UNetHandle {
   UConv conv[MAXCONV];
   size_t wo_off, bo_off, nparam;
   float *p = nullptr, *grad = nullptr, *m = nullptr, *v = nullptr;
+  // forward's and grad's inputs, grad's target as FP32 and BF16: allocated by the
+  // first call that needs them and, like the activations, kept
+  float *dx = nullptr, *dt32 = nullptr;
+  bf16 *dt = nullptr;
   float *part = nullptr;   // split-K and block partials
   size_t part_n = 0;
   // activations (bf16) per level
@@ -952,6 +956,21 @@ static int u_pack(UNetHandle *u) {
   return MF6HIP_OK;
 }
 
+// the input buffers of forward, and of grad (a call that fails leaves none behind)
+static int u_inputs(UNetHandle *u, bool grad) {
+  const size_t V0 = u->g[0].V();
+  auto need = [](auto **p, size_t n) {
+    if (*p) return (int)MF6HIP_OK;
+    const int rc = ualloc(p, n);
+    if (rc) *p = nullptr;
+    return rc;
+  };
+  UCK(need(&u->dx, V0 * u->nin));
+  if (grad) UCK(need(&u->dt32, V0));
+  if (grad) UCK(need(&u->dt, V0));
+  return MF6HIP_OK;
+}
+
 // forward from the padded level-0 input u->in0 to u->y
 static int u_forward(UNetHandle *u) {
   hipStream_t s = u->stream;
@@ -1040,7 +1059,8 @@ static int u_adam(UNetHandle *u, float lr, float gscale) {
 static void u_free(UNetHandle *u) {
   if (!u) return;
   if (u->stream) hipStreamSynchronize(u->stream);
-  void *bufs[] = {u->p, u->grad, u->m, u->v, u->part, u->in0, u->y, u->lossv, u->data};
+  void *bufs[] = {u->p, u->grad, u->m, u->v, u->part, u->in0, u->y, u->lossv, u->data,
+                  u->dx, u->dt32, u->dt};
   for (void *b : bufs)
     if (b) hipFree(b);
   for (int l = 0; l < MAXLEV; l++) {
@@ -1204,15 +1224,14 @@ extern "C" int mf6hip_unet_forward(void *handle, const float *x, float *y) {
   UNetHandle *u = (UNetHandle *)handle;
   if (!u || !x || !y) { mf6hip_set_error("null argument"); return MF6HIP_EINVAL; }
   const int V0 = u->g[0].V();
-  float *dx = nullptr;
-  UCK(ualloc(&dx, (size_t)V0 * u->nin));
+  UCK(u_inputs(u, false));
+  float *dx = u->dx;
   int rc = MF6HIP_OK;
   if (hipMemcpyAsync(dx, x, sizeof(float) * V0 * u->nin, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (!rc) k_make_input<<<nblk(V0), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0);
   if (!rc) rc = u_forward(u);
   if (!rc && hipMemcpyAsync(y, u->y, sizeof(float) * V0, hipMemcpyDeviceToHost, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (hipStreamSynchronize(u->stream) != hipSuccess && !rc) rc = MF6HIP_EHIP;
-  hipFree(dx);
   if (rc == MF6HIP_EHIP) mf6hip_set_error("unet forward failed");
   return rc;
 }
@@ -1223,15 +1242,15 @@ extern "C" int mf6hip_unet_grad(void *handle, const float *x, const float *t, fl
   UNetHandle *u = (UNetHandle *)handle;
   if (!u || !x || !t || !loss || !grad) { mf6hip_set_error("null argument"); return MF6HIP_EINVAL; }
   const int V0 = u->g[0].V();
-  float *dx = nullptr;
-  bf16 *dt = nullptr;
-  UCK(ualloc(&dx, (size_t)V0 * (u->nin + 1)));
-  int rc = ualloc(&dt, (size_t)V0);
+  UCK(u_inputs(u, true));
+  float *dx = u->dx;
+  bf16 *dt = u->dt;
+  int rc = MF6HIP_OK;
   if (!rc && hipMemcpyAsync(dx, x, sizeof(float) * V0 * u->nin, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
-  if (!rc && hipMemcpyAsync(dx + (size_t)V0 * u->nin, t, sizeof(float) * V0, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
+  if (!rc && hipMemcpyAsync(u->dt32, t, sizeof(float) * V0, hipMemcpyHostToDevice, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (!rc) {
     k_make_input<<<nblk(V0), 256, 0, u->stream>>>(V0, u->nin, dx, u->in0);
-    k_f32_to_bf16<<<nblk(V0), 256, 0, u->stream>>>(V0, dx + (size_t)V0 * u->nin, dt);
+    k_f32_to_bf16<<<nblk(V0), 256, 0, u->stream>>>(V0, u->dt32, dt);
     rc = u_forward(u);
   }
   if (!rc) rc = u_backward(u, dt, 1, 0, 0);
@@ -1240,8 +1259,6 @@ extern "C" int mf6hip_unet_grad(void *handle, const float *x, const float *t, fl
   if (!rc && hipMemcpyAsync(grad, u->grad, sizeof(float) * u->nparam, hipMemcpyDeviceToHost, u->stream) != hipSuccess) rc = MF6HIP_EHIP;
   if (hipStreamSynchronize(u->stream) != hipSuccess && !rc) rc = MF6HIP_EHIP;
   *loss = lv[0];
-  hipFree(dx);
-  if (dt) hipFree(dt);
   if (rc == MF6HIP_EHIP) mf6hip_set_error("unet grad failed");
   return rc;
 }
