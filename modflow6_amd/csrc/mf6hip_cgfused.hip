@@ -899,15 +899,44 @@ static inline int col_group(const Layout &L) {
   return 0;
 }
 
+// Threads of a block of the column kernels: 64 where blocks of 64 hold both
+// colours in at most F_SMALL blocks, else 256.  Few blocks of 256 leave CUs idle and
+// others with four times the waves.  us per iteration of the deflated solve, 256
+// -> 64 threads: FP64 3x64x64 (64 blocks of 64) 50.4 -> 43.0, 10x300x300 (703) 101.0
+// -> 92.4, 7x251x333 (1306) 85.1 -> 82.0, 5x500x500 (1953) 92.9 -> 92.3, 10x700x700
+// (3828) 263 -> 266; FP16 factor 3x64x64 55.2 -> 48.1, 10x300x300 91.2 -> 84.9,
+// 5x501x499 (3907) 79.0 -> 81.2.
+constexpr int F_SMALL = 1536;
+
+// columns, or groups of them, of both colours
+template <typename TV>
+static inline int f_threads(const Layout &L) {
+  const int w = col_group<TV>(L);
+  return w ? 2 * (L.HP / w) : 2 * L.HP0;
+}
+template <typename TV>
+static inline int f_bs(const Layout &L) {
+  return (f_threads<TV>(L) + 63) / 64 <= F_SMALL ? 64 : MF6_BLOCK;
+}
+static inline int f_blocks(int n, int bs) {
+  const int g = (n + bs - 1) / bs;
+  return g > MF6_MAXBLK ? MF6_MAXBLK : (g < 1 ? 1 : g);
+}
+
 // grid of the colour kernels (one thread per group of one colour); k_f_round
 // reduces their partials over this many slots
 template <typename TV>
 static inline int colour_grid(const Layout &L) {
   const int w = col_group<TV>(L);
-  int n = w ? L.HP / w : L.HP0;
-  int g = (n + MF6_BLOCK - 1) / MF6_BLOCK;
-  if (g > MF6_MAXBLK) g = MF6_MAXBLK;
-  return g < 1 ? 1 : g;
+  return f_blocks(w ? L.HP / w : L.HP0, f_bs<TV>(L));
+}
+
+// slots of a partial array: every kernel's blocks of a round
+template <typename TV>
+static inline int f_slots(const Layout &L) {
+  const int a = f_blocks(f_threads<TV>(L), f_bs<TV>(L)), b = f_blocks(2 * L.HP0, MF6_BLOCK);
+  const int c = colour_grid<TV>(L), m = a > b ? a : b;
+  return m > c ? m : c;
 }
 
 template <typename TV, typename TX>
@@ -916,19 +945,18 @@ static void launch_f_pupdate(const Layout &L, int nb, hipStream_t s, const TV *z
                              const FState *fs, const TV *yc = nullptr,
                              const unsigned *cmask = nullptr, TwoLevel T = TwoLevel{}) {
   constexpr int WMAX = 16 / (int)sizeof(TV);
-  const int w = col_group<TV>(L);
+  const int w = col_group<TV>(L), bs = f_bs<TV>(L);
   if (w) {
-    int g = (2 * (L.HP / w) + MF6_BLOCK - 1) / MF6_BLOCK;
+    int g = f_blocks(f_threads<TV>(L), bs);
     if (g > nb) g = nb;
-    if (g < 1) g = 1;
     if (w == WMAX)
-      k_f_pupdatew<TV, TX, WMAX><<<g, MF6_BLOCK, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb,
+      k_f_pupdatew<TV, TX, WMAX><<<g, bs, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb,
                                                          yc, cmask, T);
     else
-      k_f_pupdatew<TV, TX, 2><<<g, MF6_BLOCK, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb, yc,
+      k_f_pupdatew<TV, TX, 2><<<g, bs, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb, yc,
                                                       cmask, T);
   } else {
-    k_f_pupdate<TV, TX><<<nb, MF6_BLOCK, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb, yc,
+    k_f_pupdate<TV, TX><<<nb, bs, 0, s>>>(L, z, pin, pout, x, mpart, st, fs, nb, yc,
                                                  cmask, T);
   }
 }
@@ -1163,37 +1191,37 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_f_spmvw(Layout L, const TV *__res
 #define MF6_SPMV_CH 2
 #endif
 
-// A launch of MF6_BLOCK threads; with e0 / e1 the events are recorded at the
+// A launch of blocks of bs threads; with e0 / e1 the events are recorded at the
 // kernel's own start and end (hipExtLaunchKernelGGL), so their interval is
 // the kernel's execution, as a profiler's kernel trace measures it.
 template <typename... KArgs, typename... Args>
-static void launch_timed(void (*kern)(KArgs...), int grid, hipStream_t s, hipEvent_t e0,
+static void launch_timed(void (*kern)(KArgs...), int grid, int bs, hipStream_t s, hipEvent_t e0,
                          hipEvent_t e1, Args... args) {
   if (e0)
-    hipExtLaunchKernelGGL(kern, dim3(grid), dim3(MF6_BLOCK), 0, s, e0, e1, 0, args...);
+    hipExtLaunchKernelGGL(kern, dim3(grid), dim3(bs), 0, s, e0, e1, 0, args...);
   else
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(MF6_BLOCK), 0, s, args...);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(bs), 0, s, args...);
 }
 
 template <typename TV, int W, bool CS>
 static void launch_f_spmvw(const Layout &L, int nb, hipStream_t s, const TV *A, const TV *p,
                            TV *q, double *part, const KState *st, const unsigned *cmask,
                            double *colsq, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
-  int g = (2 * (L.HP / W) + MF6_BLOCK - 1) / MF6_BLOCK;
+  const int bs = f_bs<TV>(L);
+  int g = f_blocks(f_threads<TV>(L), bs);
   if (g > nb) g = nb;
-  if (g < 1) g = 1;
   constexpr int CH = MF6_SPMV_CH;
   if (L.nlay <= 4)
-    launch_timed(k_f_spmvw<TV, W, 4, CH, CS>, g, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmvw<TV, W, 4, CH, CS>, g, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
   else if (L.nlay <= 8)
-    launch_timed(k_f_spmvw<TV, W, 8, CH, CS>, g, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmvw<TV, W, 8, CH, CS>, g, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
   else if (L.nlay <= 16)
-    launch_timed(k_f_spmvw<TV, W, 16, CH, CS>, g, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmvw<TV, W, 16, CH, CS>, g, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
   else
-    launch_timed(k_f_spmvw<TV, W, 32, CH, CS>, g, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmvw<TV, W, 32, CH, CS>, g, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
 }
 
@@ -1205,7 +1233,7 @@ static void launch_f_spmv_t(const Layout &L, int nb, hipStream_t s, const TM *A,
                             TV *q, double *part, const KState *st, const unsigned *cmask,
                             double *colsq, hipEvent_t e0, hipEvent_t e1) {
   constexpr int WMAX = 16 / (int)sizeof(TV);
-  const int w = col_group<TV>(L);
+  const int w = col_group<TV>(L), bs = f_bs<TV>(L);
   if (w == WMAX) {
     launch_f_spmvw<TV, WMAX, CS>(L, nb, s, A, p, q, part, st, cmask, colsq, e0, e1);
     return;
@@ -1215,14 +1243,14 @@ static void launch_f_spmv_t(const Layout &L, int nb, hipStream_t s, const TM *A,
     return;
   }
   if (L.nlay <= 4)
-    launch_timed(k_f_spmv<TM, TV, 4, CS>, nb, s, e0, e1, L, A, p, q, part, st, nb, cmask, colsq);
+    launch_timed(k_f_spmv<TM, TV, 4, CS>, nb, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask, colsq);
   else if (L.nlay <= 8)
-    launch_timed(k_f_spmv<TM, TV, 8, CS>, nb, s, e0, e1, L, A, p, q, part, st, nb, cmask, colsq);
+    launch_timed(k_f_spmv<TM, TV, 8, CS>, nb, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask, colsq);
   else if (L.nlay <= 16)
-    launch_timed(k_f_spmv<TM, TV, 16, CS>, nb, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmv<TM, TV, 16, CS>, nb, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
   else
-    launch_timed(k_f_spmv<TM, TV, 32, CS>, nb, s, e0, e1, L, A, p, q, part, st, nb, cmask,
+    launch_timed(k_f_spmv<TM, TV, 32, CS>, nb, bs, s, e0, e1, L, A, p, q, part, st, nb, cmask,
                  colsq);
 }
 
@@ -1546,21 +1574,22 @@ static void launch_pc_w(Mf6Handle *h, const TM *A, const TP *piv, TV *d, const T
                         const unsigned *cm, double *cs, const TV *yc, const DeflPlanes &D) {
   const Layout &L = h->L;
   hipStream_t s = h->stream;
+  const int bs = f_bs<TV>(L);
   if (yc) {
-    k_f_red_fwdw<TM, TV, TP, true, W><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_red_fwdw<TM, TV, TP, true, W><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, h->d_part, h->d_mpart, st, fs, nb, yc, D.s, D.ew, D.ns, h->tl);
-    k_f_blackw<TM, TV, TP, true, W><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_blackw<TM, TV, TP, true, W><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, z, h->d_part, h->d_mpart, st, fs, nb, sc, cm, cs, yc, D.s, D.ew,
         D.ns, h->tl);
   } else {
-    k_f_red_fwdw<TM, TV, TP, false, W><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_red_fwdw<TM, TV, TP, false, W><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, h->d_part, h->d_mpart, st, fs, nb, nullptr, nullptr, nullptr,
         nullptr, h->tl);
-    k_f_blackw<TM, TV, TP, false, W><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_blackw<TM, TV, TP, false, W><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, z, h->d_part, h->d_mpart, st, fs, nb, sc, cm, cs, nullptr, nullptr,
         nullptr, nullptr, h->tl);
   }
-  k_f_red_bwdw<TM, TV, TP, W><<<nbc, MF6_BLOCK, 0, s>>>(L, A, piv, d, zf, z, h->d_part, st, nb,
+  k_f_red_bwdw<TM, TV, TP, W><<<nbc, bs, 0, s>>>(L, A, piv, d, zf, z, h->d_part, st, nb,
                                                        sc, cm, cs);
 }
 
@@ -1576,6 +1605,7 @@ static void launch_pc(Mf6Handle *h, const TM *A, const TP *piv, TV *d, const TV 
                       TV *z, KState *st, FState *fs, int nbc, int nb, TV sc = (TV)1) {
   const Layout &L = h->L;
   hipStream_t s = h->stream;
+  const int bs = f_bs<TV>(L);
   const bool tl = h->s.preconditioner >= 2;
   const unsigned *cm = tl ? h->tl_cmask : nullptr;
   double *cs = tl ? h->tl_colsum : nullptr;
@@ -1599,21 +1629,21 @@ static void launch_pc(Mf6Handle *h, const TM *A, const TP *piv, TV *d, const TV 
     return;
   }
   if (yc) {
-    k_f_red_fwd<TM, TV, TP, true><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_red_fwd<TM, TV, TP, true><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, h->d_part, h->d_mpart, st, fs, nb, yc, D.s, D.ew, D.ns, h->tl);
-    k_f_black<TM, TV, TP, true><<<nbc, MF6_BLOCK, 0, s>>>(L, A, piv, d, q, zf, z, h->d_part,
+    k_f_black<TM, TV, TP, true><<<nbc, bs, 0, s>>>(L, A, piv, d, q, zf, z, h->d_part,
                                                           h->d_mpart, st, fs, nb, sc, cm, cs,
                                                           yc, D.s, D.ew, D.ns, h->tl);
   } else {
-    k_f_red_fwd<TM, TV, TP, false><<<nbc, MF6_BLOCK, 0, s>>>(
+    k_f_red_fwd<TM, TV, TP, false><<<nbc, bs, 0, s>>>(
         L, A, piv, d, q, zf, h->d_part, h->d_mpart, st, fs, nb, nullptr, nullptr, nullptr,
         nullptr, h->tl);
-    k_f_black<TM, TV, TP, false><<<nbc, MF6_BLOCK, 0, s>>>(L, A, piv, d, q, zf, z, h->d_part,
+    k_f_black<TM, TV, TP, false><<<nbc, bs, 0, s>>>(L, A, piv, d, q, zf, z, h->d_part,
                                                            h->d_mpart, st, fs, nb, sc, cm, cs,
                                                            nullptr, nullptr, nullptr, nullptr,
                                                            h->tl);
   }
-  k_f_red_bwd<TM, TV, TP><<<nbc, MF6_BLOCK, 0, s>>>(L, A, piv, d, zf, z, h->d_part, st, nb, sc,
+  k_f_red_bwd<TM, TV, TP><<<nbc, bs, 0, s>>>(L, A, piv, d, zf, z, h->d_part, st, nb, sc,
                                                     cm, cs);
 }
 
@@ -1695,8 +1725,7 @@ int mf6hip_run_cg_fused(Mf6Handle *h) {
   // one grid size for every kernel of a round, so that each partial array
   // has the same number of slots for the round kernel to reduce
   const int nbc = colour_grid<double>(L);
-  const int nbs = gridc(2 * L.HP0);
-  const int nb = nbs > nbc ? nbs : nbc;
+  const int nb = f_slots<double>(L);
   double *pbuf[2] = {h->p, h->p2};
   const bool graph = !h->timing && fused64_graph(h, nbc, nb);
   h->h_fold->stop = 0;   // nothing of an earlier solve is still running
@@ -1728,8 +1757,7 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
   KState *st = h->d_state;
   FState *fs = reinterpret_cast<FState *>(h->d_state + 2);
   const int nbc = colour_grid<float>(L);
-  const int nbs = gridc(2 * L.HP0);
-  const int nb = nbs > nbc ? nbs : nbc;
+  const int nb = f_slots<float>(L);
   float *pbuf[2] = {h->p32, h->p232};
   double *rout = h->d_part + 7 * MF6_MAXBLK;
   // iterations between replacements.  With the two-level preconditioner
@@ -1900,8 +1928,7 @@ int mf6hip_fused_op(Mf6Handle *h, int op, const double *x, double *y) {
   const Layout &L = h->L;
   hipStream_t s = h->stream;
   const int nbc = colour_grid<double>(L);
-  const int nbs = gridc(2 * L.HP0);
-  const int nb = nbs > nbc ? nbs : nbc;
+  const int nb = f_slots<double>(L);
   KState *st = h->d_state + 3;
   HIPCHK(hipMemsetAsync(st, 0, sizeof(KState), s));
   if (op == 4) {
@@ -1914,7 +1941,7 @@ int mf6hip_fused_op(Mf6Handle *h, int op, const double *x, double *y) {
     k_op_convert<double, float><<<gridc(MF6_NSLOT * L.NP), MF6_BLOCK, 0, s>>>(
         MF6_NSLOT * L.NP, h->A, h->A32);
     k_op_convert<double, float><<<gridc(L.NP), MF6_BLOCK, 0, s>>>(L.NP, x, h->r32);
-    launch_f_spmv<float, float>(L, nb, s, h->A32, h->r32, h->q32, h->d_part, st);
+    launch_f_spmv<float, float>(L, f_slots<float>(L), s, h->A32, h->r32, h->q32, h->d_part, st);
     k_op_convert<float, double><<<gridc(L.NP), MF6_BLOCK, 0, s>>>(L.NP, h->q32, y);
   } else if (op == 6) {
     if (h->s.preconditioner != 3 || h->s.precision != MF6HIP_FP64 || !h->tl_cmask ||
@@ -1953,8 +1980,7 @@ int mf6hip_fused_op(Mf6Handle *h, int op, const double *x, double *y) {
         return MF6HIP_EINVAL;
       }
       const int nbc32 = colour_grid<float>(L);
-      const int nbs32 = gridc(2 * L.HP0);
-      const int nb32 = nbs32 > nbc32 ? nbs32 : nbc32;
+      const int nb32 = f_slots<float>(L);
       k_op_convert<double, float><<<gridc(L.NP), MF6_BLOCK, 0, s>>>(L.NP, x, h->r32);
       HIPCHK(hipMemsetAsync(h->q32, 0, sizeof(float) * L.NP, s));
       if (h->s.precision == MF6HIP_MIXED) {
