@@ -789,7 +789,7 @@ inline int tl_grid(size_t n) {
 
 // Aggregate width and grid: the smallest ha whose aggregate grid has at most
 // target coarse unknowns and, where that costs at most a doubling of ha, at
-// most 63 aggregates per row (the bandwidth the banded setup handles).  The
+// most 63 aggregates per row (the block that the elimination handles).  The
 // default target, sqrt(2 N) within [16, 4096], keeps the coarse GEMV (nc^2
 // values per iteration) well below the fine iteration's bytes (~24 N).
 TwoLevel mf6hip_tl_shape(const Layout &L, int target) {

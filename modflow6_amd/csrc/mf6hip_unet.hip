@@ -1,7 +1,7 @@
 // mf6hip_unet.hip -- the learned preconditioner network on gfx950: a 4-level
 // 3D U-Net (channels c0..c3, 1x2x2 pooling, nearest 1x2x2 upsampling,
 // concatenated skips, ReLU, 1x1x1 output convolution) with BF16 weights and
-// activations and FP32 accumulation on MFMA (v_mfma_f32_16x16x16_bf16),
+// activations and FP32 accumulation on MFMA (v_mfma_f32_16x16x32_bf16),
 // hand-written forward and backward kernels, and an Adam optimiser.
 //
 // The network has no counterpart in the reference.  Tensors are
