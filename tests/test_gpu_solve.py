@@ -176,6 +176,24 @@ def assert_same_trajectory(ra, rb, n):
         assert ra.locdv[t] == rb.locdv[t] and ra.locr[t] == rb.locr[t]
 
 
+# more columns than the folded kernels take: the fused ones with 64 and 256
+# threads a block, grouped columns (even extents) and single ones
+@pytest.mark.parametrize("shape", [(2, 380, 380), (1, 600, 604), (2, 371, 373), (1, 601, 451)])
+def test_fused_cg_block_sizes_match_unfused(shape):
+    nlay, nrow, ncol = shape
+    case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=3)
+    sim, amat, rhs, x0 = oracle_system(case)
+    out = []
+    for variant in (0, 1):
+        sv = device_solver(case, kernel_variant=variant)
+        x, rec = x0.copy(), ConvergenceRecord(case.ims.inner_maximum)
+        icn, it = sv.solve(1, amat, rhs, x, kstp=1, record=rec)
+        sv.destroy()
+        out.append((it, rec))
+    (ia, ra), (ib, rb) = out
+    assert_same_trajectory(ra, rb, min(20, ia, ib))
+
+
 def test_fused_cg_graph_replay_matches_eager_launches():
     """Without the per-launch timing the fused FP64 CG replays captured
     eight-iteration graphs; with it, it launches every kernel.  The same
