@@ -198,7 +198,7 @@ __global__ void __launch_bounds__(BS, 2) k_b_red(Layout L, const TM *__restrict_
 __device__ inline void b_test(KState *st, BState *bs, int mixed, int par, double *hist, int *hloc,
                               FoldHost *hf) {
   if (bs->stop_seen || !bs->have) return;
-  // this round's rho is in slot par, the tested iteration's in 1 - par; the
+  // the current rho is in slot par, the tested iteration's in 1 - par; the
   // iteration before it left rho0 .. in the state
   const double rho = bs->rho[1 - par], alpha = bs->alpha[1 - par], omega = bs->omega[1 - par];
   const double ss = bs->ss;
