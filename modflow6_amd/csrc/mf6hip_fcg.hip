@@ -56,6 +56,8 @@ struct FcgState {
   int learned;                         // network steps still allowed
   int acc;                             // the last learned step was accepted
   int cand;                            // the IMS test passed: check b - A x
+  int stop;                            // converged: k_g_red's answer, which k_g_bwd copies to
+                                       // KState::stop (no kernel reads the flag that it writes)
   int icnvg, iter, learned_iters, window;
 };
 
@@ -82,6 +84,7 @@ __global__ void k_fcg_init(FcgState *fs, KState *ks, int learned) {
   fs->learned = learned;
   fs->acc = 0;
   fs->cand = 0;
+  fs->stop = 0;
   fs->icnvg = 0;
   fs->iter = 0;
   fs->learned_iters = 0;
@@ -92,16 +95,16 @@ __global__ void k_fcg_init(FcgState *fs, KState *ks, int learned) {
 }
 
 // the true residual decides a candidate: max |b - A x| <= rclose (or a test that
-// ignores the residual); the same answer in every block of BS threads
+// ignores the residual); the same answer in every thread and block of BS threads
 template <int BS>
 __device__ inline bool g_final(const MaxLoc *mpart, int nr, const FcgTest &tst, MaxLoc *mlds) {
   const MaxLoc m = call_max<BS>(cmpart<BS, G_RB / BS>(mpart + GM_T * G_MAXB, nr), mlds);
   return fabs(m.v) <= tst.rclose || tst.icnvgopt == 3;
 }
 
-__device__ inline void g_stop(FcgState *fs, KState *ks, FoldHost *hf) {
+__device__ inline void g_stop(FcgState *fs, const KState *ks, FoldHost *hf) {
   fs->icnvg = 1;
-  ks->stop = 1;
+  fs->stop = 1;
   c_publish(hf, ks, 1);
 }
 
@@ -114,7 +117,7 @@ __device__ inline void g_off(FcgState *fs, FoldHost *hf) {
 
 // the last iteration's candidate, after the last one allowed
 __global__ void __launch_bounds__(64) k_g_last(const MaxLoc *mpart, int nr, FcgTest tst,
-                                               FcgState *fs, KState *ks, FoldHost *hf) {
+                                               FcgState *fs, const KState *ks, FoldHost *hf) {
   if (ks->stop || !fs->cand) return;
   if (g_final<64>(mpart, nr, tst, nullptr) && threadIdx.x == 0) g_stop(fs, ks, hf);
 }
@@ -129,7 +132,7 @@ __global__ void __launch_bounds__(BS, 2) k_g_red(Layout L, const double *__restr
                                                  const double *__restrict__ ay,
                                                  double *__restrict__ zf, const double *part,
                                                  const MaxLoc *mpart, int nq, int nr, FcgTest tst,
-                                                 FcgState *fs, KState *ks, FoldHost *hf) {
+                                                 FcgState *fs, const KState *ks, FoldHost *hf) {
   __shared__ double lds[2][4];
   __shared__ MaxLoc mlds[4];
   const int NP = L.NP, HP = L.HP;
@@ -188,14 +191,15 @@ __global__ void __launch_bounds__(BS, 2) k_g_red(Layout L, const double *__restr
 }
 
 // forward and backward sweep of the black columns; NL bounds the layers at
-// compile time, so that a column's values stay in registers
+// compile time, so that a column's values stay in registers.  fs->stop: set by
+// k_g_red just before, or since an earlier iteration
 template <int BS, bool LEARNED, int NL>
 __global__ void __launch_bounds__(BS, NL <= 16 ? 2 : 1) k_g_black(
     Layout L, const double *__restrict__ A, const double *__restrict__ piv,
     const double *__restrict__ x, const double *__restrict__ ay, const double *__restrict__ zf,
-    double *__restrict__ z, const FcgState *fs, const KState *ks) {
+    double *__restrict__ z, const FcgState *fs) {
   const int NP = L.NP, HP = L.HP;
-  const int stop = ks->stop;
+  const int stop = fs->stop;
   const double w = LEARNED ? fs->w : 0.0;
   const int h = cblock(blockIdx.x, gridDim.x) * BS + threadIdx.x;
   if (h >= L.HP1) return;
@@ -265,9 +269,11 @@ template <int BS>
 __global__ void __launch_bounds__(BS, 2) k_g_bwd(Layout L, const double *__restrict__ A,
                                                  const double *__restrict__ piv,
                                                  const double *__restrict__ zf,
-                                                 double *__restrict__ z, const KState *ks) {
+                                                 double *__restrict__ z, const FcgState *fs,
+                                                 KState *ks) {
   const int NP = L.NP, HP = L.HP;
-  const int stop = ks->stop;
+  const int stop = fs->stop;
+  if (stop && blockIdx.x == 0 && threadIdx.x == 0) ks->stop = 1;
   const int h = cblock(blockIdx.x, gridDim.x) * BS + threadIdx.x;
   if (h >= L.HP0) return;
   const CGeo G(L, 0, h);
@@ -750,13 +756,13 @@ void g_ilu(const Fcg &c, const double *x, const double *ay, double *z) {
   k_g_red<BS, LEARNED><<<c.g.nc, BS, 0, s>>>(L, A, piv, x, ay, h->zf, c.part, h->d_mpart, c.g.nb,
                                              c.nr, c.tst, c.fs, h->d_state, h->h_fold);
 #define MF6_G(N) \
-  k_g_black<BS, LEARNED, N><<<c.g.nc, BS, 0, s>>>(L, A, piv, x, ay, h->zf, z, c.fs, h->d_state)
+  k_g_black<BS, LEARNED, N><<<c.g.nc, BS, 0, s>>>(L, A, piv, x, ay, h->zf, z, c.fs)
   if (L.nlay <= 4) MF6_G(4);
   else if (L.nlay <= 8) MF6_G(8);
   else if (L.nlay <= 16) MF6_G(16);
   else MF6_G(32);
 #undef MF6_G
-  k_g_bwd<BS><<<c.g.nc, BS, 0, s>>>(L, A, piv, h->zf, z, h->d_state);
+  k_g_bwd<BS><<<c.g.nc, BS, 0, s>>>(L, A, piv, h->zf, z, c.fs, h->d_state);
 }
 
 template <int BS, int MODE>
