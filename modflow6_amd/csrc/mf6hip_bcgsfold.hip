@@ -713,6 +713,9 @@ bool mf6hip_bcgs_fold_takes(const Mf6Handle *h) {
 }
 
 int mf6hip_run_bcgs_fold(Mf6Handle *h) {
+  // INNER_MAXIMUM 0: the state stays as initialised.  (An iteration is tested by the
+  // kernels of the next one, so the first would run.)
+  if (h->s.iter1 == 0) return MF6HIP_OK;
   const BVec<double, double, double, double> b{h->A, h->invpiv, h->x, h->d, h->p, h->v, h->q,
                                                h->phat, h->qhat, h->t, h->dhat, h->zf,
                                                h->d_state, 0};

@@ -6,6 +6,8 @@ column red-black permuted matrix the device follows the same Krylov
 trajectory up to dot-product summation order, so iteration counts agree
 within 2 % and heads within 10 x INNER_DVCLOSE; the first iterations
 agree to 1e-9 relative."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -248,6 +250,25 @@ def test_folded_bicgstab_matches_one_pass(shape):
         sv.destroy()
         assert icn == 1
         assert np.max(np.abs(x - xb)) < 10 * case.ims.inner_dvclose
+
+
+@pytest.mark.parametrize("precision", [_lib.MF6HIP_FP64, _lib.MF6HIP_MIXED])
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("most", [0, 1])
+def test_bicgstab_inner_maximum(most, variant, precision):
+    """INNER_MAXIMUM 0 leaves the heads alone (the reference's loop runs from 1
+    to it); 1 takes one iteration."""
+    case = configs.transient_newton(seed=5, nlay=3, nrow=30, ncol=32, nwel=3, nper=1, nstp=2,
+                                    perlen=10.0)
+    case = dataclasses.replace(case, ims=dataclasses.replace(case.ims, inner_maximum=most))
+    sim, amat, rhs, x0 = oracle_system(case)
+    sv = device_solver(case, precision=precision, kernel_variant=variant)
+    for _ in range(2):                      # also after a solve of the same handle
+        x = x0.copy()
+        icn, it = sv.solve(1, amat, rhs, x, kstp=1)
+        assert icn == 0 and it == most
+        assert np.array_equal(x, x0) == (most == 0)
+    sv.destroy()
 
 
 @pytest.mark.parametrize("precision", [_lib.MF6HIP_MIXED, _lib.MF6HIP_MIXED_FP16])
