@@ -64,6 +64,15 @@ enum { BM_X = 0, BM_R = 1 };                                       // maxima
 // squeezed copies sit behind the raw partials
 constexpr size_t B_SQP = 6 * (size_t)MF6_MAXBLK, B_SQM = 3 * (size_t)MF6_MAXBLK;
 
+// Grids of at most B_THIN layers have kernels of their own (THIN) that load the
+// layers which exist; the others load whole chunks of C_CH, clamped to the last
+// layer, so that no branch stands between the loads.  us per iteration, clamped ->
+// own: FP64 1x700x700 109 -> 71, 1x1000x1000 224 -> 126, 2x1000x1000 266 -> 208, FP16
+// factor 1x1000x1000 152 -> 113, 2x1000x1000 174 -> 157.  With three layers or more
+// the branches cost more than the loads: 3x1000x1000 FP16 185 -> 187, 7x300x300 80 ->
+// 87, 32x200x200 142 -> 176.
+constexpr int B_THIN = 2;
+
 template <int BS>
 constexpr int NI_B = BS == 64 ? 512 / 64 : B_RAW / BS;
 
@@ -110,13 +119,14 @@ __global__ void __launch_bounds__(64) k_b_squeeze(double *part, MaxLoc *mpart, i
 // Q false: w = p = d + beta (p - omega v); Q true: w = q = d - alpha v; then the
 // forward sweep of the red columns into zf.  Q false: three more blocks reduce
 // the maxima and d.d of the last iteration for the test.
-template <int BS, bool Q, typename TM, typename TV, typename TP>
+template <int BS, bool Q, bool THIN, typename TM, typename TV, typename TP>
 __global__ void __launch_bounds__(BS, 2) k_b_red(Layout L, const TM *__restrict__ A,
                                                  const TP *__restrict__ piv,
                                                  const TV *__restrict__ d,
                                                  const TV *__restrict__ v, TV *__restrict__ w,
                                                  TV *__restrict__ zf, BPart pt, BState *bs, int nc,
                                                  int par) {
+  constexpr int CH = THIN ? B_THIN : C_CH;
   __shared__ double lds[4];
   __shared__ MaxLoc mlds[4];
   if (!Q && (int)blockIdx.x >= nc) {
@@ -139,12 +149,13 @@ __global__ void __launch_bounds__(BS, 2) k_b_red(Layout L, const TM *__restrict_
   const int h2 = lb * BS + threadIdx.x;
   const bool in = h2 < L.HP0;
   const int h = in ? h2 : 0;
-  TV dv[C_CH], vv[C_CH], wv[C_CH];
-  TM a1[C_CH];
-  TV pv[C_CH];
+  TV dv[CH], vv[CH], wv[CH];
+  TM a1[CH];
+  TV pv[CH];
   auto load = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
+      if (THIN && u > 0 && k0 + u >= L.nlay) break;
       const int p = (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * HP + h;
       dv[u] = d[p];
       vv[u] = v[p];
@@ -175,7 +186,7 @@ __global__ void __launch_bounds__(BS, 2) k_b_red(Layout L, const TM *__restrict_
   for (int k0 = 0; k0 < L.nlay; k0 += C_CH) {
     if (k0) load(k0);
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
       const int k = k0 + u;
       if (k < L.nlay) {
         const int p = k * HP + h;
@@ -259,6 +270,8 @@ __global__ void __launch_bounds__(BS, NL <= 16 ? 2 : 1) k_b_black(
     const TV *__restrict__ v, TV *__restrict__ w, const TV *__restrict__ zf, TV *__restrict__ z,
     KState *st, BState *bs, int nc, int par, int mixed, double *hist, int *hloc,
     FoldHost *hf) {
+  constexpr bool THIN = NL <= B_THIN;
+  constexpr int CH = THIN ? B_THIN : C_CH;
   if (!Q && (int)blockIdx.x == nc) {
     if (threadIdx.x == 0) b_test(st, bs, mixed, par, hist, hloc, hf);
     return;
@@ -276,11 +289,11 @@ __global__ void __launch_bounds__(BS, NL <= 16 ? 2 : 1) k_b_black(
 #pragma unroll
   for (int k0 = 0; k0 < NL; k0 += C_CH) {
     if (k0 >= L.nlay) break;
-    TM a1[C_CH], ab[C_CH], al[C_CH], ar[C_CH], af[C_CH];
-    TV pb[C_CH], zb[C_CH], pl[C_CH], zl[C_CH], pr[C_CH], zr[C_CH], pf[C_CH], zf_[C_CH], dv[C_CH],
-        vv[C_CH], wv[C_CH];
+    TM a1[CH], ab[CH], al[CH], ar[CH], af[CH];
+    TV pb[CH], zb[CH], pl[CH], zl[CH], pr[CH], zr[CH], pf[CH], zf_[CH], dv[CH], vv[CH], wv[CH];
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
+      if (THIN && u > 0 && k0 + u >= L.nlay) break;
       const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
       const int pos = L.H + k * HP + h, rb = k * HP;
       dv[u] = d[pos];
@@ -304,7 +317,7 @@ __global__ void __launch_bounds__(BS, NL <= 16 ? 2 : 1) k_b_black(
     }
     if (stop) return;
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
       const int k = k0 + u;
       if (k < L.nlay) {
         TV x;
@@ -337,11 +350,12 @@ __global__ void __launch_bounds__(BS, NL <= 16 ? 2 : 1) k_b_black(
 }
 
 // backward sweep of the red columns: cell below, then the black neighbours
-template <int BS, bool Q, typename TM, typename TV, typename TP>
+template <int BS, bool Q, bool THIN, typename TM, typename TV, typename TP>
 __global__ void __launch_bounds__(BS, 2) k_b_bwd(Layout L, const TM *__restrict__ A,
                                                  const TP *__restrict__ piv,
                                                  const TV *__restrict__ zf, TV *__restrict__ z,
                                                  BState *bs, int nc) {
+  constexpr int CH = THIN ? B_THIN : C_CH;
   const int lb = cblock(blockIdx.x, nc);
   const int NP = L.NP, HP = L.HP;
   const int stop = bs->stop;
@@ -350,11 +364,12 @@ __global__ void __launch_bounds__(BS, 2) k_b_bwd(Layout L, const TM *__restrict_
   if (h >= L.HP0) return;
   const CGeo G(L, 0, h);
   TV zdn = (TV)0;
-  for (int k0 = L.nlay - 1; k0 >= 0; k0 -= C_CH) {
-    TV zv[C_CH], zb[C_CH], zl[C_CH], zr[C_CH], zq[C_CH], pv[C_CH];
-    TM a6[C_CH], ab[C_CH], al[C_CH], ar[C_CH], af[C_CH];
+  for (int k0 = L.nlay - 1; k0 >= 0; k0 -= CH) {
+    TV zv[CH], zb[CH], zl[CH], zr[CH], zq[CH], pv[CH];
+    TM a6[CH], ab[CH], al[CH], ar[CH], af[CH];
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
+      if (THIN && u > k0) break;
       const int k = k0 - u > 0 ? k0 - u : 0;
       const int pos = k * HP + h, bb = L.H + k * HP;
       zv[u] = zf[pos];
@@ -371,7 +386,7 @@ __global__ void __launch_bounds__(BS, 2) k_b_bwd(Layout L, const TM *__restrict_
     }
     if (stop) return;
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
       const int k = k0 - u;
       if (k >= 0) {
         TV tv = zv[u];
@@ -390,11 +405,12 @@ __global__ void __launch_bounds__(BS, 2) k_b_bwd(Layout L, const TM *__restrict_
 
 // y = A x (amux order); T false: partials of w.y (dhat.v); T true: of y.w and
 // y.y (t.q and t.t).  One thread per column and ny-th of its layers.
-template <int BS, bool T, typename TM, typename TV>
+template <int BS, bool T, bool THIN, typename TM, typename TV>
 __global__ void __launch_bounds__(BS, 2) k_b_mv(Layout L, const TM *__restrict__ A,
                                                 const TV *__restrict__ x, TV *__restrict__ y,
                                                 const TV *__restrict__ w, double *part,
                                                 const BState *bs, int nq, int ny) {
+  constexpr int CH = THIN ? B_THIN : C_CH;
   __shared__ double lds[4], lds2[4];
   const int lb = cblock(blockIdx.x, nq);
   const int NP = L.NP, HP = L.HP;
@@ -410,16 +426,18 @@ __global__ void __launch_bounds__(BS, 2) k_b_mv(Layout L, const TM *__restrict__
     const CGeo G(L, c, h);
     const int own = c * L.H + h, oth = (1 - c) * L.H;
     for (int k0 = ka; k0 < kb; k0 += C_CH) {
-      TV xo[C_CH + 2], xb[C_CH], xl[C_CH], xr[C_CH], xf[C_CH], wv[C_CH];
-      TM a0[C_CH], a1[C_CH], ab[C_CH], al[C_CH], ar[C_CH], af[C_CH], a6[C_CH];
+      TV xo[CH + 2], xb[CH], xl[CH], xr[CH], xf[CH], wv[CH];
+      TM a0[CH], a1[CH], ab[CH], al[CH], ar[CH], af[CH], a6[CH];
 #pragma unroll
-      for (int u = 0; u < C_CH + 2; u++) {
+      for (int u = 0; u < CH + 2; u++) {
+        if (THIN && u > 1 && k0 + u > L.nlay) break;
         int k = k0 + u - 1;
         k = k < 0 ? 0 : (k < L.nlay ? k : L.nlay - 1);
         xo[u] = x[own + k * HP];
       }
 #pragma unroll
-      for (int u = 0; u < C_CH; u++) {
+      for (int u = 0; u < CH; u++) {
+        if (THIN && u > 0 && k0 + u >= L.nlay) break;
         const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
         const int pos = own + k * HP, ob = oth + k * HP;
         a0[u] = A[pos];
@@ -437,7 +455,7 @@ __global__ void __launch_bounds__(BS, 2) k_b_mv(Layout L, const TM *__restrict__
       }
       if (stop) return;
 #pragma unroll
-      for (int u = 0; u < C_CH; u++) {
+      for (int u = 0; u < CH; u++) {
         const int k = k0 + u;
         if (k < L.nlay) {
           TV q = (TV)0;
@@ -466,13 +484,14 @@ __global__ void __launch_bounds__(BS, 2) k_b_mv(Layout L, const TM *__restrict__
 
 // INIT: dhat = d and the partials of dhat.d; else the end of an iteration (see
 // the file's head)
-template <int BS, bool INIT, typename TV, typename TX>
+template <int BS, bool INIT, bool THIN, typename TV, typename TX>
 __global__ void __launch_bounds__(BS) k_b_upd(Layout L, TX *__restrict__ x,
                                               const TV *__restrict__ phat,
                                               const TV *__restrict__ qhat, TV *__restrict__ d,
                                               const TV *__restrict__ q, const TV *__restrict__ t_,
                                               TV *__restrict__ dhat, BPart pt, double *part,
                                               MaxLoc *mpart, BState *bs, int nq, int ny, int par) {
+  constexpr int CH = THIN ? B_THIN : C_CH;
   __shared__ double lds[4][4];
   __shared__ MaxLoc mlds[2][4];
   const int lb = cblock(blockIdx.x, nq);
@@ -490,11 +509,12 @@ __global__ void __launch_bounds__(BS) k_b_upd(Layout L, TX *__restrict__ x,
   const int own = c * L.H + (in ? h2 : 0);
   const int chunks = (L.nlay + C_CH - 1) / C_CH, cy = lb % ny;
   const int ka = chunks * cy / ny * C_CH, kb = chunks * (cy + 1) / ny * C_CH;
-  TV ph[C_CH], qh[C_CH], qv[C_CH], tv_[C_CH], dh[C_CH];
-  TX xv[C_CH];
+  TV ph[CH], qh[CH], qv[CH], tv_[CH], dh[CH];
+  TX xv[CH];
   auto load = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < C_CH; u++) {
+    for (int u = 0; u < CH; u++) {
+      if (THIN && u > 0 && k0 + u >= L.nlay) break;
       const int pos = own + (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * HP;
       if (INIT) {
         dh[u] = d[pos];
@@ -529,7 +549,7 @@ __global__ void __launch_bounds__(BS) k_b_upd(Layout L, TX *__restrict__ x,
     for (int k0 = ka; k0 < kb; k0 += C_CH) {
       if (k0 != ka) load(k0);
 #pragma unroll
-      for (int u = 0; u < C_CH; u++) {
+      for (int u = 0; u < CH; u++) {
         const int k = k0 + u;
         if (k < L.nlay) {
           const int pos = own + k * HP;
@@ -597,6 +617,7 @@ struct BVec {
 
 template <int BS, int NL, typename B>
 void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
+  constexpr bool THIN = NL <= B_THIN;
   const Layout &L = h->L;
   hipStream_t s = h->stream;
   BState *bs = reinterpret_cast<BState *>(h->d_state + 2);
@@ -609,12 +630,12 @@ void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
   };
   for (int r = 0; r < n; r++) {
     const int par = r & 1;
-    k_b_red<BS, false><<<g.nc + 3, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p, b.zf, pt, bs, g.nc,
+    k_b_red<BS, false, THIN><<<g.nc + 3, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p, b.zf, pt, bs, g.nc,
                                                par);
     k_b_black<BS, false, NL><<<g.nc + 1, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p, b.zf, b.phat,
                                                      b.st, bs, g.nc, par, b.mixed, h->d_hist,
                                                      h->d_hloc, h->h_fold);
-    k_b_bwd<BS, false><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.phat, bs, g.nc);
+    k_b_bwd<BS, false, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.phat, bs, g.nc);
     hipEvent_t e1 = nullptr;
     if (h->timing && (h->spmv_calls++ % h->spmv_sample) == 0 &&
         2 * (h->last_spmv_n + 1) <= (int)h->spmv_ev.size()) {
@@ -622,17 +643,17 @@ void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
       (void)hipEventRecord(h->spmv_ev[2 * slot], s);
       e1 = h->spmv_ev[2 * slot + 1];
     }
-    k_b_mv<BS, false><<<g.nq, BS, 0, s>>>(L, b.A, b.phat, b.v, b.dhat, part, bs, g.nq, g.ny);
+    k_b_mv<BS, false, THIN><<<g.nq, BS, 0, s>>>(L, b.A, b.phat, b.v, b.dhat, part, bs, g.nq, g.ny);
     if (e1) (void)hipEventRecord(e1, s);
     squeeze(BP_DV, 1, 0);
-    k_b_red<BS, true><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, pt, bs, g.nc, par);
+    k_b_red<BS, true, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, pt, bs, g.nc, par);
     k_b_black<BS, true, NL><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, b.qhat, b.st,
                                                 bs, g.nc, par, b.mixed, h->d_hist, h->d_hloc,
                                                 h->h_fold);
-    k_b_bwd<BS, true><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.qhat, bs, g.nc);
-    k_b_mv<BS, true><<<g.nq, BS, 0, s>>>(L, b.A, b.qhat, b.t, b.q, part, bs, g.nq, g.ny);
+    k_b_bwd<BS, true, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.qhat, bs, g.nc);
+    k_b_mv<BS, true, THIN><<<g.nq, BS, 0, s>>>(L, b.A, b.qhat, b.t, b.q, part, bs, g.nq, g.ny);
     squeeze(BP_TQ, 2, 0);
-    k_b_upd<BS, false><<<g.nq, BS, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, pt, part,
+    k_b_upd<BS, false, THIN><<<g.nq, BS, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, pt, part,
                                            mpart, bs, g.nq, g.ny, par);
     squeeze(BP_SS, 2, 1);
   }
@@ -644,7 +665,8 @@ template <typename B>
 void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
   const int nl = h->L.nlay;
 #define MF6_B(N) (g.bs == 64 ? enqueue_b<64, N>(h, g, b, n) : enqueue_b<256, N>(h, g, b, n))
-  if (nl <= 4) MF6_B(4);
+  if (nl <= B_THIN) MF6_B(B_THIN);
+  else if (nl <= 4) MF6_B(4);
   else if (nl <= 8) MF6_B(8);
   else if (nl <= 16) MF6_B(16);
   else MF6_B(32);
@@ -684,10 +706,10 @@ int run_b(Mf6Handle *h, const B &b, int si) {
   HIPCHK(hipMemsetAsync(bs, 0, sizeof(BState), s));
   const BPart none{};
   if (g.bs == 64)
-    k_b_upd<64, true><<<g.nq, 64, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, none,
+    k_b_upd<64, true, false><<<g.nq, 64, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, none,
                                           h->d_part, h->d_mpart, bs, g.nq, g.ny, 0);
   else
-    k_b_upd<256, true><<<g.nq, 256, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, none,
+    k_b_upd<256, true, false><<<g.nq, 256, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, none,
                                             h->d_part, h->d_mpart, bs, g.nq, g.ny, 0);
   if (g.squeeze) k_b_squeeze<<<B_SQ, 64, 0, s>>>(h->d_part, h->d_mpart, g.nq, BP_RHO, 1, 0);
   h->h_fold->stop = 0;
