@@ -216,11 +216,13 @@ def test_fcg_without_network_matches_pcg():
 
 # the layer bounds of the sweeps (4, 8, 16, 32) with partial chunks, 64 and 256
 # threads a block, a column or a chunk of it per thread, a single row; more
-# directions than one pass of dot products takes (fcg_m > 8)
+# directions than one pass of dot products takes (fcg_m > 8); more columns than
+# 2048 blocks hold, so that a block walks several groups of them (the last)
 @pytest.mark.parametrize("shape,fcg_m,net", [
     ((1, 1, 64), 8, False), ((3, 33, 17), 12, False), ((5, 24, 21), 8, True),
     ((9, 20, 31), 9, True), ((17, 14, 15), 3, False), ((32, 10, 11), 8, False),
-    ((3, 130, 141), 8, True), ((1, 380, 367), 8, False)])
+    ((3, 130, 141), 8, True), ((1, 380, 367), 8, False), ((2, 40, 37), 8, True),
+    ((1, 730, 730), 3, False)])
 def test_fcg_shapes_match_pcg(shape, fcg_m, net):
     nlay, nrow, ncol = shape
     case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=5 if nrow > 1 else 1)
