@@ -110,7 +110,8 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_red_fwd(const BSys *sys, const T
         float dv[C_CH], qv[C_CH], a6[C_CH], pq[C_CH];
 #pragma unroll
         for (int u = 0; u < C_CH; u++) {
-          const int pos = (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * L.HP + h2;
+          if (u > 0 && k0 + u >= L.nlay) break;
+          const int pos = (k0 + u) * L.HP + h2;
           dv[u] = dd[pos];
           qv[u] = qq[pos];
           a6[u] = A6[pos];
@@ -188,7 +189,8 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_black(const BSys *sys, const Til
         float zb[C_CH], zl[C_CH], zq[C_CH], zw[C_CH], qv[C_CH];
 #pragma unroll
         for (int u = 0; u < C_CH; u++) {
-          const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
+          if (u > 0 && k0 + u >= L.nlay) break;
+          const int k = k0 + u;
           const int pos = L.H + k * HP + h2, rb = k * HP;
           dc[k0 + u] = dd[pos];
           qv[u] = qq[pos];
@@ -286,7 +288,8 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_red_bwd(const BSys *sys, const T
             zq[C_CH], zw[C_CH], pp[C_CH], dv[C_CH];
 #pragma unroll
         for (int u = 0; u < C_CH; u++) {
-          const int k = k0 - u > 0 ? k0 - u : 0;
+          if (u > k0) break;
+          const int k = k0 - u;
           const int pos = k * HP + h2, bb = L.H + k * HP;
           zv[u] = zr[pos];
           a6[u] = A[6 * NP + pos];
@@ -360,7 +363,8 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_pupdate(const BSys *sys, const T
         float zv[C_CH], po[C_CH], ev[C_CH];
 #pragma unroll
         for (int u = 0; u < C_CH; u++) {
-          const int pos = own + (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * L.HP;
+          if (u > 0 && k0 + u >= L.nlay) break;
+          const int pos = own + (k0 + u) * L.HP;
           zv[u] = zz[pos];
           po[u] = pin[pos];
           ev[u] = ee[pos];
@@ -417,10 +421,11 @@ __global__ void __launch_bounds__(MF6_BLOCK) kb_spmv(const BSys *sys, const Tile
             pl[C_CH], pr[C_CH], pf[C_CH];
 #pragma unroll
         for (int u = 0; u < C_CH + 1; u++)
-          po[u] = p[own + (k0 + u < L.nlay ? k0 + u : L.nlay - 1) * HP];
+          if (u == 0 || k0 + u < L.nlay) po[u] = p[own + (k0 + u) * HP];
 #pragma unroll
         for (int u = 0; u < C_CH; u++) {
-          const int k = k0 + u < L.nlay ? k0 + u : L.nlay - 1;
+          if (u > 0 && k0 + u >= L.nlay) break;
+          const int k = k0 + u;
           const int pos = own + k * HP, ob = oth + k * HP;
           a0[u] = A[pos];
           a6[u] = A[6 * NP + pos];
