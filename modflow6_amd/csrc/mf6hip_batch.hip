@@ -76,7 +76,9 @@ enum { M_D_R = 0, M_D_B = 1, M_P = 2, M_TRUE = 3 };
 // the loads of C_CH layers are issued before the first is used.  Eight systems of
 // 64 to 320 columns a side and five layers: 15.6 ms with loops that loaded layer
 // by layer, scalar kernels that reduced through LDS shuffles and heads reordered
-// on the host, 10.3 ms now.
+// on the host, 10.3 ms now.  A chunk loads the layers that exist only (clamped to
+// the last layer instead, four systems of 1x500x500 took 27.3 ms for 24.1, eight of
+// five layers 14.2 for 13.2).
 // ---------------------------------------------------------------------------
 
 __global__ void __launch_bounds__(MF6_BLOCK) kb_red_fwd(const BSys *sys, const Tile *tiles,
@@ -1321,12 +1323,26 @@ extern "C" int mf6hip_batch_solve(void *handle, int *icnvg, int *iters, double *
   return MF6HIP_OK;
 }
 
+// Systems of at most this many cells are put into natural order on the host: a
+// launch costs more than the loop.  us per call, host and device: 2x8x8 14 and 24,
+// 1x33x33 20 and 25, 2x48x48 (4608 cells) 23 and 25, 2x52x52 (5408) 25 and 25, 2x64x64 33
+// and 26, 2x200x200 239 and 52.
+constexpr int BATCH_HOST_X = 5120;
+
 // Heads of one system (natural order, host).
 extern "C" int mf6hip_batch_get_x(void *handle, int isys, double *x) {
   BatchHandle *b = (BatchHandle *)handle;
   if (!b || !b->finalized || !x) { mf6hip_set_error("bad argument"); return MF6HIP_EINVAL; }
   if (isys < 0 || isys >= b->nsys) { mf6hip_set_error("system index out of range"); return MF6HIP_EINVAL; }
   const Layout &L = b->sys[isys].L;
+  if (L.N <= BATCH_HOST_X) {
+    double tmp[BATCH_HOST_X + 32];   // padding: at most one slot a layer
+    // every call that writes x64 waits for its stream before it returns
+    HIPCHK(hipMemcpy(tmp, b->x64 + b->sys[isys].voff, sizeof(double) * L.NP,
+                     hipMemcpyDeviceToHost));
+    for (int n = 0; n < L.N; n++) x[n] = tmp[pos_of_natural(L, n)];
+    return MF6HIP_OK;
+  }
   // into natural order on the device (one buffer: a lock for callers' threads)
   std::lock_guard<std::mutex> lock(b->xmut);
   kb_natural<<<(2 * L.HP0 + 255) / 256, 256, 0, b->stream>>>(L, b->x64 + b->sys[isys].voff,
