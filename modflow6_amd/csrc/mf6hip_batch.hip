@@ -1223,12 +1223,14 @@ extern "C" int mf6hip_batch_autotune(void *handle, char *report, int report_len)
     BCK(build_tiles(b, cpts[ci]));
     for (int gi = 0; gi < 3; gi++) {
       b->grid = gmul[gi] * ncu;
-      HIPCHK(hipMemcpy(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice));
+      HIPCHK(hipMemcpyAsync(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice,
+                            b->stream));
       BCK(reset_states(b));
       BCK(capture(b));
       HIPCHK(hipGraphLaunch(b->gexec, b->stream));   // warm
       HIPCHK(hipStreamSynchronize(b->stream));
-      HIPCHK(hipMemcpy(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice));
+      HIPCHK(hipMemcpyAsync(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice,
+                            b->stream));
       BCK(reset_states(b));
       HIPCHK(hipEventRecord(e0, b->stream));
       HIPCHK(hipGraphLaunch(b->gexec, b->stream));
@@ -1245,7 +1247,9 @@ extern "C" int mf6hip_batch_autotune(void *handle, char *report, int report_len)
   hipEventDestroy(e1);
   b->grid = bg;
   BCK(build_tiles(b, bc));
-  HIPCHK(hipMemcpy(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice));
+  HIPCHK(hipMemcpyAsync(b->x64, xsave, sizeof(double) * b->vtot, hipMemcpyDeviceToDevice,
+                        b->stream));
+  HIPCHK(hipStreamSynchronize(b->stream));   // mf6hip_batch_get_x may follow
   rep += "chosen cpt " + std::to_string(bc) + " grid " + std::to_string(bg);
   if (b->tl) rep += "; coarse setups at staging " + std::to_string(b->tl_setup_ms) + " ms";
   b->tune = rep;

@@ -5,7 +5,7 @@ against the oracle's FP64 ILU0-PCG solve of each realisation: heads within
 import numpy as np
 import pytest
 
-from modflow6_amd.ensemble import Ensemble, realisation
+from modflow6_amd.ensemble import Ensemble, fixed_system, realisation
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -59,6 +59,26 @@ def test_ensemble_layer_bounds(nlay_range, pre, tune):
         ho, icn, ito = oracle_heads(c)
         assert ic == 1 and icn == 1
         assert np.max(np.abs(h - ho)) < 10 * c.ims.inner_dvclose
+
+
+@pytest.mark.parametrize("tune", [False, True])
+def test_ensemble_heads_before_a_solve(tune):
+    """The start heads as staged, in natural order, also after an autotune (which
+    restores them): systems that are reordered on the host and on the device,
+    odd and even extents."""
+    cases = [realisation(s, nlay_range=(nl, nl), n_range=(n, n), nwel_range=(0, 4))
+             for s, (nl, n) in enumerate([(1, 9), (3, 41), (3, 42), (2, 90), (5, 71)])]
+    rng = np.random.default_rng(5)
+    systems = []
+    for c in cases:
+        amat, rhs, x0 = fixed_system(c)
+        systems.append((amat, rhs, rng.standard_normal(x0.size)))
+    ens = Ensemble(cases, preconditioner=2, systems=systems)
+    if tune:
+        ens.autotune()
+    for i, (_, _, x0) in enumerate(systems):
+        assert np.array_equal(ens.heads(i), x0)
+    ens.destroy()
 
 
 def test_ensemble_solve_twice_same_result():
