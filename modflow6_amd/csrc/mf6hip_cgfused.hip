@@ -1818,17 +1818,21 @@ static int run_cg_reliable(Mf6Handle *h, const TMP *Apc, const TP *piv32, float 
   h->h_fold->stop = 0;   // nothing of an earlier solve is still running
   while (!done) {
     // batches of four rounds up to the replacement, one queued ahead of the
-    // one waited for (a round after the stop costs its launches)
+    // one waited for (a round after the stop costs its launches).  A solve's first two
+    // batches are waited for alone, since an outer loop's last solves end there.
     const int due = last_replace + period;
     int ev = 0, stop = 0;
+    int alone = last_replace == 0 ? 2 : 0;
     CK(enqueue(4, 0));
     while (true) {
       const bool more = round < due;
-      if (more) CK(enqueue(4, ev ^ 1));
+      if (more && alone == 0) CK(enqueue(4, ev ^ 1));
       HIPCHK(hipEventSynchronize(h->ev_batch[ev]));
       stop = __atomic_load_n(&h->h_fold->stop, __ATOMIC_ACQUIRE);
       if (stop != 0 || !more) break;
-      ev ^= 1;
+      if (alone > 0) CK(enqueue(4, ev));
+      else ev ^= 1;
+      if (alone > 0) alone--;
     }
     if (stop != 0) h->h_state[0] = h->h_fold->st;
     const KState hs = h->h_state[0];   // read where stop != 0 only
