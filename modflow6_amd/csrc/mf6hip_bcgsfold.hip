@@ -21,7 +21,9 @@
 // Every workgroup of a kernel that needs a scalar adds the partials itself, in
 // the same order (the same bits everywhere); on grids with many partials a
 // squeeze to 256 comes first.  Extra workgroups of k_b_red reduce what the
-// convergence test needs, one of k_b_black runs it.  The arithmetic of every
+// convergence test needs, one of k_b_black runs it; on the largest grids, where the
+// two sweeps before that answer cost more than a launch, k_b_test ends the
+// iteration with it.  The arithmetic of every
 // vector element is that of the one-pass kernels, in the same order.
 //
 // Measured (us per iteration, one-pass -> folded), FP64: 1x100x100 63.5 -> 29.0,
@@ -52,8 +54,8 @@ struct BState {
   double beta;
   int have;        // an iteration was completed (written by k_b_upd)
   int stop;        // the test's result (k_b_black); read from k_b_bwd on
-  int stop_seen;   // its copy (k_b_bwd); read by k_b_red and k_b_black
-  double ss;       // reduced by k_b_red for the test
+  int stop_seen;   // its copy (k_b_bwd, k_b_test); read by k_b_red and k_b_black
+  double ss;       // reduced for the test (k_b_red, k_b_test)
   MaxLoc mx, mr;
 };
 
@@ -586,9 +588,30 @@ __global__ void __launch_bounds__(BS) k_b_upd(Layout L, TX *__restrict__ x,
   }
 }
 
+// the convergence test of iteration r = 2 m + par, at its end (one block)
+__global__ void __launch_bounds__(64) k_b_test(BPart pt, KState *st, BState *bs, int mixed, int par,
+                                               double *hist, int *hloc, FoldHost *hf) {
+  const MaxLoc mx = cmax(cmpart<64, B_SQ / 64>(pt.m + BM_X * pt.ld, B_SQ));
+  const MaxLoc mr = cmax(cmpart<64, B_SQ / 64>(pt.m + BM_R * pt.ld, B_SQ));
+  const double ss = csum(cpart<64, B_SQ / 64>(pt.s + BP_SS * pt.ld, B_SQ));
+  if (threadIdx.x != 0) return;
+  bs->mx = mx;
+  bs->mr = mr;
+  bs->ss = ss;
+  b_test(st, bs, mixed, 1 - par, hist, hloc, hf);
+  bs->stop_seen = bs->stop;
+}
+
+// Positions above which k_b_test runs: its launch takes about 4 us an iteration, the
+// red and black sweeps that otherwise run for nothing at the end of a solve 160 us at
+// 10x1000x1000 (a solve of one iteration 1933 -> 1773 us, of twenty 21.1 -> 21.0 ms) and in
+// proportion to the cells, so that at four million a solve of some twenty iterations
+// breaks even.
+constexpr int B_TEST_NP = 1 << 22;
+
 struct BGrid {
   int bs, nc, ny, nq;   // threads; blocks of one colour; chunks a column; blocks of all
-  bool squeeze;
+  bool squeeze, test;   // test: k_b_test
 };
 
 // 64 threads a block where 512 blocks hold every chunk, else 256; a chunk of
@@ -601,6 +624,7 @@ BGrid b_grid(const Layout &L) {
   g.nc = (L.HP0 + g.bs - 1) / g.bs;
   g.nq = (2 * L.HP0 + g.bs - 1) / g.bs * g.ny;
   g.squeeze = g.nq > B_RAW;
+  g.test = g.squeeze && L.NP > B_TEST_NP;
   return g;
 }
 
@@ -630,11 +654,11 @@ void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
   };
   for (int r = 0; r < n; r++) {
     const int par = r & 1;
-    k_b_red<BS, false, THIN><<<g.nc + 3, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p, b.zf, pt, bs, g.nc,
-                                               par);
-    k_b_black<BS, false, NL><<<g.nc + 1, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p, b.zf, b.phat,
-                                                     b.st, bs, g.nc, par, b.mixed, h->d_hist,
-                                                     h->d_hloc, h->h_fold);
+    k_b_red<BS, false, THIN><<<g.nc + (g.test ? 0 : 3), BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.p,
+                                                                    b.zf, pt, bs, g.nc, par);
+    k_b_black<BS, false, NL><<<g.nc + (g.test ? 0 : 1), BS, 0, s>>>(
+        L, b.A, b.piv, b.d, b.v, b.p, b.zf, b.phat, b.st, bs, g.nc, par, b.mixed, h->d_hist,
+        h->d_hloc, h->h_fold);
     k_b_bwd<BS, false, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.phat, bs, g.nc);
     hipEvent_t e1 = nullptr;
     if (h->timing && (h->spmv_calls++ % h->spmv_sample) == 0 &&
@@ -646,16 +670,19 @@ void enqueue_b(Mf6Handle *h, const BGrid &g, const B &b, int n) {
     k_b_mv<BS, false, THIN><<<g.nq, BS, 0, s>>>(L, b.A, b.phat, b.v, b.dhat, part, bs, g.nq, g.ny);
     if (e1) (void)hipEventRecord(e1, s);
     squeeze(BP_DV, 1, 0);
-    k_b_red<BS, true, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, pt, bs, g.nc, par);
+    k_b_red<BS, true, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, pt, bs, g.nc,
+                                                par);
     k_b_black<BS, true, NL><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.d, b.v, b.q, b.zf, b.qhat, b.st,
                                                 bs, g.nc, par, b.mixed, h->d_hist, h->d_hloc,
                                                 h->h_fold);
     k_b_bwd<BS, true, THIN><<<g.nc, BS, 0, s>>>(L, b.A, b.piv, b.zf, b.qhat, bs, g.nc);
     k_b_mv<BS, true, THIN><<<g.nq, BS, 0, s>>>(L, b.A, b.qhat, b.t, b.q, part, bs, g.nq, g.ny);
     squeeze(BP_TQ, 2, 0);
-    k_b_upd<BS, false, THIN><<<g.nq, BS, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, pt, part,
-                                           mpart, bs, g.nq, g.ny, par);
+    k_b_upd<BS, false, THIN><<<g.nq, BS, 0, s>>>(L, b.x, b.phat, b.qhat, b.d, b.q, b.t, b.dhat, pt,
+                                                 part, mpart, bs, g.nq, g.ny, par);
     squeeze(BP_SS, 2, 1);
+    if (g.test)
+      k_b_test<<<1, 64, 0, s>>>(pt, b.st, bs, b.mixed, par, h->d_hist, h->d_hloc, h->h_fold);
   }
 }
 

@@ -222,11 +222,12 @@ def test_fused_cg_graph_replay_matches_eager_launches():
 
 # the folded BiCGSTAB against the one-pass kernels: layer bounds (2, 4, 8, 16,
 # 32) with partial chunks, 64 and 256 threads, a column or a chunk of it per
-# thread, a single row; the squeeze of the partials (more than 2048 blocks:
-# the last)
+# thread, a single row; the squeeze of the partials (more than 2048 blocks) and,
+# on the last, the test in a kernel of its own
 @pytest.mark.parametrize("shape", [(1, 1, 64), (2, 30, 32), (3, 33, 17), (5, 24, 21), (9, 20, 31),
                                    (17, 14, 15), (32, 10, 11), (3, 130, 141), (4, 300, 240),
-                                   (2, 263, 261), (6, 263, 261), (1, 730, 730)])
+                                   (2, 263, 261), (6, 263, 261), (1, 730, 730),
+                                   (5, 1000, 841)])
 def test_folded_bicgstab_matches_one_pass(shape):
     nlay, nrow, ncol = shape
     case = configs.transient_newton(seed=5, nlay=nlay, nrow=nrow, ncol=ncol, nwel=3, nper=1,
