@@ -212,6 +212,13 @@ struct GwfDev {
   double satomega;
 };
 
+// npf_cf's sat without NEWTON, of values already loaded
+__device__ inline double cell_sat0(int icelltype, int ibound, double top, double bot, double h) {
+  if (icelltype == 0) return 1.0;
+  if (ibound == 0) return 0.0;
+  return h >= top ? 1.0 : (h - bot) / (top - bot);
+}
+
 __device__ inline double cell_sat(const GwfDev &g, int p, double h) {
   // npf_cf: sat of convertible cells; confined cells keep sat = 1
   if (g.icelltype[p] == 0) return 1.0;
@@ -477,11 +484,19 @@ __global__ void __launch_bounds__(MF6_BLOCK) k_sat(GwfDev g, const double *__res
 }
 
 // sln_buildsystem for one model: one thread per row.  The values of the six
-// neighbours that most rows need are loaded together, before the first is used
+// neighbours that the rows need are loaded together, before the first is used
 // (an absent neighbour reads the cell itself); derv holds k_sat's derivatives.
-// 5x500x500 under NEWTON 170 us (the loads inside each neighbour's branch) -> 108
-// and 15 for k_sat; 10x1000x1000 confined 502 -> 368.  Bound by latency still:
-// three waves a SIMD, and the boundary list's dependent loads.
+// Bound by latency: three waves a SIMD, and the boundary list's dependent loads.
+// MODE: what the cells need of their neighbours (one kernel that loaded all of it for
+// every model was slower than the branches for convertible cells without NEWTON and
+// for confined ones under NEWTON).  us of a formulate call, loads inside each neighbour's
+// branch -> this: 10x1000x1000 confined 606 -> 406, convertible 1079 -> 764, NEWTON 1524 ->
+// 757 (k_sat included); 5x500x500 82 -> 62, 128 -> 105, 172 -> 113; 1x1000x1000 82 -> 72,
+// 119 -> 106, 156 -> 118.
+enum { F_CONF = 0,   // every cell is confined: the faces' condsat alone
+       F_CONV = 1,   // convertible cells without NEWTON: tops, bottoms, conductivities
+       F_NEWT = 2 }; // convertible cells under NEWTON: k_sat's arrays
+template <int MODE>
 __global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd, GncDev G, HfbDev F,
                                                          int iss,
                                                          double delt,
@@ -496,8 +511,6 @@ __global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd,
     int c, k, i, j, l;
     if (!pos_to_cell(L, p, c, k, i, j, l)) continue;
     const double hcell = x[p];
-    // npf_cf (gwf-npf.f90:444-470); under NEWTON k_sat has run
-    if (g.inewton == 0) g.sat[p] = cell_sat(g, p, hcell);
     // neighbour table in ascending natural order: up, back, left, right,
     // front, down.  nb = position, dir = connection plane, lower = pair
     // (nb, n) has nb first
@@ -519,27 +532,41 @@ __global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd,
       npos[4] = pres[4] ? ob + hn(l, L.ncol) : p;
     }
     const int dirs[6] = {2, 1, 0, 0, 1, 2};
-    const int ibp = g.ibound[p], ictp = g.icelltype[p];
-    double xm[6], cs[6], sm[6], dm[6], satp = 0.0, dervp = 0.0;
+    const int ibp = g.ibound[p], ictp = MODE == F_CONF ? 0 : g.icelltype[p];
+    double xm[6], cs[6], sm[6], dm[6], tm[6], bm[6], km[6], satp = 1.0, dervp = 0.0;
     int ibm[6], ictm[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) {
       const int m = npos[s];
-      xm[s] = x[m];
       cs[s] = g.condsat[dirs[s] * N + (s < 3 ? m : p)];
       ibm[s] = g.ibound[m];
+      ictm[s] = 0;
+      if (MODE == F_CONF) continue;
+      xm[s] = x[m];
       ictm[s] = g.icelltype[m];
-      sm[s] = dm[s] = 0.0;
-    }
-    if (g.inewton != 0) {
-      satp = g.sat[p];
-#pragma unroll
-      for (int s = 0; s < 6; s++) sm[s] = g.sat[npos[s]];
-      if (g.fn) {
-        dervp = derv[p];
-#pragma unroll
-        for (int s = 0; s < 6; s++) dm[s] = derv[npos[s]];
+      if (MODE == F_CONV) {
+        tm[s] = g.top[m];
+        bm[s] = g.bot[m];
+        if (dirs[s] != 2) km[s] = hk(g, dirs[s], m);
+      } else {
+        sm[s] = g.sat[m];
+        dm[s] = g.fn ? derv[m] : 0.0;
       }
+    }
+    // npf_cf (gwf-npf.f90:444-470); for F_NEWT k_sat has run
+    double tp_ = 0.0, bp_ = 0.0;
+    if (MODE == F_NEWT) {
+      satp = g.sat[p];
+      if (g.fn) dervp = derv[p];
+    } else {
+      if (MODE == F_CONV) {
+        tp_ = g.top[p];
+        bp_ = g.bot[p];
+        satp = cell_sat0(ictp, ibp, tp_, bp_, hcell);
+#pragma unroll
+        for (int s = 0; s < 6; s++) sm[s] = cell_sat0(ictm[s], ibm[s], tm[s], bm[s], xm[s]);
+      }
+      g.sat[p] = satp;
     }
     double off[6];
     double diag = 0.0;
@@ -551,19 +578,33 @@ __global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd,
       int m = npos[s];
       int dir = dirs[s];
       double cond;
+      // the pair (a, b): a the lower node (m for s < 3), at row ia and column ja
+      const bool lo = s < 3;
+      const int ia = i - (s == 1), ja = j - (s == 2);
       // the cases of hcond and vcond that need no more than the values above
       if (ibp == 0 || ibm[s] == 0) {
         cond = 0.0;
-      } else if ((ictp == 0 && ictm[s] == 0) || (dir == 2 && g.ivarcv == 0)) {
+      } else if (MODE == F_CONF || (ictp == 0 && ictm[s] == 0) || (dir == 2 && g.ivarcv == 0)) {
         cond = cs[s];
-      } else if (dir != 2 && g.inewton == 1) {
-        const bool upm = s < 3 ? xm[s] > hcell : !(hcell > xm[s]);   // m upstream
+      } else if (MODE == F_NEWT && dir != 2) {
+        const bool upm = lo ? xm[s] > hcell : !(hcell > xm[s]);   // m upstream
         cond = (upm ? sm[s] : satp) * cs[s];
-      } else if (s < 3) {   // m < n: pair (m, n), condsat stored at m
-        int im = i - (s == 1), jm = j - (s == 2);
-        cond = pair_cond(g, dir, m, p, im, jm, xm[s], hcell, cs[s]);
+      } else if (MODE == F_NEWT) {
+        cond = lo ? pair_cond(g, dir, m, p, ia, ja, xm[s], hcell, cs[s])
+                  : pair_cond(g, dir, p, m, ia, ja, hcell, xm[s], cs[s]);
+      } else if (dir == 2) {
+        cond = vcond(1, 1, 1, 1, 1, g.idewatcv, cs[s], lo ? xm[s] : hcell, lo ? hcell : xm[s],
+                     g.k33[lo ? m : p], g.k33[lo ? p : m], lo ? sm[s] : satp, lo ? satp : sm[s],
+                     lo ? tm[s] : tp_, lo ? tp_ : tm[s], lo ? bm[s] : bp_, lo ? bp_ : bm[s],
+                     g.delr[ja] * g.delc[ia]);
       } else {
-        cond = pair_cond(g, dir, p, m, i, j, hcell, xm[s], cs[s]);
+        const double kp = hk(g, dir, p);
+        const double cl1 = 0.5 * (dir == 0 ? g.delr[ja] : g.delc[ia]);
+        const double cl2 = 0.5 * (dir == 0 ? g.delr[ja + 1] : g.delc[ia + 1]);
+        cond = hcond(1, 1, 1, 1, 0, g.icellavg, cs[s], 0.0, 0.0, lo ? sm[s] : satp,
+                     lo ? satp : sm[s], lo ? km[s] : kp, lo ? kp : km[s], lo ? tm[s] : tp_,
+                     lo ? tp_ : tm[s], lo ? bm[s] : bp_, lo ? bp_ : bm[s], cl1, cl2,
+                     dir == 0 ? g.delc[ia] : g.delr[ja]);
       }
       off[s] = off[s] + cond;
       diag = diag + (-cond);
@@ -668,10 +709,10 @@ __global__ void __launch_bounds__(MF6_BLOCK, 3) k_formulate(GwfDev g, BndDev bd,
       diag = diag + bd.hcof[pk][idx];
     }
     // --- npf_fn
-    if (g.fn) {
+    if (MODE != F_CONV && g.fn) {
 #pragma unroll
       for (int s = 0; s < 6; s++) {
-        if (!pres[s]) continue;
+        if (MODE == F_CONF || !pres[s]) continue;
         int dir = dirs[s];
         if (dir == 2 && g.ivarcv == 0) continue;
         // pair (a, b), a the lower node: this row is b for s < 3
@@ -1485,6 +1526,7 @@ extern "C" int mf6hip_gwf_create(void *handle, const mf6hip_gwf_model *m) {
       else sat0[n] = hs >= tp ? 1.0 : (hs - bt) / (tp - bt);
     }
     h->h_icelltype = ict;
+    h->convertible = std::any_of(ict.begin(), ict.end(), [](int t) { return t != 0; });
     CK(upload_pos(h, &h->icelltype, ict.data()));
     CK(upload_pos(h, &h->sat0, sat0.data()));
     CK(upload_pos(h, &h->hn0, hn0.data()));
@@ -2094,10 +2136,19 @@ extern "C" int mf6hip_gwf_formulate(void *handle, int kiter, int inewton, double
   }
   GwfDev g = make_dev(h);
   g.fn = h->m.inewton && inewton;
-  // z: free between solves
-  if (g.inewton != 0) k_sat<<<ggrid(L.N), MF6_BLOCK, 0, s>>>(g, h->x, h->z);
-  k_formulate<<<ggrid(L.N), MF6_BLOCK, 0, s>>>(g, bd, gnc_dev(h), hfb_dev(h), h->iss, h->delt, h->x,
-                                               h->xold, h->z, h->A, h->b);
+  const int grid = ggrid(L.N);
+#define MF6_F(M)                                                                                  \
+  k_formulate<M><<<grid, MF6_BLOCK, 0, s>>>(g, bd, gnc_dev(h), hfb_dev(h), h->iss, h->delt, h->x, \
+                                            h->xold, h->z, h->A, h->b)
+  if (!h->convertible) {
+    MF6_F(F_CONF);
+  } else if (g.inewton == 0) {
+    MF6_F(F_CONV);
+  } else {
+    k_sat<<<grid, MF6_BLOCK, 0, s>>>(g, h->x, h->z);   // z: free between solves
+    MF6_F(F_NEWT);
+  }
+#undef MF6_F
   HIPCHK(hipGetLastError());
   if (amat_out || rhs_out) CK(mf6hip_copy_system(h, amat_out, rhs_out));
   return MF6HIP_OK;

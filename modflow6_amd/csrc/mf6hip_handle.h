@@ -134,6 +134,7 @@ struct Mf6Handle {
   double *d_gnc_a = nullptr, *d_gnc_cond = nullptr;
   int *d_gnc_off = nullptr, *d_gnc_ent = nullptr;
   std::vector<int> h_icelltype;   // natural order, host copy for the checks
+  bool convertible = false;       // some icelltype is not 0
   double *sat = nullptr;      // npf sat of the last formulate (per position)
   // budget (gwf_cq + gwf_bd) work arrays, allocated on first use
   double *flowja = nullptr;   // nja, CSR order

@@ -43,7 +43,7 @@ def _averaging(icellavg):
 
 # the averagings with a logarithmic mean (condmean, GwfConductanceUtils.f90:
 # 226-305)
-LOG_MEANS = {"logarithmic", "amt_lmk"}
+LOG_MEANS = {"logarithmic", "amt_lmk", "logarithmic_plain", "amt_lmk_plain"}
 
 def _k22(base, seed=8):
     c = base()
@@ -71,6 +71,14 @@ def _thickstrt(newton, seed=10):
     return dataclasses.replace(c, icelltype=ic, thickstrt=True)
 
 
+def _cell_types(newton, share, ivarcv=0, seed=11):
+    """A share of the cells confined (1: all of them), every cell's storage
+    convertible."""
+    c = _convertible(newton, ivarcv, 0, seed)
+    rng = np.random.default_rng(seed)
+    return dataclasses.replace(c, icelltype=(rng.random(c.nodes) >= share).astype(np.int32))
+
+
 CASES = {
     "varcv_newton": lambda: _convertible(True, 1, 0),
     "varcv_dewatered_newton": lambda: _convertible(True, 1, 1),
@@ -91,6 +99,12 @@ CASES = {
                                                            iconf_ss=1),
     "thickstrt_newton": lambda: _thickstrt(True),
     "thickstrt_plain": lambda: _thickstrt(False),
+    # convertible cells without NEWTON
+    "logarithmic_plain": lambda: dataclasses.replace(_convertible(False, 0, 0), icellavg=1),
+    "amt_lmk_plain": lambda: dataclasses.replace(_convertible(False, 1, 0), icellavg=2),
+    "amt_hmk_plain": lambda: dataclasses.replace(_convertible(False, 1, 1), icellavg=3),
+    "k22_plain": lambda: _k22(lambda: _convertible(False, 0, 0)),
+    "angles_plain": lambda: _angles(lambda: _convertible(False, 1, 0), True),
 }
 
 
@@ -132,6 +146,40 @@ def test_formulate_and_budget_bit_exact(name):
     assert bad.size == 0, (bad[:8], amat[bad[:8]], sim.amat[bad[:8]])
     assert np.array_equal(rhs.view(np.int64), sim.rhs.view(np.int64))
     assert np.array_equal(db["flowja"].view(np.int64), ob["flowja"].view(np.int64))
+
+
+# cells of both types, and confined cells alone (formulated without the values that
+# convertible cells need)
+CELL_TYPES = {
+    "mixed_types_newton": lambda: _cell_types(True, 0.4),
+    "mixed_types_varcv_newton": lambda: _cell_types(True, 0.4, 1),
+    "mixed_types_plain": lambda: _cell_types(False, 0.4),
+    "mixed_types_varcv_plain": lambda: _cell_types(False, 0.4, 1),
+    "confined_newton": lambda: _cell_types(True, 1.0),
+    "confined_varcv_newton": lambda: _cell_types(True, 1.0, 1),
+    "confined_plain": lambda: _cell_types(False, 1.0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CELL_TYPES))
+def test_cell_types_bit_exact(name):
+    case = CELL_TYPES[name]()
+    sim = O.GwfSimulation(case)
+    perlen, nstp, steady = case.periods[0]
+    sim.kper, sim.kstp = 1, 1
+    sim.advance(perlen / nstp, steady)
+    sim.formulate(1)
+    gs = GwfSolution(case)
+    try:
+        gs.kper, gs.kstp = 1, 1
+        gs.prepare_timestep(perlen / nstp, steady)
+        amat, rhs = gs.formulate(1, want_system=True)
+        db = gs.budget()
+    finally:
+        gs.destroy()
+    assert np.array_equal(amat.view(np.int64), sim.amat.view(np.int64))
+    assert np.array_equal(rhs.view(np.int64), sim.rhs.view(np.int64))
+    assert np.array_equal(db["flowja"].view(np.int64), sim.budget()["flowja"].view(np.int64))
 
 
 @pytest.mark.parametrize("name", ["varcv_dewatered_newton", "logarithmic", "k22_newton",
