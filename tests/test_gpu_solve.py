@@ -119,8 +119,9 @@ def test_mixed_precision_steady_small(precision, shape):
 
 @pytest.mark.parametrize("shape", [(3, 100, 100), (1, 51, 51), (5, 33, 17)])
 def test_fused_cg_matches_unfused(shape):
-    """The fused thread-per-column CG and the one-kernel-per-pass CG run the
-    same iteration; only the time at which x / d are updated and the dot
+    """The thread-per-column CG (on these grids the folded kernels; the fused
+    ones in the test of the block sizes) and the one-kernel-per-pass CG run
+    the same iteration; only the time at which x / d are updated and the dot
     summation order differ."""
     nlay, nrow, ncol = shape
     case = configs.steady_small(seed=9, nlay=nlay, nrow=nrow, ncol=ncol,
@@ -179,8 +180,11 @@ def assert_same_trajectory(ra, rb, n):
 
 
 # more columns than the folded kernels take: the fused ones with 64 and 256
-# threads a block, grouped columns (even extents) and single ones
-@pytest.mark.parametrize("shape", [(2, 380, 380), (1, 600, 604), (2, 371, 373), (1, 601, 451)])
+# threads a block, grouped columns (even extents) and single ones, every
+# compile-time bound of the layers (4, 8, 16, 32)
+@pytest.mark.parametrize("shape", [(2, 380, 380), (1, 600, 604), (2, 371, 373), (1, 601, 451),
+                                   (6, 364, 364), (5, 365, 363), (12, 363, 364), (9, 363, 365),
+                                   (17, 363, 364), (18, 363, 363)])
 def test_fused_cg_block_sizes_match_unfused(shape):
     nlay, nrow, ncol = shape
     case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=3)
@@ -191,26 +195,41 @@ def test_fused_cg_block_sizes_match_unfused(shape):
         x, rec = x0.copy(), ConvergenceRecord(case.ims.inner_maximum)
         icn, it = sv.solve(1, amat, rhs, x, kstp=1, record=rec)
         sv.destroy()
-        out.append((it, rec))
-    (ia, ra), (ib, rb) = out
-    assert_same_trajectory(ra, rb, min(20, ia, ib))
+        assert icn == 1
+        out.append((x, it, rec))
+    (xa, ia, ra), (xb, ib, rb) = out
+    assert abs(ia - ib) <= max(3, ib // 50) and min(ia, ib) >= 20
+    # the head update of the last iteration included
+    assert np.max(np.abs(xa - xb)) < 10 * case.ims.inner_dvclose
+    assert_same_trajectory(ra, rb, 20)
 
 
-def test_fused_cg_graph_replay_matches_eager_launches():
-    """Without the per-launch timing the fused FP64 CG replays captured
-    eight-iteration graphs; with it, it launches every kernel.  The same
-    kernels run in the same order, so heads and iteration counts agree bit
-    for bit, on the first and on a repeated run of the same handle (the
-    graph is reused; host synchronisations sit between the replays)."""
-    case = configs.steady_small(nlay=3, nrow=40, ncol=40, nwel=8)
-    eager = GwfSolution(case, timing=True)
+# the folded CG, the fused one (grouped and single columns) and its two-level
+# forms, the folded BiCGSTAB
+@pytest.mark.parametrize("shape,kw", [((3, 40, 40), {}), ((2, 380, 380), {}), ((2, 371, 373), {}),
+                                      ((3, 40, 40), dict(preconditioner=2)),
+                                      ((3, 41, 43), dict(preconditioner=3)),
+                                      ((3, 30, 32), dict(newton=True))])
+def test_fused_cg_graph_replay_matches_eager_launches(shape, kw):
+    """Without the per-launch timing a solve replays captured graphs of a few
+    iterations; with it, it launches every kernel.  The same kernels run in
+    the same order, so heads and iteration counts agree bit for bit, on the
+    first and on a repeated run of the same handle (the graph is reused; host
+    synchronisations sit between the replays)."""
+    nlay, nrow, ncol = shape
+    kw = dict(kw)
+    if kw.pop("newton", False):
+        case = configs.transient_newton(seed=5, nlay=nlay, nrow=nrow, ncol=ncol, nwel=3, nper=1,
+                                        nstp=1, perlen=10.0)
+    else:
+        case = configs.steady_small(nlay=nlay, nrow=nrow, ncol=ncol, nwel=8)
+    eager = GwfSolution(case, timing=True, **kw)
     he = eager.run()
     inner_e = [r.inner for r in eager.log[0]]
     eager.destroy()
-    gs = GwfSolution(case)
+    gs = GwfSolution(case, **kw)
     for rep in range(2):
         if rep:
-            from modflow6_amd import _lib
             _lib.check(gs.L.mf6hip_gwf_set_x(gs.h, _lib.dptr(np.ascontiguousarray(case.strt))),
                        "set_x")
             gs.log.clear()
