@@ -196,16 +196,17 @@ __device__ inline void c_publish(FoldHost *hf, const KState *st, int stop) {
 // `iters` iterations.  The first two batches, up to eight iterations, are waited for
 // alone, since many solves end there (an outer loop's last ones take an iteration
 // or two: CG at 1x362x362 391 us with a batch queued behind the first, 297 alone,
-// BiCGSTAB at 5x500x500 475 and 415, one iteration each); then one batch is queued ahead of the one the host waits for, and a
-// batch grows with the iterations done (the end of a batch costs the GPU about
-// 10 us, an iteration after the stop 2 us per kernel): 1, 2, 4 or 8 graphs from 0, 64,
-// 256 and 1024 iterations on.
+// BiCGSTAB at 5x500x500 475 and 415, one iteration each); then one batch is queued ahead of the one the host waits for.
+// A batch is one graph, from 1024 iterations on four: its end costs the GPU a few us,
+// an iteration after the stop 2 us per kernel.  (Growing from 64 iterations on, 2, 4, 8
+// graphs, took 5.71 ms for 5.52 at 3x100x100, 275 iterations, and 17.25 for 16.96 at
+// 12x150x150; never growing 157.8 for 157.3 at 10x500x500, 1370 iterations.)
 template <typename F>
 int fold_batches(Mf6Handle *h, int iters, F launch) {
   FoldHost *hf = h->h_fold;
   int done = 0;
   auto batch = [&](int b) -> int {
-    const int n = done < 64 ? 1 : done < 256 ? 2 : done < 1024 ? 4 : 8;
+    const int n = done < 1024 ? 1 : 4;
     for (int r = 0; r < n; r++) {
       const int rc = launch();
       if (rc != MF6HIP_OK) return rc;
