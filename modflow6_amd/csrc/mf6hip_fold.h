@@ -199,8 +199,8 @@ __device__ inline void c_publish(FoldHost *hf, const KState *st, int stop) {
 // BiCGSTAB at 5x500x500 475 and 415, one iteration each); then one batch is queued ahead of the one the host waits for.
 // A batch is one graph, from 1024 iterations on four: its end costs the GPU a few us,
 // an iteration after the stop 2 us per kernel.  (Growing from 64 iterations on, 2, 4, 8
-// graphs, took 5.71 ms for 5.52 at 3x100x100, 275 iterations, and 17.25 for 16.96 at
-// 12x150x150; never growing 157.8 for 157.3 at 10x500x500, 1370 iterations.)
+// graphs, took 5.71 ms a step for 5.52 at 3x100x100 and 17.25 for 16.96 at 12x150x150;
+// never growing 157.8 for 157.3 at 10x500x500, with well over a thousand iterations.)
 template <typename F>
 int fold_batches(Mf6Handle *h, int iters, F launch) {
   FoldHost *hf = h->h_fold;

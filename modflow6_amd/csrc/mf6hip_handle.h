@@ -252,9 +252,9 @@ int mf6hip_is_symmetric(Mf6Handle *h, int *sym);
 int mf6hip_dxmax(Mf6Handle *h, double *hncg, int *lrch, const double *xa,
                  const double *xb, bool active_only);
 
-// solver pieces shared with the flexible CG (mf6hip_fcg.hip)
-// z = ILU0(r); the kernels return at once when st is given and st->stop is set
+// flexible CG with the learned correction (mf6hip_fcg.hip)
 int mf6hip_run_fcg(Mf6Handle *h);
+// a system in the reference's CSR layout into planes, with its ILU0 pivots (ensemble)
 int mf6hip_stage_system(const Layout &L, const int *ia1, int nja, const double *amat,
                         const double *rhs, const double *x0, double relax, double *A64,
                         double *b64, double *x64, double *piv64, hipStream_t s);
